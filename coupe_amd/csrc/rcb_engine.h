@@ -145,6 +145,7 @@ struct Context {
     bool graphs = false;             // replay a call of a known shape as one captured graph
     uint32_t copy_parts = 256;       // levels of at most this many parts flush into per-XCD copies
     uint32_t search_chunk = 2;       // consecutive tiles a workgroup takes at a time in the search passes
+    bool small = true;               // problems of few points take one workgroup each (rcb_small.h)
     double move_nt_bytes = 2.5e9;    // moves and id descents of more bytes than this go non-temporal
     int max_bins = kMaxBins;         // bins per part of the later search passes (16..256, a power of two)
     int wg_cap = 0;                  // workgroups per CU of the persistent kernels (0: as many as fit)
@@ -178,6 +179,7 @@ struct Context {
         hints.back().shape = shape;
         return hints.back();
     }
+    DevBuf small_table, small_report;   // the small problems of a batch and what they report
     DevBuf loads;                    // per-part loads (imbalance)
     DevBuf tile_bins;                // per-tile bin counts of the histogram passes
     DevBuf gparts[2], gaxis, gchunk, gcount, gctr;   // Grid::rcb: subgrids, axis sums, chunk offsets
@@ -272,6 +274,12 @@ inline double move_nt_bytes_from_env() {
     return b < 0 ? 0.0 : b;
 }
 
+// COUPE_HIP_SMALL=0: problems of few points take the general path too.
+inline bool small_from_env() {
+    const char *v = getenv("COUPE_HIP_SMALL");
+    return !(v && v[0] == '0');
+}
+
 // COUPE_HIP_SEARCH_CHUNK=k: the later search passes hand k consecutive
 // tiles at a time to each workgroup (default 2, at most 64).
 inline uint32_t search_chunk_from_env() {
@@ -336,6 +344,7 @@ inline void configure_from_env(Context &c) {
     c.graphs = graphs_from_env();
     c.copy_parts = copy_parts_from_env();
     c.search_chunk = search_chunk_from_env();
+    c.small = small_from_env();
     c.move_nt_bytes = move_nt_bytes_from_env();
     c.max_bins = bins_from_env();
     c.wg_cap = wg_cap_from_env();

@@ -15,6 +15,7 @@
 #include "rcb_engine.h"
 #include "rcb_kernels.h"
 #include "rcb_pairs.h"
+#include "rcb_small.h"
 
 namespace coupe_hip {
 
@@ -257,10 +258,16 @@ void scan_u64(Context &cx, hipStream_t st, uint64_t *data, const uint32_t *n_dev
 // (its first one and one per pass) in the context's last call of the same
 // shape: none when the first decision ended every search there (the split
 // at the first candidate, the usual case on even data), else the passes it
-// took plus one to spare, at most spec.
-static int queued_passes(int spec, uint32_t decisions) {
-    if (decisions <= 1) return 0;
-    return std::min(spec, (int)decisions);
+// took plus one to spare, at most spec.  Calls of kSparePoints points or more
+// queue one and two more: a queued pass whose gate stays closed costs about
+// 8 us, the run with host checks that a search outlasting its passes brings
+// costs the call again (5.8e8 points in 4096 instances, three data sets in
+// turn: 39.2 -> 29.6 ms; 2^27-point grids: 6.51 -> 6.62 ms, but no run of 13 ms).
+constexpr uint64_t kSparePoints = 1ull << 26;
+static int queued_passes(int spec, uint32_t decisions, uint64_t n) {
+    const int more = n >= kSparePoints ? 1 : 0;
+    if (decisions <= 1) return std::min(spec, more);
+    return std::min(spec, (int)decisions + 2 * more);
 }
 
 // Bins per part of the standalone LDS passes, bounded by the bin buffers.
@@ -392,7 +399,7 @@ static bool run_levels(Context &cx, hipStream_t st, const BatchPlan &B, int wrap
     const Hints *seen = cx.hints_for(shape);
     std::vector<int> depth(L, spec_passes);
     if (spec_passes > 0 && seen && seen->level_passes.size() == L)
-        for (size_t l = 0; l < L; l++) depth[l] = queued_passes(spec_passes, seen->level_passes[l]);
+        for (size_t l = 0; l < L; l++) depth[l] = queued_passes(spec_passes, seen->level_passes[l], n);
     std::vector<uint8_t> used(L, 0);   // decisions per level in this call
     std::vector<uint32_t> open1(L, 0);  // parts still searching after each level's first decision
     const std::vector<uint32_t> last_open = seen && seen->level_open.size() == L ? seen->level_open
@@ -1214,7 +1221,7 @@ static uint64_t graph_key(const Context &cx, const BatchPlan &B, size_t dim, int
     mix((uint64_t)(int64_t)(e ? e->weight_hint : cx.weight_hint));
     const size_t L = B.max_levels;
     for (size_t l = 0; l < L; l++) {
-        const int d = e && e->level_passes.size() == L ? queued_passes(spec, e->level_passes[l]) : spec;
+        const int d = e && e->level_passes.size() == L ? queued_passes(spec, e->level_passes[l], B.n) : spec;
         const bool ff = e && e->level_open.size() == L &&
                         2 * (uint64_t)e->level_open[l] > std::max<uint64_t>(B.parts_ub[l], 1);
         mix((uint64_t)d | (uint64_t)ff << 16);
@@ -1305,6 +1312,189 @@ static int run_captured(Context &cx, hipStream_t caller, const BatchPlan &B, siz
     return unfinished ? 1 : 0;
 }
 
+// ---------------------------------------------------------------------------
+// Small problems: one workgroup each (rcb_small.h).
+// ---------------------------------------------------------------------------
+// A problem the small kernel takes: its points fit a workgroup's registers
+// and the slots of its last level fit its LDS.
+static bool is_small(const Context &cx, uint64_t count, size_t levels) {
+    return cx.small && count > 0 && count <= kSmallPoints && levels <= kSmallLevels;
+}
+
+// Points per workgroup of the three shapes: 256 threads of 8 points (several
+// workgroups per CU), 512 threads of 16, and 512 of 32.
+constexpr uint32_t kSmallShape[3] = {256 * 8, 512 * 16, 512 * 32};
+static_assert(kSmallShape[2] == kSmallPoints, "the last shape takes every small problem");
+
+template <int D, typename WIN>
+static void launch_small(Context &cx, hipStream_t st, const std::vector<SmallProblem> &problems,
+                         const SmallProblem *table, const double *pts, const WIN *w, int wrap32, uint64_t *out,
+                         uint32_t *report) {
+    // problems come sorted by shape; a shape's run is one launch
+    size_t at = 0;
+    for (int shape = 0; shape < 3; shape++) {
+        size_t end = at;
+        uint32_t levels = 1;
+        double points = 0.0;
+        while (end < problems.size() && problems[end].count <= kSmallShape[shape]) {
+            levels = std::max(levels, problems[end].levels);
+            points += problems[end].count;
+            end++;
+        }
+        if (end == at) continue;
+        Rotation rot;
+        memset(&rot, 0, sizeof rot);
+        if (cx.rot) rot = *cx.rot;
+        const float *c0 = cx.slot0[0], *c1 = cx.slot0[1], *c2 = cx.slot0[2];
+        auto launch = [&](auto kernel, int tpb) {
+            const uint32_t lds = sub_lds(levels, tpb);
+            if (lds > 65536)
+                check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            // algorithmic bytes: points and weights read, ids written
+            timed(cx, st, COUPE_HIP_K_OTHER, points * (8.0 * D + sizeof(WIN) + 8.0), [&] {
+                kernel<<<(unsigned)(end - at), tpb, lds, st>>>(problems[at], table ? table + at : nullptr, pts, c0, c1,
+                                                              c2, w, wrap32, cx.rot ? 1 : 0, rot, out, report + at);
+            });
+        };
+        if (shape == 0) launch(k_small<D, 256, 8, WIN>, 256);
+        else if (shape == 1) launch(k_small<D, 512, 16, WIN>, 512);
+        else launch(k_small<D, 512, 32, WIN>, 512);
+        at = end;
+    }
+}
+
+// Runs the small problems of a call and waits for them.  One problem is
+// passed as the kernel's argument and reports straight into the pinned
+// readback area; several are copied as a table.
+static void run_small(Context &cx, hipStream_t st, std::vector<SmallProblem> &problems, size_t dim,
+                      const double *pts, int wkind, const void *w, uint64_t *out) {
+    std::stable_sort(problems.begin(), problems.end(),
+                     [](const SmallProblem &a, const SmallProblem &b) { return a.count < b.count; });
+    const bool one = problems.size() == 1;
+    const bool pinned = one && !cx.borrowed_host;
+    const SmallProblem *table = nullptr;
+    uint32_t *report = (uint32_t *)cx.host_scratch;
+    if (!one) {
+        cx.small_table.ensure(problems.size() * sizeof(SmallProblem));
+        table = (const SmallProblem *)cx.small_table.ptr;
+        check(hipMemcpyAsync(cx.small_table.ptr, problems.data(), problems.size() * sizeof(SmallProblem),
+                             hipMemcpyHostToDevice, st));
+    }
+    if (!pinned) {
+        cx.small_report.ensure(problems.size() * sizeof(uint32_t));
+        report = (uint32_t *)cx.small_report.ptr;
+    }
+    auto run = [&](auto dtag) {
+        constexpr int D = decltype(dtag)::value;
+        if (wkind == COUPE_INT) launch_small<D>(cx, st, problems, table, pts, (const int32_t *)w, 1, out, report);
+        else if (wkind == COUPE_INT64) launch_small<D>(cx, st, problems, table, pts, (const int64_t *)w, 0, out, report);
+        else launch_small<D>(cx, st, problems, table, pts, (const double *)w, 0, out, report);
+    };
+    if (dim == 2) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 3>{});
+    std::vector<uint32_t> got(problems.size());
+    if (!pinned)
+        check(hipMemcpyAsync(got.data(), report, got.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    check(hipStreamSynchronize(st));
+    if (pinned) got[0] = *(volatile uint32_t *)report;
+    uint32_t all = 0, levels = 0;
+    for (uint32_t g : got) all |= g;
+    for (const SmallProblem &p : problems) {
+        levels = std::max(levels, p.levels);
+        cx.stats.points += p.count;
+    }
+    if (all & kSmallError) throw HipFailure{hipErrorUnknown};
+    // the stored width the general path would choose
+    const uint32_t wb = (all & (kSmallReal | kSmallWide)) ? 8u : ((all & kSmallNot16) || !cx.weights16 ? 4u : 2u);
+    cx.stats.weight_mode |= (all & kSmallReal) ? 1u : 0u;
+    cx.stats.weight_bytes = std::max(cx.stats.weight_bytes, wb);
+    cx.stats.levels = std::max(cx.stats.levels, levels);
+    cx.stats.bins = std::max<uint32_t>(cx.stats.bins, kSubMaxNb);
+}
+
+// The general path of a batch: every part of a level at once, level by level
+// (the caller checked the arguments and set the call's scope and switches).
+static enum coupe_err rcb_general(Context &cx, hipStream_t st, uint64_t *d_out, size_t dim, const double *d_points,
+                         int wkind, const void *d_weights, const uint64_t *counts, const size_t *levels,
+                         const double *tols, size_t n_inst, const Rotation *rot, const uint64_t *src_idx,
+                         const uint64_t *src_pt) {
+    try {
+        BatchPlan B = plan_batch(counts, levels, tols, n_inst, dim, src_idx, src_pt);
+        cx.stats.points = B.n;
+        if (B.n == 0) return COUPE_ERR_OK;            // BoundingBox::from_points is None (:685-688)
+        if (B.n > 0xffffffffull) return COUPE_ERR_ALLOC;
+        if (B.inst.size() > 1 && !B.dense) return COUPE_ERR_BAD_TYPE;
+        check(hipSetDevice(cx.device));
+        if (!cx.host_scratch) check(hipHostMalloc(&cx.host_scratch, kHostScratch, hipHostMallocDefault));
+        if (cx.cu_count <= 0) {
+            check(hipDeviceGetAttribute(&cx.cu_count, hipDeviceAttributeMultiprocessorCount, cx.device));
+            if (cx.cu_count <= 0) cx.cu_count = 1;
+        }
+        auto run = [&](int spec, hipStream_t s) {
+            return dim == 2 ? run_dim<2>(cx, s, d_out, B, d_points, wkind, d_weights, spec)
+                            : run_dim<3>(cx, s, d_out, B, d_points, wkind, d_weights, spec);
+        };
+        // Passes queued per level: the configured depth, or fewer (never
+        // under 2) when this context's last call needed fewer (its deepest
+        // search's decisions); each queued pass costs two launches even when
+        // its gate is closed.
+        // A shape run before queues as many as its deepest search needed then
+        // (2..16; a level queues no more than it needed).
+        int spec = cx.search_passes;
+        const Hints *seen = cx.hints_for(B.shape);
+        const int passes_hint = seen ? seen->passes_hint : 0;
+        if (passes_hint > 0 && spec > 0)
+            spec = std::max(2, std::min(16, passes_hint + (B.n >= kSparePoints ? 2 : 0)));
+        // A shape this context has run (hints known, buffers sized) runs as
+        // one captured graph: 0 done, 1 a search outran its queued passes,
+        // 2 not run that way (or its data needs another weight mode).
+        int how = 2;
+        if (cx.graphs && !rot && !cx.prof.enabled && !t_arena && spec > 0 && cx.bins_clean && seen &&
+            seen->weight_hint >= 0 && seen->level_passes.size() == B.max_levels)
+            how = run_captured(cx, st, B, dim, wkind, d_out, d_points, d_weights, spec, run);
+        if (how == 3) how = 2;   // first sight of the graph key: eager
+        const bool unfinished = how == 1 || (how == 2 && run(spec, st));
+        if (unfinished) {
+            // a split search needed more passes than were queued: again,
+            // checking every pass on the host
+            cx.stats = coupe_hip_stats{};
+            cx.stats.points = B.n;
+            cx.stats.reruns = 1;
+            run(0, st);
+        }
+        cx.remember(B.shape).passes_hint = (int)cx.stats.max_passes;
+    } catch (const HipFailure &f) {
+        cx.bins_clean = false;
+        (void)hipGetLastError();
+        return map_hip_error(f.err);
+    } catch (const std::bad_alloc &) {
+        cx.bins_clean = false;
+        return COUPE_ERR_ALLOC;
+    } catch (const std::length_error &) {
+        cx.bins_clean = false;
+        return COUPE_ERR_ALLOC;
+    }
+    return COUPE_ERR_OK;
+}
+
+// The instances the general path would take of a batch (all of them when none
+// does): the batch's class for the autotuner is theirs.
+static uint64_t batch_tune_key(const Context &cx, const uint64_t *counts, const size_t *levels, const double *tols,
+                               size_t n_inst, size_t dim) {
+    std::vector<uint64_t> c;
+    std::vector<size_t> l;
+    std::vector<double> t;
+    for (size_t q = 0; q < n_inst; q++)
+        if (!is_small(cx, counts[q], levels[q])) {
+            c.push_back(counts[q]);
+            l.push_back(levels[q]);
+            t.push_back(tols[q]);
+        }
+    if (c.empty()) return tune_key(plan_batch(counts, levels, tols, n_inst, dim), dim);
+    return tune_key(plan_batch(c.data(), l.data(), t.data(), c.size(), dim), dim);
+}
+
 enum coupe_err rcb_batch(Context &cx, hipStream_t st, uint64_t *d_out, size_t dim, const double *d_points,
                          int wkind, const void *d_weights, const uint64_t *counts, const size_t *levels,
                          const double *tols, size_t n_inst, const Rotation *rot, const ResidentSource *src,
@@ -1351,76 +1541,72 @@ enum coupe_err rcb_batch(Context &cx, hipStream_t st, uint64_t *d_out, size_t di
             c.search_chunk = chunk;
         }
     } tune_scope(cx);
+    enum coupe_err err = COUPE_ERR_OK;
     try {
-        BatchPlan B = plan_batch(counts, levels, tols, n_inst, dim, src_idx, src_pt);
         bool tuned = false;
-        if (!cx.tuning_now) {
-            const uint64_t tk = tune_key(B, dim);
+        if (!cx.tuning_now && !cx.tuned.empty()) {
+            const uint64_t tk = batch_tune_key(cx, counts, levels, tols, n_inst, dim);
             for (const auto &e : cx.tuned)
                 if (e.first == tk) {
                     apply_tuning(cx, e.second);
                     tuned = true;
                 }
         }
-        cx.stats.points = B.n;
-        if (B.n == 0) return COUPE_ERR_OK;            // BoundingBox::from_points is None (:685-688)
-        if (B.n > 0xffffffffull) return COUPE_ERR_ALLOC;
-        if (B.inst.size() > 1 && !B.dense) return COUPE_ERR_BAD_TYPE;
-        check(hipSetDevice(cx.device));
-        if (!cx.host_scratch) check(hipHostMalloc(&cx.host_scratch, kHostScratch, hipHostMallocDefault));
-        if (cx.cu_count <= 0) {
-            check(hipDeviceGetAttribute(&cx.cu_count, hipDeviceAttributeMultiprocessorCount, cx.device));
-            if (cx.cu_count <= 0) cx.cu_count = 1;
+        // The small problems first, one workgroup each, then the rest as a
+        // batch of the general path.  A call the general path refuses
+        // (too many points, a batch of deep trees) goes to it whole, and so
+        // does one that is replayed as a captured graph.
+        bool split = cx.small && !cx.graphs && total > 0 && total <= 0xffffffffull;
+        for (size_t q = 0; q < n_inst && n_inst > 1; q++) split = split && levels[q] <= (size_t)kDenseLevels;
+        std::vector<SmallProblem> small;
+        std::vector<uint64_t> cnt, at, at_pt;
+        std::vector<size_t> lev;
+        std::vector<double> tol;
+        if (split) {
+            uint64_t begin = 0;
+            for (size_t q = 0; q < n_inst; q++) {
+                const uint64_t s = src_idx ? src_idx[q] : begin, sp = src_pt ? src_pt[q] : begin * dim;
+                begin += counts[q];
+                if (is_small(cx, counts[q], levels[q])) {
+                    small.push_back(SmallProblem{s, sp, tols[q], (uint32_t)counts[q], (uint32_t)levels[q]});
+                } else if (counts[q] > 0) {
+                    cnt.push_back(counts[q]);
+                    lev.push_back(levels[q]);
+                    tol.push_back(tols[q]);
+                    at.push_back(s);
+                    at_pt.push_back(sp);
+                }
+            }
         }
-        auto run = [&](int spec, hipStream_t s) {
-            return dim == 2 ? run_dim<2>(cx, s, d_out, B, d_points, wkind, d_weights, spec)
-                            : run_dim<3>(cx, s, d_out, B, d_points, wkind, d_weights, spec);
-        };
-        // Passes queued per level: the configured depth, or fewer (never
-        // under 2) when this context's last call needed fewer (its deepest
-        // search's decisions); each queued pass costs two launches even when
-        // its gate is closed.
-        // A shape run before queues as many as its deepest search needed then
-        // (2..16; a level queues no more than it needed).
-        int spec = cx.search_passes;
-        const Hints *seen = cx.hints_for(B.shape);
-        const int passes_hint = seen ? seen->passes_hint : 0;
-        if (passes_hint > 0 && spec > 0) spec = std::max(2, std::min(16, passes_hint));
-        // A shape this context has run (hints known, buffers sized) runs as
-        // one captured graph: 0 done, 1 a search outran its queued passes,
-        // 2 not run that way (or its data needs another weight mode).
-        int how = 2;
-        if (cx.graphs && !rot && !cx.prof.enabled && !t_arena && spec > 0 && cx.bins_clean && seen &&
-            seen->weight_hint >= 0 && seen->level_passes.size() == B.max_levels)
-            how = run_captured(cx, st, B, dim, wkind, d_out, d_points, d_weights, spec, run);
-        if (how == 3) how = 2;   // first sight of the graph key: eager
-        const bool unfinished = how == 1 || (how == 2 && run(spec, st));
-        if (unfinished) {
-            // a split search needed more passes than were queued: again,
-            // checking every pass on the host
-            cx.stats = coupe_hip_stats{};
-            cx.stats.points = B.n;
-            cx.stats.reruns = 1;
-            run(0, st);
+        if (small.empty()) {
+            err = rcb_general(cx, st, d_out, dim, d_points, wkind, d_weights, counts, levels, tols, n_inst, rot,
+                              src_idx, src_pt);
+        } else {
+            if (!cnt.empty())
+                err = rcb_general(cx, st, d_out, dim, d_points, wkind, d_weights, cnt.data(), lev.data(), tol.data(),
+                                  cnt.size(), rot, at.data(), at_pt.data());
+            if (err == COUPE_ERR_OK) {
+                check(hipSetDevice(cx.device));
+                if (!cx.host_scratch) check(hipHostMalloc(&cx.host_scratch, kHostScratch, hipHostMallocDefault));
+                run_small(cx, st, small, dim, d_points, wkind, d_weights, d_out);
+            }
         }
-        cx.remember(B.shape).passes_hint = (int)cx.stats.max_passes;
-        cx.stats.tuned = tuned ? 1u : 0u;
-        cx.stats.tuning = current_tuning(cx);
-        cx.prof.collect();
-        cx.prof.out[COUPE_HIP_K_HIST].algo_bytes += cx.swept_bytes;   // first passes + standalone passes
+        if (err == COUPE_ERR_OK) {
+            cx.stats.tuned = tuned ? 1u : 0u;
+            cx.stats.tuning = current_tuning(cx);
+            cx.prof.collect();
+            cx.prof.out[COUPE_HIP_K_HIST].algo_bytes += cx.swept_bytes;   // first passes + standalone passes
+        }
     } catch (const HipFailure &f) {
-        cx.bins_clean = false;
         (void)hipGetLastError();
         return map_hip_error(f.err);
     } catch (const std::bad_alloc &) {
-        cx.bins_clean = false;
         return COUPE_ERR_ALLOC;
     } catch (const std::length_error &) {
-        cx.bins_clean = false;
         return COUPE_ERR_ALLOC;
     }
-    cx.stats.device_bytes = cx.device_bytes();
-    return COUPE_ERR_OK;
+    if (err == COUPE_ERR_OK) cx.stats.device_bytes = cx.device_bytes();
+    return err;
 }
 
 enum coupe_err rcb_batch_mixed(Context &cx, hipStream_t st, uint64_t *d_out, const double *d_points, int wkind,
@@ -1471,7 +1657,7 @@ enum coupe_err autotune(Context &cx, hipStream_t st, uint64_t *d_out, const doub
                 l.push_back(levels[q]);
                 t.push_back(tols[q]);
             }
-        if (!c.empty()) keys.push_back(tune_key(plan_batch(c.data(), l.data(), t.data(), c.size(), d), d));
+        if (!c.empty()) keys.push_back(batch_tune_key(cx, c.data(), l.data(), t.data(), c.size(), d));
     }
     struct Restore {   // the context's own switches come back after the tuning
         Context &c;
@@ -1566,7 +1752,7 @@ void Context::for_each_buf(F &&f) {
                      &tile_bins2, &tile4, &bcnt, &bw, &bmin, &xcnt, &xw, &xmin, &nchild, &ntiles, &bsum, &nodes, &leaf,
                      &heap_split, &instances, &tiles0, &below, &tile_left, &loads, &rib_moments, &tile_bins,
                      &gparts[0], &gparts[1], &gaxis, &gchunk, &gcount, &gctr, &gsat, &gcol, &grow, &gheap, &gscan,
-                     &ired, &counters, &in_points, &in_weights, &out_ids};
+                     &small_table, &small_report, &ired, &counters, &in_points, &in_weights, &out_ids};
     for (DevBuf *d : all) f(*d);
 }
 
