@@ -86,6 +86,8 @@ struct Hints {
     std::vector<uint8_t> level_passes;  // decisions each level's search needed
     std::vector<uint32_t> level_open;   // parts of each level still searching after the first decision
     uint64_t graph_key = 0;             // graph key of its last call (a key is captured when it repeats)
+    int mid = -1;                       // the midpoint tree took its last call (-1: not tried, 0: no)
+    uint32_t mid_open = 1;              // open nodes the midpoint tree left (0: none)
     int moves_coherent = -1;            // its moved tiles went to few destinations (-1: not known)
 };
 
@@ -146,6 +148,7 @@ struct Context {
     uint32_t copy_parts = 256;       // levels of at most this many parts flush into per-XCD copies
     uint32_t search_chunk = 2;       // consecutive tiles a workgroup takes at a time in the search passes
     bool small = true;               // problems of few points take one workgroup each (rcb_small.h)
+    bool mid = true;                 // try the tree of box midpoints first (rcb_mid.h)
     double move_nt_bytes = 2.5e9;    // moves and id descents of more bytes than this go non-temporal
     int max_bins = kMaxBins;         // bins per part of the later search passes (16..256, a power of two)
     int wg_cap = 0;                  // workgroups per CU of the persistent kernels (0: as many as fit)
@@ -179,6 +182,8 @@ struct Context {
         hints.back().shape = shape;
         return hints.back();
     }
+    DevBuf mid_code, mid_cnt, mid_w, mid_map, mid_inst, mid_open, mid_cursor, mid_lists, mid_slots;   // midpoint tree
+    bool mid_clean = false;          // its cells are all zero
     DevBuf small_table, small_report;   // the small problems of a batch and what they report
     DevBuf loads;                    // per-part loads (imbalance)
     DevBuf tile_bins;                // per-tile bin counts of the histogram passes
@@ -280,6 +285,13 @@ inline bool small_from_env() {
     return !(v && v[0] == '0');
 }
 
+// COUPE_HIP_MID=0: the levels are searched one after the other even where the
+// parts split at the middle of their box.
+inline bool mid_from_env() {
+    const char *v = getenv("COUPE_HIP_MID");
+    return !(v && v[0] == '0');
+}
+
 // COUPE_HIP_SEARCH_CHUNK=k: the later search passes hand k consecutive
 // tiles at a time to each workgroup (default 2, at most 64).
 inline uint32_t search_chunk_from_env() {
@@ -345,6 +357,7 @@ inline void configure_from_env(Context &c) {
     c.copy_parts = copy_parts_from_env();
     c.search_chunk = search_chunk_from_env();
     c.small = small_from_env();
+    c.mid = mid_from_env();
     c.move_nt_bytes = move_nt_bytes_from_env();
     c.max_bins = bins_from_env();
     c.wg_cap = wg_cap_from_env();

@@ -16,6 +16,7 @@
 #include "rcb_kernels.h"
 #include "rcb_pairs.h"
 #include "rcb_small.h"
+#include "rcb_mid.h"
 
 namespace coupe_hip {
 
@@ -163,6 +164,7 @@ struct Counters {
     Prologue pro[kCopies];                      // the prologue's weight flags
     uint32_t forwarded[kCopies];                // parts whose children's first pass the move forwarded
     uint32_t unfinished;                        // a speculative search did not end in its passes
+    MidCounters mid;                            // the midpoint tree's open nodes
     uint32_t error;                             // the node-record descent found an inconsistent tree
     uint32_t spec[kSpecSlots * kCopies];        // parts still searching after pass p of level l (slot's copies)
     uint32_t end;                               // end of the call's readback
@@ -211,6 +213,8 @@ static bool finish_levels(Context &cx) {
         Hints &e = cx.remember(P.shape);
         e.level_passes = used;
         e.level_open = open1;
+        // the midpoint tree again when every part of the first levels split at its midpoint
+        if (e.mid == 0 && P.levels >= 3 && open1[0] == 0 && open1[1] == 0 && open1[2] == 0) e.mid = -1;
     }
     return h->unfinished != 0;
 }
@@ -1062,6 +1066,179 @@ static void prologue(Context &cx, hipStream_t st, const BatchPlan &B, const doub
     }
 }
 
+// ---------------------------------------------------------------------------
+// The midpoint tree (rcb_mid.h).
+// ---------------------------------------------------------------------------
+constexpr uint64_t kMidCells = 1ull << 21;        // cells of a call, at most
+constexpr uint64_t kMidCopied = 1ull << 16;       // cells kept in one copy per XCD up to here
+
+// Whether a call takes it: its levels fit the cells, no switch asks for the
+// general path's passes or its graph, its buffers may grow, and the last call
+// of the shape did not end on the general path.
+static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
+    if (!cx.mid || !cx.pairs || !cx.forward || spec_passes <= 0 || cx.capturing || cx.graphs || t_arena) return false;
+    if (!B.dense || B.max_levels == 0 || B.max_levels > kMidLevels) return false;
+    if (B.heap_total + B.inst.size() > kMidCells) return false;
+    const Hints *seen = cx.hints_for(B.shape);
+    return !seen || seen->mid != 0;
+}
+
+template <typename K>
+static void allow_lds(K kernel, uint32_t lds) {
+    if (lds > 65536)
+        check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds));
+}
+
+// Runs a call on the midpoint tree after its prologue.  w: the stored weights,
+// or the caller's (w_src).  Waits for the stream and reads the call's
+// counters.  False when an open node is too large for a workgroup: nothing
+// was written then, and the call goes on on the general path.
+template <int D, typename WL, typename Acc>
+static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
+                    int w_src) {
+    Counters *ctr = (Counters *)cx.counters.ptr;
+    MidCounters *mid = (MidCounters *)((char *)ctr + offsetof(Counters, mid));
+    const uint32_t n_inst = (uint32_t)B.inst.size(), nt = (uint32_t)B.tiles0;
+    const uint64_t n = B.n, cells = B.heap_total + n_inst;
+    const uint32_t copies = cells <= kMidCopied ? (uint32_t)kCopies : 1u;
+    const uint32_t max_cells = 1u << B.max_levels;
+    const bool fresh = cx.mid_cnt.bytes < copies * cells * 4 || cx.mid_w.bytes < copies * cells * 8;
+    cx.mid_code.ensure(n * 2);
+    cx.mid_cnt.ensure(copies * cells * 4);
+    cx.mid_w.ensure(copies * cells * 8);
+    cx.mid_map.ensure(cells * 4);
+    cx.mid_inst.ensure(n_inst * sizeof(MidInstance));
+    cx.mid_open.ensure(cells * sizeof(MidOpen));
+    cx.mid_cursor.ensure(cells * 4);
+    cx.mid_lists.ensure(kMidClasses * cells * 4);
+    cx.mid_slots.ensure(n * 2);
+    cx.heap_split.ensure(std::max<uint64_t>(B.heap_total, 1) * sizeof(float));
+    cx.w[1].ensure(n * sizeof(WL));
+    uint32_t *gcnt = (uint32_t *)cx.mid_cnt.ptr;
+    Acc *gw = (Acc *)cx.mid_w.ptr;
+    if (fresh || !cx.mid_clean) {   // k_mid_tree leaves them clear
+        k_fill_u32<<<1024, kBlock, 0, st>>>(gcnt, cx.mid_cnt.bytes / 4, 0u);
+        k_fill_u32<<<1024, kBlock, 0, st>>>((uint32_t *)gw, cx.mid_w.bytes / 4, 0u);
+    }
+    cx.mid_clean = false;   // until this call completes
+    const Tile *tiles = (const Tile *)cx.tiles0.ptr;
+    Instance *insts = (Instance *)cx.instances.ptr;
+    const InstReduce *red = (const InstReduce *)cx.ired.ptr;
+    MidInstance *minst = (MidInstance *)cx.mid_inst.ptr;
+    MidOpen *open = (MidOpen *)cx.mid_open.ptr;
+    uint32_t *map = (uint32_t *)cx.mid_map.ptr, *cursor = (uint32_t *)cx.mid_cursor.ptr;
+    uint32_t *lists = (uint32_t *)cx.mid_lists.ptr;
+    uint16_t *code = (uint16_t *)cx.mid_code.ptr;
+    float *heap = (float *)cx.heap_split.ptr;
+    const float *c[3], *g[3];
+    float *gc[3];
+    for (int k = 0; k < 3; k++) {
+        c[k] = k < D ? cx.coords0(k) : nullptr;
+        g[k] = gc[k] = k < D ? (float *)cx.cx[1][k].ptr : nullptr;
+    }
+    WL *gwt = (WL *)cx.w[1].ptr;
+    // workgroups of a kernel with `lds` bytes each: as many as fit the CUs
+    auto grid_of = [&](auto kernel, uint64_t items, uint32_t lds) {
+        const unsigned by_lds = (unsigned)cx.cu_count * std::max(1u, kSubLds / (lds + 4096));
+        return std::min(persistent_grid(cx, kernel, items), by_lds);
+    };
+    {
+        // 16-bit weights share a word with the count (unless a workgroup's share is large)
+        const bool one_word = packable<WL, Acc>() && n / (uint64_t)cx.cu_count < (1ull << 23);
+        const uint32_t lds = max_cells * (one_word ? 8u : 12u);
+        const unsigned grid = grid_of(k_mid_count<D, WL, Acc>, nt, lds);
+        timed(cx, st, COUPE_HIP_K_HIST, (4.0 * D + sizeof(WL) + 2.0) * (double)n, [&] {
+            k_mid_count<D, WL, Acc><<<grid, kBlock, lds, st>>>(tiles, nt, insts, red, n_inst, c[0], c[1], c[2], w,
+                                                              w_src, code, gcnt, gw, cells, copies);
+        });
+    }
+    // An open node past the register classes is searched by one workgroup from
+    // memory, about 0.55 ns per point and level; the general path takes about
+    // 40 us per level and 50 ps per point of the call.  Beyond half of that
+    // the call takes the general path.
+    const uint64_t most = 36000ull * B.max_levels + n / 22;
+    timed(cx, st, COUPE_HIP_K_DECIDE, 0.0, [&] {
+        const uint32_t lds = mid_tree_lds(B.max_levels);
+        auto launch = [&](auto kernel, int tpb) {
+            allow_lds(kernel, lds);
+            kernel<<<n_inst, tpb, lds, st>>>(insts, red, n_inst, wrap32, gcnt, gw, cells, copies, heap, map, minst,
+                                             open, cursor, lists, cells, most, mid);
+        };
+        if (B.max_levels > 9) launch(k_mid_tree<D, 1024, Acc>, 1024);
+        else launch(k_mid_tree<D, 256, Acc>, 256);
+    });
+    auto search_open = [&] {
+        timed(cx, st, COUPE_HIP_K_PARTITION, 0.0, [&] {
+            const unsigned grid = persistent_grid(cx, k_mid_gather<D, WL>, nt);
+            k_mid_gather<D, WL><<<grid, kBlock, 0, st>>>(tiles, nt, insts, minst, c[0], c[1], c[2], w, w_src, code,
+                                                        map, cursor, gc[0], gc[1], gc[2], gwt, mid);
+        });
+        timed(cx, st, COUPE_HIP_K_HIST, 0.0, [&] {
+            auto launch = [&](auto kernel, int tpb, int k, unsigned per_cu) {
+                const uint32_t lds = sub_lds(B.max_levels, tpb);
+                allow_lds(kernel, lds);
+                const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)cx.cu_count * per_cu, cells);
+                kernel<<<grid, tpb, lds, st>>>(open, lists + k * cells, &mid->of_class[k], insts, g[0], g[1], g[2],
+                                               (const WL *)gwt, wrap32, heap, mid);
+            };
+            launch(k_mid_subtrees<D, 256, 8, WL, Acc>, 256, 0, 2);
+            launch(k_mid_subtrees<D, 512, 16, WL, Acc>, 512, 1, 1);
+            const uint32_t lds = sub_lds(B.max_levels, kMidStreamThreads);
+            allow_lds(k_mid_streams<D, WL, Acc>, lds);
+            const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)cx.cu_count, cells);
+            k_mid_streams<D, WL, Acc><<<grid, kMidStreamThreads, lds, st>>>(
+                open, lists + 2 * cells, &mid->of_class[2], insts, g[0], g[1], g[2], gwt, (uint16_t *)cx.mid_slots.ptr,
+                wrap32, heap, mid);
+        });
+    };
+    auto ids = [&] {
+        const double bytes = 10.0 * (double)n;
+        auto launch = [&](auto kernel) {
+            const unsigned grid = persistent_grid(cx, kernel, nt);
+            timed(cx, st, COUPE_HIP_K_IDS, bytes, [&] {
+                kernel<<<grid, kBlock, 0, st>>>(tiles, nt, insts, minst, code, map, heap, c[0], c[1], c[2], d_out, mid);
+            });
+        };
+        // non-temporal ids for calls the caches cannot hold (see run_levels' descent)
+        if ((4.0 * D + 8.0) * (double)n > cx.move_nt_bytes) launch(k_mid_ids<D, true>);
+        else launch(k_mid_ids<D, false>);
+    };
+    auto wait = [&] {
+        char *h_rb = (char *)cx.host_scratch + 256;
+        const size_t off = offsetof(Counters, swept);
+        check(hipMemcpyAsync(h_rb, (char *)ctr + off, offsetof(Counters, spec) - off, hipMemcpyDeviceToHost, st));
+        check(hipStreamSynchronize(st));
+        return *(const MidCounters *)(h_rb + (offsetof(Counters, mid) - off));
+    };
+    // a shape whose last call left no node open queues no search; open nodes
+    // after all are searched once the counters are read
+    const Hints *seen = cx.hints_for(B.shape);
+    const bool expect = !seen || seen->mid < 0 || seen->mid_open > 0;
+    if (expect) search_open();
+    ids();
+    MidCounters m = wait();
+    if (!expect && m.open && !m.big) {
+        cx.stats.reruns = 1;
+        search_open();
+        ids();
+        m = wait();
+    }
+    if (m.error) throw HipFailure{hipErrorUnknown};
+    cx.mid_clean = true;
+    cx.pending.shape = B.shape;
+    Hints &h = cx.remember(B.shape);
+    h.mid = m.big ? 0 : 1;
+    h.mid_open = m.open;
+    if (m.big) return false;
+    cx.stats.levels = B.max_levels;
+    cx.stats.passes = B.max_levels;
+    cx.stats.max_passes = std::max(cx.stats.max_passes, 1u);
+    cx.stats.unit_points = kTile;
+    cx.stats.bins = m.open ? (uint32_t)kSubMaxNb : 2u;
+    return true;
+}
+
 template <int D, typename WIN>
 static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchPlan &B, const double *pts,
                       const WIN *win, int wkind, int spec_passes) {
@@ -1128,6 +1305,21 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
         }
         cx.pending.mode = mode;
         cx.pending.wkind = wkind;
+        if (mid_fits(cx, B, spec_passes)) {
+            cx.stats.weight_mode = mode == 3 ? 1 : 0;
+            cx.stats.weight_bytes = weight_bytes(mode);
+            bool done;
+            if (mode == 0) done = run_mid<D, uint16_t, uint64_t>(cx, st, B, wrap32, d_out, (uint16_t *)cx.w16.ptr, 0);
+            else if (mode == 1) done = run_mid<D, int32_t, uint64_t>(cx, st, B, wrap32, d_out, (int32_t *)cx.w[0].ptr, 0);
+            else if (mode == 2) done = run_mid<D, WIN, uint64_t>(cx, st, B, wrap32, d_out, win, 1);
+            else if constexpr (std::is_same<WIN, double>::value)
+                done = run_mid<D, WIN, double>(cx, st, B, 0, d_out, win, 1);
+            else
+                done = false;   // (integers never need f64 sums)
+            if (!mode_held(cx)) continue;
+            if (done) return false;
+            cx.stats.reruns = 1;   // on the general path, from the prologue's arrays
+        }
         const bool unfinished = run_mode(mode);
         if (cx.capturing) return false;   // checked once the graph has run
         if (!mode_held(cx)) continue;     // complete: run_levels waited for the stream
@@ -1348,9 +1540,7 @@ static void launch_small(Context &cx, hipStream_t st, const std::vector<SmallPro
         const float *c0 = cx.slot0[0], *c1 = cx.slot0[1], *c2 = cx.slot0[2];
         auto launch = [&](auto kernel, int tpb) {
             const uint32_t lds = sub_lds(levels, tpb);
-            if (lds > 65536)
-                check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            allow_lds(kernel, lds);
             // algorithmic bytes: points and weights read, ids written
             timed(cx, st, COUPE_HIP_K_OTHER, points * (8.0 * D + sizeof(WIN) + 8.0), [&] {
                 kernel<<<(unsigned)(end - at), tpb, lds, st>>>(problems[at], table ? table + at : nullptr, pts, c0, c1,
@@ -1752,6 +1942,7 @@ void Context::for_each_buf(F &&f) {
                      &tile_bins2, &tile4, &bcnt, &bw, &bmin, &xcnt, &xw, &xmin, &nchild, &ntiles, &bsum, &nodes, &leaf,
                      &heap_split, &instances, &tiles0, &below, &tile_left, &loads, &rib_moments, &tile_bins,
                      &gparts[0], &gparts[1], &gaxis, &gchunk, &gcount, &gctr, &gsat, &gcol, &grow, &gheap, &gscan,
+                     &mid_code, &mid_cnt, &mid_w, &mid_map, &mid_inst, &mid_open, &mid_cursor, &mid_lists, &mid_slots,
                      &small_table, &small_report, &ired, &counters, &in_points, &in_weights, &out_ids};
     for (DevBuf *d : all) f(*d);
 }

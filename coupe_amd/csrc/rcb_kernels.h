@@ -454,7 +454,7 @@ k_sweep(const Part *__restrict__ parts, const Tile *__restrict__ tiles, const ui
 constexpr int kPackShift = 40;
 
 template <typename WS, typename Acc>
-__device__ __forceinline__ constexpr bool packable() {
+__host__ __device__ constexpr bool packable() {
     return std::is_same<WS, uint16_t>::value && std::is_same<Acc, uint64_t>::value;
 }
 

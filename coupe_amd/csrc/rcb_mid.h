@@ -1,0 +1,645 @@
+// rcb_mid.h -- all levels of a call from one sweep over its points, where the
+// parts split at the middle of their box.
+//
+// coupe's search starts at the midpoint of a part's box and ends there when
+// the halves balance within the tolerance: the usual case on meshes, all the
+// way down on regular ones.  The general path finds that out level by level
+// and moves the points every two levels.  Here the tree of midpoints is laid
+// out ahead (it depends on the root's box alone), one sweep counts and weighs
+// the points of each of its 2^L cells, and the sums up the tree settle, node
+// by node from the root, whether coupe's loop ends at the midpoint: then that
+// node's split is exactly coupe's.  A node whose search goes on is *open*;
+// its ancestors are settled, so its box, points and weight are coupe's.  The
+// points of the open nodes are gathered and each subtree is searched by one
+// workgroup (rcb_subtree.h).  The ids come from each point's cell, or from a
+// walk down the searched splits below an open node.
+//
+// Bound by memory: 4 D + w bytes read and 2 written per point by the sweep,
+// 10 by the ids, besides the open points; the levels' moves (2 (4 D + w) per
+// two levels) and passes are not made.  2^27 points 3D, 12 levels, 16-bit
+// weights: see k_mid_count and k_mid_ids.
+#pragma once
+
+#include "rcb_small.h"
+
+namespace coupe_hip {
+
+constexpr uint32_t kMidLevels = 12;            // most levels: 4096 cells, two 16-bit halves of a map entry
+constexpr uint32_t kMidDone = 0xffffffffu;     // map: the cell's points are settled
+constexpr uint32_t kMidClasses = 3;            // open nodes of at most 2048 and 8192 points, and larger
+constexpr uint32_t kMidClass[2] = {256 * 8, 512 * 16};
+
+// An open node: its points are gathered at [begin, begin + count).
+struct MidOpen {
+    uint64_t sum;            // weight, accumulator bits
+    float lo[kMaxDim], hi[kMaxDim];
+    uint32_t begin, count;
+    uint32_t node;           // heap index in its instance
+    uint32_t inst;
+    uint32_t axis, levels;   // axis of its split, levels left
+};
+
+// Counters of a call on this path (among the call's counters).
+struct MidCounters {
+    uint32_t open;                  // open nodes
+    uint32_t points;                // their points
+    uint32_t of_class[kMidClasses];
+    uint32_t big;                   // open nodes too large for a workgroup: the call takes the general path
+    uint32_t error;                 // a subtree's search did not end
+    uint32_t pad;
+};
+
+// An instance's figures on this path: its open nodes are
+// [first_open, first_open + n_open) of the table.
+struct MidInstance {
+    uint32_t first_open, n_open;
+};
+
+__device__ __forceinline__ uint64_t mid_cell_base(const Instance &I, uint32_t q) { return I.heap_base + q; }
+__device__ __forceinline__ uint32_t mid_axis_levels(uint32_t levels, int a, int dim) {
+    return (levels + (uint32_t)(dim - 1 - a)) / (uint32_t)dim;
+}
+
+// Box of an instance's root from the prologue's copies, as f32 (:604-605).
+template <int D>
+__device__ __forceinline__ void mid_box(const InstReduce *__restrict__ red, uint32_t n_inst, uint32_t q, int a,
+                                        float &lo, float &hi) {
+    uint64_t l = ~0ull, h = 0;
+    for (int c = 0; c < kCopies; c++) {
+        const InstReduce &r = red[(uint64_t)c * n_inst + q];
+        l = r.bmin[a] < l ? r.bmin[a] : l;
+        h = r.bmax[a] > h ? r.bmax[a] : h;
+    }
+    lo = (float)key_f64(l);
+    hi = (float)key_f64(h);
+}
+
+// ---------------------------------------------------------------------------
+// The sweep.  Per axis the midpoints of its levels, sorted; a point's rank
+// among them gives its bits of the cell's path, spread to the levels of that
+// axis.  Entry r of an axis: midpoint below, midpoint above (NaN past the
+// ends), spread bits.
+// ---------------------------------------------------------------------------
+constexpr int kMidRanks = 1 << (kMidLevels / 2);   // of an axis: 64 in 2D, 16 in 3D
+
+struct MidTables {
+    float4 rank[kMaxDim][kMidRanks];
+    float lo[kMaxDim], hi[kMaxDim];
+};
+
+template <int D>
+__device__ __forceinline__ void mid_tables(MidTables &T, uint32_t levels) {
+    constexpr float nan = __builtin_nanf("");
+    for (int a = 0; a < D; a++) {
+        const uint32_t la = mid_axis_levels(levels, a, D), n = 1u << la;
+        for (uint32_t r = threadIdx.x; r < n; r += kBlock) {
+            uint32_t bits = 0;
+            for (uint32_t j = 0; j < la; j++)
+                bits |= ((r >> (la - 1 - j)) & 1u) << (levels - 1 - (uint32_t)a - j * D);
+            T.rank[a][r] = make_float4(r ? candidate(T.lo[a], T.hi[a], (int)r - 1, (int)n) : nan,
+                                       r + 1 < n ? candidate(T.lo[a], T.hi[a], (int)r, (int)n) : nan,
+                                       __builtin_bit_cast(float, bits), 0.0f);
+        }
+    }
+}
+
+// The spread bits of x on an axis of n ranks: the rank by an estimate, moved
+// while the midpoints around it say so (whole wavefronts; seldom at all, at
+// most n times).  NaN: rank 0, like !(c >= t).
+__device__ __forceinline__ uint32_t mid_rank(const float4 *rank, int n, float x, float lo, float scale) {
+    const float e = (x - lo) * scale;
+    int r = (int)fminf(fmaxf(e, 0.0f), (float)(n - 1));
+    float4 t = rank[r];
+    for (int it = 0; it < n; it++) {
+        const bool down = x < t.x, up = x >= t.y;
+        if (__ballot(down | up) == 0) break;
+        r += (up ? 1 : 0) - (down ? 1 : 0);
+        t = rank[r];
+    }
+    return __builtin_bit_cast(uint32_t, t.z);
+}
+
+// w: the stored weights (w_src 0) or the caller's (w_src 1, 64-bit weights
+// are not stored on this path).  cells: per copy (copies of them), the count
+// and weight of every instance's cells.  code: each point's cell.
+template <int D, typename WL, typename Acc>
+__global__ void __launch_bounds__(kBlock)
+k_mid_count(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__restrict__ insts,
+            const InstReduce *__restrict__ red, uint32_t n_inst, const float *__restrict__ c0,
+            const float *__restrict__ c1, const float *__restrict__ c2, const WL *__restrict__ w, int w_src,
+            uint16_t *__restrict__ code, uint32_t *__restrict__ gcnt, Acc *__restrict__ gw, uint64_t cells,
+            uint32_t copies) {
+    __shared__ MidTables T;
+    extern __shared__ __align__(16) char mid_lds[];
+    uint32_t t0, t1;
+    tile_range(n_tiles, t0, t1);
+    if (t0 >= t1) return;
+    // 16-bit weights: count and weight of a cell in one word (a workgroup's
+    // share stays below 2^24 points)
+    const bool packed = packable<WL, Acc>() && (uint64_t)(t1 - t0) * kTile < (1ull << 24);
+    Acc *sw = (Acc *)mid_lds;
+    uint32_t *sc = nullptr;
+    const int tid = threadIdx.x;
+    uint32_t cur = 0xffffffffu, levels = 0, n_cells = 0;
+    uint64_t gbase = 0, wbase = 0;
+    float lo[D], scale[D];
+    int ranks[D];
+    auto flush = [&]() {
+        for (uint32_t c = tid; c < n_cells; c += kBlock) {
+            uint32_t cnt;
+            Acc sum = sw[c];
+            if (packed) {
+                if constexpr (std::is_same<Acc, uint64_t>::value) {
+                    cnt = (uint32_t)(sum >> kPackShift);
+                    sum &= (1ull << kPackShift) - 1;
+                } else {
+                    cnt = sc[c];
+                }
+            } else {
+                cnt = sc[c];
+            }
+            if (cnt) {
+                atomicAdd(&gcnt[gbase + c], cnt);
+                atomic_add_acc(&gw[gbase + c], sum);
+            }
+        }
+    };
+    for (uint32_t t = t0; t < t1; t++) {
+        const Tile U = tiles[t];
+        if (U.part != cur) {
+            __syncthreads();
+            if (cur != 0xffffffffu) flush();
+            cur = U.part;
+            const Instance &I = insts[cur];
+            levels = I.levels;
+            n_cells = 1u << levels;
+            gbase = (uint64_t)(blockIdx.x % copies) * cells + mid_cell_base(I, cur);
+            wbase = w_src ? I.src - I.begin : 0;   // (wraps: added to positions of the instance)
+            sc = (uint32_t *)(mid_lds + (uint64_t)n_cells * sizeof(Acc));
+            if (tid < D) mid_box<D>(red, n_inst, cur, tid, T.lo[tid], T.hi[tid]);
+            __syncthreads();
+            mid_tables<D>(T, levels);
+            for (uint32_t c = tid; c < n_cells; c += kBlock) {
+                sw[c] = (Acc)0;
+                if (!packed) sc[c] = 0;
+            }
+#pragma unroll
+            for (int a = 0; a < D; a++) {
+                ranks[a] = 1 << mid_axis_levels(levels, a, D);
+                lo[a] = T.lo[a];
+                scale[a] = (float)ranks[a] / (T.hi[a] - T.lo[a]);
+            }
+            __syncthreads();
+        }
+        // every load of the tile issued first (clamped, unconditional)
+        float x[kItems][D];
+        WL wk[kItems];
+#pragma unroll
+        for (int k = 0; k < kItems; k++) {
+            const uint64_t i = U.begin + min((uint32_t)(k * kBlock + tid), U.count - 1u);
+            x[k][0] = c0[i];
+            x[k][1] = c1[i];
+            if constexpr (D == 3) x[k][2] = c2[i];
+            wk[k] = w[wbase + i];
+        }
+#pragma unroll
+        for (int k = 0; k < kItems; k++) {
+            uint32_t c = 0;
+#pragma unroll
+            for (int a = 0; a < D; a++) c |= mid_rank(T.rank[a], ranks[a], x[k][a], lo[a], scale[a]);
+            const uint32_t p = (uint32_t)(k * kBlock + tid);
+            if (p >= U.count) continue;
+            code[U.begin + p] = (uint16_t)c;
+            if (packed) {
+                if constexpr (std::is_same<Acc, uint64_t>::value)
+                    atomicAdd((unsigned long long *)&sw[c],
+                              (1ull << kPackShift) + (unsigned long long)AccOps<Acc>::of(wk[k]));
+            } else {
+                atomicAdd(&sc[c], 1u);
+                atomic_add_acc(&sw[c], AccOps<Acc>::of(wk[k]));
+            }
+        }
+    }
+    __syncthreads();
+    flush();
+}
+
+// ---------------------------------------------------------------------------
+// The tree: one workgroup per instance sums the cells up the tree (the copies
+// are left clear), settles the nodes from the root down, and lists the open
+// ones.  map: per cell the open node above it (heap index, and its number
+// among the instance's open nodes << 16), or kMidDone.
+// ---------------------------------------------------------------------------
+constexpr uint32_t mid_tree_lds(uint32_t levels) { return (1u << levels) * (2 * 12 + 4); }
+
+template <int D, int TPB, typename Acc>
+__global__ void __launch_bounds__(TPB)
+k_mid_tree(Instance *__restrict__ insts, const InstReduce *__restrict__ red, uint32_t n_inst, int wrap32,
+           uint32_t *__restrict__ gcnt, Acc *__restrict__ gw, uint64_t cells, uint32_t copies,
+           float *__restrict__ heap_split, uint32_t *__restrict__ map, MidInstance *__restrict__ minst,
+           MidOpen *__restrict__ open, uint32_t *__restrict__ cursor, uint32_t *__restrict__ lists, uint64_t list_stride,
+           uint64_t most, MidCounters *ctr) {
+    using Ops = AccOps<Acc>;
+    extern __shared__ __align__(16) char mid_lds[];
+    __shared__ float s_lo[kMaxDim], s_hi[kMaxDim];
+    __shared__ uint32_t s_open, s_first, s_min;
+    const uint32_t q = blockIdx.x, tid = threadIdx.x;
+    Instance &I = insts[q];
+    const uint32_t levels = __builtin_amdgcn_readfirstlane(I.levels), n_cells = 1u << levels;
+    const uint64_t cbase = mid_cell_base(I, q), hb = I.heap_base;
+    Acc *w = (Acc *)mid_lds;                          // by heap index, 2 n_cells - 1 of each
+    uint32_t *cnt = (uint32_t *)(w + 2 * n_cells);
+    uint32_t *state = cnt + 2 * n_cells;              // 0: no point or above it open, 1: settled, 2 + number: open
+    if (tid < (uint32_t)D) mid_box<D>(red, n_inst, q, (int)tid, s_lo[tid], s_hi[tid]);
+    if (tid == 0) {
+        s_open = 0;
+        s_min = 0xffffffffu;
+    }
+    for (uint32_t c = tid; c < n_cells; c += TPB) {
+        uint32_t n = 0;
+        Acc s = (Acc)0;
+        for (uint32_t k = 0; k < copies; k++) {
+            const uint64_t g = (uint64_t)k * cells + cbase + c;
+            n += gcnt[g];
+            s += gw[g];
+            gcnt[g] = 0;
+            gw[g] = (Acc)0;
+        }
+        cnt[n_cells - 1 + c] = n;
+        w[n_cells - 1 + c] = s;
+    }
+    __syncthreads();
+    for (int l = (int)levels - 1; l >= 0; l--) {
+        for (uint32_t s = tid; s < 1u << l; s += TPB) {
+            const uint32_t h = (1u << l) - 1 + s;
+            cnt[h] = cnt[2 * h + 1] + cnt[2 * h + 2];
+            w[h] = w[2 * h + 1] + w[2 * h + 2];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {   // the root's weight as the general path has it
+        uint64_t su = 0;
+        double sf = 0.0;
+        for (int c = 0; c < kCopies; c++) {
+            su += red[(uint64_t)c * n_inst + q].sum_u64;
+            sf += red[(uint64_t)c * n_inst + q].sum_f64;
+        }
+        if constexpr (std::is_same<Acc, double>::value) w[0] = sf;
+        else w[0] = su;
+    }
+    __syncthreads();
+    float lo[kMaxDim], hi[kMaxDim];
+    bool finite = true;   // and so is every midpoint
+#pragma unroll
+    for (int a = 0; a < kMaxDim; a++) {
+        lo[a] = a < D ? s_lo[a] : 0.0f;
+        hi[a] = a < D ? s_hi[a] : 0.0f;
+        finite = finite && fabsf(lo[a]) < 1.0e38f && fabsf(hi[a]) < 1.0e38f;
+    }
+    const double tol = I.tol;
+    // the box of node (l, s) on axis a: the bisections of its ancestors there
+    auto window = [&](uint32_t l, uint32_t s, int a, float &bl, float &bh) {
+        bl = sel3(a, lo[0], lo[1], lo[2]);
+        bh = sel3(a, hi[0], hi[1], hi[2]);
+        for (uint32_t m = (uint32_t)a; m < l; m += D) {
+            const float t = (bl + bh) / 2.0f;
+            const bool right = (s >> (l - m - 1)) & 1u;
+            bl = right ? t : bl;
+            bh = right ? bh : t;
+        }
+    };
+    for (uint32_t l = 0; l < levels; l++) {
+        for (uint32_t s = tid; s < 1u << l; s += TPB) {
+            const uint32_t h = (1u << l) - 1 + s, n = cnt[h];
+            const bool live = n > 0 && (l == 0 || state[(h - 1) / 2] == 1u);
+            uint32_t st = 0;
+            if (live) {
+                const uint32_t cl = cnt[2 * h + 1];
+                const Acc S = w[h], wl = w[2 * h + 1];
+                if (finite && cl != n && within(Ops::f64(wl, wrap32), Ops::f64(S, wrap32) / 2.0, tol)) {
+                    float bl, bh;
+                    window(l, s, (int)(l % D), bl, bh);
+                    heap_split[hb + h] = (bl + bh) / 2.0f;
+                    w[2 * h + 2] = Ops::sub(S, wl);   // the right child's weight (:603-641)
+                    st = 1;
+                } else {
+                    st = 2u + atomicAdd(&s_open, 1u);
+                }
+            }
+            state[h] = st;
+        }
+        __syncthreads();
+    }
+    const uint32_t n_open = s_open;
+    if (tid == 0) {
+        s_first = n_open ? atomicAdd(&ctr->open, n_open) : 0u;
+        minst[q] = MidInstance{s_first, n_open};
+    }
+    __syncthreads();
+    const uint32_t first = s_first;
+    for (uint32_t h = tid; h < n_cells - 1; h += TPB) {
+        const uint32_t st = state[h];
+        if (st < 2) continue;
+        const uint32_t l = 31u - (uint32_t)__builtin_clz(h + 1), s = h + 1 - (1u << l), e = first + st - 2;
+        MidOpen O;
+        O.sum = Ops::to_bits(w[h]);
+        O.count = cnt[h];
+        O.begin = atomicAdd(&ctr->points, O.count);
+        O.node = h;
+        O.inst = q;
+        O.axis = l % D;
+        O.levels = levels - l;
+        for (int a = 0; a < kMaxDim; a++) {
+            O.lo[a] = O.hi[a] = 0.0f;
+            if (a < D) window(l, s, a, O.lo[a], O.hi[a]);
+        }
+        open[e] = O;
+        cursor[e] = O.begin;
+        const uint32_t k = O.count <= kMidClass[0] ? 0u : (O.count <= kMidClass[1] ? 1u : 2u);
+        lists[k * list_stride + atomicAdd(&ctr->of_class[k], 1u)] = e;
+        if (O.count > kMidClass[1] && (uint64_t)O.count * O.levels > most) atomicAdd(&ctr->big, 1u);
+    }
+    uint32_t m = 0xffffffffu;   // smallest settled leaf
+    for (uint32_t c = tid; c < n_cells; c += TPB) {
+        uint32_t entry = kMidDone;
+        for (uint32_t l = 0; l < levels; l++) {
+            const uint32_t h = (1u << l) - 1 + (c >> (levels - l)), st = state[h];
+            if (st != 1u) {
+                if (st >= 2u) entry = h | (st - 2u) << 16;
+                break;
+            }
+        }
+        map[cbase + c] = entry;
+        if (entry == kMidDone && cnt[n_cells - 1 + c]) m = min(m, n_cells - 1 + c);
+    }
+    m = wave_min(m);
+    if (lane_id() == 0) atomicMin(&s_min, m);
+    __syncthreads();
+    if (tid == 0) I.min_id = s_min == 0xffffffffu ? ~0ull : (uint64_t)s_min;   // (the subtrees lower it)
+}
+
+// ---------------------------------------------------------------------------
+// The open nodes' points, gathered node by node (their order within a node is
+// free).  Workgroups take contiguous shares of the tiles: each counts its
+// points per open node, takes places for them (one atomic per node) and
+// writes them, reading the 2-byte cells twice.
+// ---------------------------------------------------------------------------
+template <int D, typename WL>
+__global__ void __launch_bounds__(kBlock)
+k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__restrict__ insts,
+             const MidInstance *__restrict__ minst, const float *__restrict__ c0, const float *__restrict__ c1,
+             const float *__restrict__ c2, const WL *__restrict__ w, int w_src, const uint16_t *__restrict__ code,
+             const uint32_t *__restrict__ map, uint32_t *__restrict__ cursor, float *__restrict__ o0,
+             float *__restrict__ o1, float *__restrict__ o2, WL *__restrict__ ow, const MidCounters *ctr) {
+    if (ctr->open == 0 || ctr->big) return;
+    __shared__ uint16_t num[1 << kMidLevels];            // open node of a cell, 0xffff: settled
+    __shared__ uint32_t place[1 << (kMidLevels - 1)];    // at most half as many open nodes as cells
+    const int tid = threadIdx.x;
+    uint32_t t0, t1;
+    tile_range(n_tiles, t0, t1);
+    for (uint32_t t = t0; t < t1;) {
+        const uint32_t q = tiles[t].part;
+        uint32_t e = t;   // [t, e): this share's tiles of instance q
+        const Instance &I = insts[q];
+        {
+            const uint32_t last = I.tile_begin + (uint32_t)((I.count + kTile - 1) / kTile);
+            e = last < t1 ? last : t1;
+        }
+        const MidInstance M = minst[q];
+        if (M.n_open == 0) {
+            t = e;
+            continue;
+        }
+        const uint32_t n_cells = 1u << I.levels;
+        const uint64_t cbase = mid_cell_base(I, q), wbase = w_src ? I.src - I.begin : 0;
+        __syncthreads();
+        for (uint32_t c = tid; c < n_cells; c += kBlock) {
+            const uint32_t m = map[cbase + c];
+            num[c] = m == kMidDone ? (uint16_t)0xffffu : (uint16_t)(m >> 16);
+        }
+        for (uint32_t k = tid; k < M.n_open; k += kBlock) place[k] = 0;
+        __syncthreads();
+        const uint64_t begin = tiles[t].begin, end = tiles[e - 1].begin + tiles[e - 1].count;
+        for (uint64_t i = begin + tid; i < end; i += kBlock) {
+            const uint16_t o = num[code[i]];
+            if (o != 0xffffu) atomicAdd(&place[o], 1u);
+        }
+        __syncthreads();
+        for (uint32_t k = tid; k < M.n_open; k += kBlock)
+            if (place[k]) place[k] = atomicAdd(&cursor[M.first_open + k], place[k]);
+        __syncthreads();
+        for (uint64_t i = begin + tid; i < end; i += kBlock) {
+            const uint16_t o = num[code[i]];
+            if (o == 0xffffu) continue;
+            const uint32_t d = atomicAdd(&place[o], 1u);
+            o0[d] = c0[i];
+            o1[d] = c1[i];
+            if constexpr (D == 3) o2[d] = c2[i];
+            ow[d] = w[wbase + i];
+        }
+        t = e;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The open nodes' subtrees, one workgroup each.
+// ---------------------------------------------------------------------------
+// Root of an open node's subtree, and where its splits go.
+template <typename WL>
+__device__ __forceinline__ SubRoot mid_root(const MidOpen &O, const Instance &I, int wrap32) {
+    SubRoot R;
+    for (int a = 0; a < kMaxDim; a++) { R.lo[a] = O.lo[a]; R.hi[a] = O.hi[a]; }
+    R.axis = __builtin_amdgcn_readfirstlane(O.axis);
+    R.levels = __builtin_amdgcn_readfirstlane(O.levels);
+    R.tol = I.tol;
+    R.wrap32 = wrap32;
+    R.packed = std::is_same<WL, uint16_t>::value && O.count < (1u << 24);
+    return R;
+}
+
+// split_out of a subtree: the split into the instance's heap (its heap index
+// from the subtree's), and at the last level the smallest leaf present.
+struct MidSplits {
+    float *heap;         // the instance's heap
+    uint32_t node;       // heap index of the subtree's root
+    uint32_t levels;     // of the subtree
+    uint32_t *min_leaf;  // LDS
+    __device__ __forceinline__ void operator()(uint32_t level, uint32_t slot, uint32_t n, uint32_t left,
+                                               float split) const {
+        if (n == 0) return;
+        const uint32_t h = ((node + 1) << level) - 1 + slot;
+        heap[h] = left == n ? __builtin_nanf("") : split;   // every point left: as the descent walks it
+        if (level + 1 == levels) atomicMin(min_leaf, left ? 2 * h + 1 : 2 * h + 2);
+    }
+};
+
+// Points in registers: the nodes of one class.
+template <int D, int TPB, int IT, typename WL, typename Acc>
+__global__ void __launch_bounds__(TPB)
+k_mid_subtrees(const MidOpen *__restrict__ open, const uint32_t *__restrict__ list, const uint32_t *n_list,
+               Instance *__restrict__ insts, const float *__restrict__ c0, const float *__restrict__ c1,
+               const float *__restrict__ c2, const WL *__restrict__ w, int wrap32, float *__restrict__ heap_split,
+               MidCounters *ctr) {
+    if (ctr->big) return;
+    SmallShared &sh = *(SmallShared *)sub_lds_base;
+    const uint32_t n = *n_list;
+    for (uint32_t g = blockIdx.x; g < n; g += gridDim.x) {
+        const MidOpen &O = open[list[g]];
+        Instance &I = insts[O.inst];
+        const uint32_t count = __builtin_amdgcn_readfirstlane(O.count), begin = __builtin_amdgcn_readfirstlane(O.begin);
+        const SubRoot R = mid_root<WL>(O, I, wrap32);
+        float x[IT][D];
+        small_points<D, TPB, IT>(count, x, [&](uint64_t i, float (&p)[D]) {
+            p[0] = c0[begin + i];
+            p[1] = c1[begin + i];
+            if constexpr (D == 3) p[2] = c2[begin + i];
+        });
+        __syncthreads();   // the last node's LDS is free
+        if (threadIdx.x == 0) sh.min_slot = 0xffffffffu;
+        const MidSplits out{heap_split + I.heap_base, O.node, R.levels, &sh.min_slot};
+        RegSlots<IT> slot;
+        const bool ok = reg_levels<D, TPB, IT, kWeightAcc, WL, Acc>(count, x, w + begin, R,
+                                                                    AccOps<Acc>::from_bits(O.sum), sh.ctr, slot, out);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            atomicMin((unsigned long long *)&I.min_id, (unsigned long long)sh.min_slot);
+            if (!ok) atomicOr(&ctr->error, 1u);
+        }
+    }
+}
+
+// Larger nodes: the points stay in memory (a node's are read again per pass,
+// from the caches), their slots beside them.
+constexpr int kMidStreamThreads = 1024;
+template <int D, typename WL, typename Acc>
+__global__ void __launch_bounds__(kMidStreamThreads)
+k_mid_streams(const MidOpen *__restrict__ open, const uint32_t *__restrict__ list, const uint32_t *n_list,
+              Instance *__restrict__ insts, const float *__restrict__ c0, const float *__restrict__ c1,
+              const float *__restrict__ c2, const WL *__restrict__ w, uint16_t *__restrict__ slots, int wrap32,
+              float *__restrict__ heap_split, MidCounters *ctr) {
+    if (ctr->big) return;
+    constexpr int TPB = kMidStreamThreads, B = kAhead;
+    SmallShared &sh = *(SmallShared *)sub_lds_base;
+    const uint32_t n = *n_list, tid = threadIdx.x;
+    for (uint32_t g = blockIdx.x; g < n; g += gridDim.x) {
+        const MidOpen &O = open[list[g]];
+        Instance &I = insts[O.inst];
+        const uint32_t count = __builtin_amdgcn_readfirstlane(O.count), begin = __builtin_amdgcn_readfirstlane(O.begin);
+        const SubRoot R = mid_root<WL>(O, I, wrap32);
+        __syncthreads();   // the last node's LDS is free
+        if (tid == 0) sh.min_slot = 0xffffffffu;
+        const MidSplits out{heap_split + I.heap_base, O.node, R.levels, &sh.min_slot};
+        SubTree<Acc, TPB> T(sub_slots(R.levels));
+        uint16_t *sl = slots + begin;
+        const WL *wp = w + begin;
+        bool first = true;   // every point in slot 0: not read
+        const bool ok = sub_levels<D, TPB, Acc>(
+            T, R, count, AccOps<Acc>::from_bits(O.sum), sh.ctr,
+            [&](int nb, int a) {
+                const float *c = (a == 0 ? c0 : (a == 1 ? c1 : c2)) + begin;
+                for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
+                    uint32_t s[B];
+                    float xa[B];
+                    Acc wk[B];
+                    bool valid[B];
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        const uint32_t i = i0 + (uint32_t)(j * TPB) + tid, p = i < count ? i : count - 1;
+                        valid[j] = i < count;
+                        xa[j] = c[p];
+                        wk[j] = AccOps<Acc>::of(wp[p]);
+                        s[j] = first ? 0u : (uint32_t)sl[p];
+                    }
+                    sub_bin<B, TPB, Acc>(T, s, xa, wk, valid, nb, R.packed);
+                }
+            },
+            [&](int a) {
+                const float *c = (a == 0 ? c0 : (a == 1 ? c1 : c2)) + begin;
+                for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        const uint32_t i = i0 + (uint32_t)(j * TPB) + tid;
+                        if (i < count) {   // (each thread its own points: no other reads them)
+                            const uint32_t s = first ? 0u : (uint32_t)sl[i];
+                            sl[i] = (uint16_t)(2 * s + (c[i] >= T.at(s).win.x ? 1u : 0u));
+                        }
+                    }
+                }
+                first = false;
+            },
+            out);
+        __syncthreads();
+        if (tid == 0) {
+            atomicMin((unsigned long long *)&I.min_id, (unsigned long long)sh.min_slot);
+            if (!ok) atomicOr(&ctr->error, 1u);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Ids in input order: a settled cell is its leaf; below an open node the
+// point walks the searched splits (the tile's coordinates are read only then).
+// ---------------------------------------------------------------------------
+template <int D, bool NT>
+__global__ void __launch_bounds__(kBlock)
+k_mid_ids(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__restrict__ insts,
+          const MidInstance *__restrict__ minst, const uint16_t *__restrict__ code, const uint32_t *__restrict__ map,
+          const float *__restrict__ heap_split, const float *__restrict__ c0, const float *__restrict__ c1,
+          const float *__restrict__ c2, uint64_t *__restrict__ out, const MidCounters *ctr) {
+    if (ctr->big) return;
+    __shared__ uint16_t node[1 << kMidLevels];   // open node of a cell, 0xffff: settled
+    const int tid = threadIdx.x;
+    uint32_t t0, t1;
+    tile_range(n_tiles, t0, t1);
+    uint32_t cur = 0xffffffffu, levels = 0, leaf0 = 0;
+    uint64_t off = 0, src = 0;
+    const float *heap = heap_split;
+    bool any_open = false;
+    for (uint32_t t = t0; t < t1; t++) {
+        const Tile U = tiles[t];
+        if (U.part != cur) {
+            cur = U.part;
+            const Instance &I = insts[cur];
+            levels = I.levels;
+            leaf0 = (1u << levels) - 1;
+            off = I.min_id;
+            src = I.src - I.begin;
+            heap = heap_split + I.heap_base;
+            any_open = minst[cur].n_open != 0;
+            if (any_open) {
+                const uint64_t cbase = mid_cell_base(I, cur);
+                __syncthreads();
+                for (uint32_t c = tid; c <= leaf0; c += kBlock) node[c] = (uint16_t)map[cbase + c];   // kMidDone: 0xffff
+                __syncthreads();
+            }
+        }
+        uint32_t c[kItems];
+#pragma unroll
+        for (int k = 0; k < kItems; k++) {
+            const uint64_t i = U.begin + min((uint32_t)(k * kBlock + tid), U.count - 1u);
+            if constexpr (NT) c[k] = __builtin_nontemporal_load(&code[i]);
+            else c[k] = code[i];
+        }
+#pragma unroll
+        for (int k = 0; k < kItems; k++) {
+            const uint32_t p = (uint32_t)(k * kBlock + tid);
+            if (p >= U.count) continue;
+            const uint64_t i = U.begin + p;
+            uint32_t h = leaf0 + c[k];
+            if (any_open && node[c[k]] != 0xffffu) {
+                h = node[c[k]];
+                uint32_t l = 31u - (uint32_t)__builtin_clz(h + 1);
+                const float x0 = c0[i], x1 = c1[i], x2 = D == 3 ? c2[i] : 0.0f;
+                int a = (int)(l % D);
+                for (; l < levels; l++) {
+                    h = 2 * h + (sel3(a, x0, x1, x2) >= heap[h] ? 2u : 1u);
+                    a = a + 1 == D ? 0 : a + 1;
+                }
+            }
+            if constexpr (NT) __builtin_nontemporal_store((uint64_t)h - off, &out[src + i]);
+            else out[src + i] = (uint64_t)h - off;
+        }
+    }
+}
+
+}  // namespace coupe_hip

@@ -73,38 +73,45 @@ enum : int { kWeightAcc, kWeight16, kWeightLoad };
 constexpr int kAhead = 4;   // points of a lane whose lookups are issued together
 constexpr int kLoad = 8;    // points of a lane loaded together
 
-// The levels of one small problem with the points in registers; their slots
-// two to a register.  Points are taken kAhead at a time, up to the uniform end.
-template <int D, int TPB, int IT, int KW, typename WIN, typename Acc>
-__device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x)[IT][D], const WIN *__restrict__ win,
-                                          const SubRoot &R, Acc sum, SmallShared &sh,
-                                          uint64_t *__restrict__ out, uint32_t kind, uint32_t *report) {
+// The levels of a subtree of `count` points in registers, their weights in
+// win; the slots two to a register.  Points are taken kAhead at a time, up to
+// the uniform end.
+template <int IT>
+struct RegSlots {
+    uint32_t two[IT / 2];
+    __device__ __forceinline__ uint32_t operator()(int k) const {
+        return k & 1 ? two[k / 2] >> 16 : two[k / 2] & 0xffffu;
+    }
+};
+template <int D, int TPB, int IT, int KW, typename WIN, typename Acc, typename Split>
+__device__ __forceinline__ bool reg_levels(uint32_t count, const float (&x)[IT][D], const WIN *__restrict__ win,
+                                           const SubRoot &R, Acc sum, uint32_t *ctr, RegSlots<IT> &slot,
+                                           Split &&split_out) {
     constexpr int B = kAhead;
     const uint32_t tid = threadIdx.x;
-    SubTree<Acc, TPB> T(sub_slots(P.levels));
-    uint32_t slots[IT / 2], w16[KW == kWeight16 ? IT / 2 : 1];
+    SubTree<Acc, TPB> T(sub_slots(R.levels));
+    uint32_t w16[KW == kWeight16 ? IT / 2 : 1];
     Acc wacc[KW == kWeightAcc ? IT : 1];
-    auto slot = [&](int k) { return k & 1 ? slots[k / 2] >> 16 : slots[k / 2] & 0xffffu; };
 #pragma unroll
-    for (int k = 0; k < IT / 2; k++) slots[k] = 0;
+    for (int k = 0; k < IT / 2; k++) slot.two[k] = 0;
     if constexpr (KW != kWeightLoad) {
 #pragma unroll
         for (int k = 0; k < IT; k++) {
             const uint32_t i = (uint32_t)(k * TPB) + tid;
-            const WIN v = win[i < P.count ? i : P.count - 1];
+            const WIN v = win[i < count ? i : count - 1];
             if constexpr (KW == kWeightAcc) wacc[k] = AccOps<Acc>::of(v);
             else w16[k / 2] = k & 1 ? w16[k / 2] | (uint32_t)v << 16 : (uint32_t)v;
         }
     }
-    const bool ok = sub_levels<D, TPB, Acc>(
-        T, R, P.count, sum, sh.ctr,
+    return sub_levels<D, TPB, Acc>(
+        T, R, count, sum, ctr,
         [&](int nb, int a) {
             const AxisSelect<D> on(a);
             uint32_t first = tid;   // opaque: what follows from it is not kept across passes
             asm volatile("" : "+v"(first));
 #pragma unroll
             for (int k0 = 0; k0 < IT; k0 += B) {
-                if ((uint32_t)(k0 * TPB) >= P.count) continue;   // uniform: no point left
+                if ((uint32_t)(k0 * TPB) >= count) continue;   // uniform: no point left
                 uint32_t s[B];
                 float xa[B];
                 Acc w[B];
@@ -113,11 +120,11 @@ __device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x
                 for (int j = 0; j < B; j++) {
                     const int k = k0 + j;
                     const uint32_t i = (uint32_t)(k * TPB) + first;
-                    valid[j] = i < P.count;
+                    valid[j] = i < count;
                     s[j] = slot(k);   // opaque like the weights: nothing made of them is kept
                     asm volatile("" : "+v"(s[j]));
                     xa[j] = on(x[k]);
-                    if constexpr (KW == kWeightLoad) w[j] = AccOps<Acc>::of(win[valid[j] ? i : P.count - 1]);
+                    if constexpr (KW == kWeightLoad) w[j] = AccOps<Acc>::of(win[valid[j] ? i : count - 1]);
                     else if constexpr (KW == kWeight16) {
                         uint32_t v = w16[k / 2];
                         asm volatile("" : "+v"(v));
@@ -134,7 +141,7 @@ __device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x
             const AxisSelect<D> on(a);
 #pragma unroll
             for (int k0 = 0; k0 < IT; k0 += B) {
-                if ((uint32_t)(k0 * TPB) >= P.count) continue;
+                if ((uint32_t)(k0 * TPB) >= count) continue;
                 float t[B];
 #pragma unroll
                 for (int j = 0; j < B; j++) t[j] = T.at(slot(k0 + j)).win.x;
@@ -143,11 +150,22 @@ __device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x
                     const int k = k0 + j;
                     const uint32_t s0 = 2 * slot(k) + (on(x[k]) >= t[j] ? 1u : 0u);
                     const uint32_t s1 = 2 * slot(k + 1) + (on(x[k + 1]) >= t[j + 1] ? 1u : 0u);
-                    slots[k / 2] = s0 | s1 << 16;
+                    slot.two[k / 2] = s0 | s1 << 16;
                 }
             }
         },
-        [](uint32_t, uint32_t, uint32_t, uint32_t, float) {});
+        split_out);
+}
+
+// One small problem: its levels, then its ids.
+template <int D, int TPB, int IT, int KW, typename WIN, typename Acc>
+__device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x)[IT][D], const WIN *__restrict__ win,
+                                          const SubRoot &R, Acc sum, SmallShared &sh,
+                                          uint64_t *__restrict__ out, uint32_t kind, uint32_t *report) {
+    const uint32_t tid = threadIdx.x;
+    RegSlots<IT> slot;
+    const bool ok = reg_levels<D, TPB, IT, KW, WIN, Acc>(P.count, x, win, R, sum, sh.ctr, slot,
+                                                        [](uint32_t, uint32_t, uint32_t, uint32_t, float) {});
     // ids: the leaf's path less the smallest one present (:589-601, :698-702)
     uint32_t m = 0xffffffffu;
 #pragma unroll
@@ -263,19 +281,19 @@ k_small(SmallProblem one, const SmallProblem *__restrict__ table, const double *
             if constexpr (std::is_same<WIN, double>::value) {
                 const double av = fabs(v[j]);
                 const bool whole = (v[j] == trunc(v[j])) & (av <= 9007199254740992.0);
-                su += here & whole ? (uint64_t)(int64_t)v[j] : 0ull;
+                su += (here & whole) ? (uint64_t)(int64_t)v[j] : 0ull;
                 sf += here ? v[j] : 0.0;
                 sa += here ? av : 0.0;
                 fl |= whole ? 0u : (uint32_t)(kSmallReal | kSmallWide | kSmallNot16);
-                fl |= (v[j] >= -2147483648.0) & (v[j] <= 2147483647.0) ? 0u : (uint32_t)kSmallWide;
-                fl |= (v[j] >= 0.0) & (v[j] <= 65535.0) ? 0u : (uint32_t)kSmallNot16;
+                fl |= ((v[j] >= -2147483648.0) & (v[j] <= 2147483647.0)) ? 0u : (uint32_t)kSmallWide;
+                fl |= ((v[j] >= 0.0) & (v[j] <= 65535.0)) ? 0u : (uint32_t)kSmallNot16;
                 fl |= v[j] >= 0.0 ? 0u : (uint32_t)kSmallNegative;   // or NaN
             } else {
                 const int64_t u = (int64_t)v[j];
                 su += here ? (uint64_t)u : 0ull;
                 sa += here ? fabs((double)u) : 0.0;
-                fl |= (u < INT32_MIN) | (u > INT32_MAX) ? (uint32_t)kSmallWide : 0u;
-                fl |= (u < 0) | (u > 65535) ? (uint32_t)kSmallNot16 : 0u;
+                fl |= ((u < INT32_MIN) | (u > INT32_MAX)) ? (uint32_t)kSmallWide : 0u;
+                fl |= ((u < 0) | (u > 65535)) ? (uint32_t)kSmallNot16 : 0u;
                 fl |= u < 0 ? (uint32_t)kSmallNegative : 0u;
             }
         }
