@@ -182,10 +182,11 @@ struct Context {
         hints.back().shape = shape;
         return hints.back();
     }
-    DevBuf mid_code, mid_cnt, mid_w, mid_map, mid_inst, mid_open, mid_cursor, mid_lists, mid_slots;   // midpoint tree
+    DevBuf mid_code, mid_cnt, mid_w, mid_map, mid_inst, mid_open, mid_cursor, mid_lists, mid_slots, mid_points;   // midpoint tree
     bool mid_clean = false;          // its cells are all zero
     DevBuf small_table, small_report;   // the small problems of a batch and what they report
     DevBuf loads;                    // per-part loads (imbalance)
+    bool loads_clean = false;        // the sums are all zero
     DevBuf tile_bins;                // per-tile bin counts of the histogram passes
     DevBuf gparts[2], gaxis, gchunk, gcount, gctr;   // Grid::rcb: subgrids, axis sums, chunk offsets
     DevBuf gsat, gcol, grow, gheap, gscan;   // Grid::rcb summed-area path: table, carries, heap of splits, chunk sums
