@@ -95,6 +95,19 @@ __device__ __forceinline__ uint32_t wave_total_min(uint32_t v) {
     v = min(v, dpp_row<0x118, false>(kId, v));   // row_shr:8
     return min(min(rows_last_lane(v, 0), rows_last_lane(v, 1)), min(rows_last_lane(v, 2), rows_last_lane(v, 3)));
 }
+template <int Ctrl>
+__device__ __forceinline__ uint64_t dpp_row64_keep(uint64_t v) {   // lanes shifted past the row's start keep all ones
+    return (uint64_t)dpp_row<Ctrl, false>(0xffffffffu, (uint32_t)v) |
+           (uint64_t)dpp_row<Ctrl, false>(0xffffffffu, (uint32_t)(v >> 32)) << 32;
+}
+__device__ __forceinline__ uint64_t wave_total_min64(uint64_t v) {
+    auto low = [](uint64_t a, uint64_t b) { return a < b ? a : b; };
+    v = low(v, dpp_row64_keep<0x111>(v));
+    v = low(v, dpp_row64_keep<0x112>(v));
+    v = low(v, dpp_row64_keep<0x114>(v));
+    v = low(v, dpp_row64_keep<0x118>(v));
+    return low(low(rows_last_lane64(v, 0), rows_last_lane64(v, 1)), low(rows_last_lane64(v, 2), rows_last_lane64(v, 3)));
+}
 __device__ __forceinline__ uint32_t wave_total(uint32_t v) {
     v += dpp_row<0x111, true>(0u, v);
     v += dpp_row<0x112, true>(0u, v);

@@ -306,6 +306,7 @@ static unsigned persistent_grid(Context &cx, K kernel, uint64_t work_items) {
 struct BatchPlan {
     std::vector<Instance> inst;   // begin, count, levels, tile_begin, tol, heap_base
     uint64_t n = 0;               // points of all instances
+    uint64_t span = 0;            // positions of the working arrays (instances start at whole lines)
     uint32_t max_levels = 0;
     uint64_t tiles0 = 0;          // level-0 tiles
     std::vector<uint64_t> parts_ub;   // parts at each level, upper bound
@@ -324,7 +325,12 @@ static BatchPlan plan_batch(const uint64_t *counts, const size_t *levels, const 
                             size_t dim, const uint64_t *src = nullptr, const uint64_t *src_pt = nullptr) {
     BatchPlan b;
     b.inst.resize(n_inst);
-    uint64_t begin = 0, tile = 0;
+    // In a batch every instance starts at a multiple of kAlignPoints positions:
+    // the prologue writes the working arrays once, past the caches, and a line
+    // written in two parts costs two (4096 instances, both dimensions: the
+    // prologues 6.23 -> 4.69 ms, the sweeps 2.04 -> 1.74).
+    constexpr uint64_t kAlignPoints = 128;   // whole lines of the 16-bit weights
+    uint64_t begin = 0, tile = 0, packed = 0;   // packed: the instance's place in the caller's arrays
     uint64_t h = 0xcbf29ce484222325ull ^ (uint64_t)dim;   // FNV-1a over the table
     auto mix = [&](uint64_t v) {
         for (int k = 0; k < 8; k++) {
@@ -340,17 +346,19 @@ static BatchPlan plan_batch(const uint64_t *counts, const size_t *levels, const 
         I.levels = (uint32_t)std::min<size_t>(levels[q], 0xffffffffu);
         I.tile_begin = (uint32_t)tile;
         I.tol = tols[q];
-        I.src = src ? src[q] : begin;
-        I.src_pt = src_pt ? src_pt[q] : begin * dim;
+        I.src = src ? src[q] : packed;
+        I.src_pt = src_pt ? src_pt[q] : packed * dim;
         mix(I.count);
         mix(I.levels);
         mix(__builtin_bit_cast(uint64_t, I.tol));
-        begin += counts[q];
+        packed += counts[q];
+        b.span = begin + counts[q];
+        begin = (b.span + kAlignPoints - 1) / kAlignPoints * kAlignPoints;
         tile += (counts[q] + kTile - 1) / kTile;
         if (counts[q] > 0) b.max_levels = std::max<uint32_t>(b.max_levels, I.levels);
         if (I.levels > (uint32_t)kDenseLevels) b.dense = false;
     }
-    b.n = begin;
+    b.n = packed;
     b.tiles0 = tile;
     // parts at level l: one root per instance at level 0, then at most
     // min(2^l, n_i) for the instances still splitting
@@ -799,7 +807,7 @@ static bool run_levels(Context &cx, hipStream_t st, const BatchPlan &B, int wrap
                     timed(cx, st, COUPE_HIP_K_PARTITION, moved * (double)n, [&] {
                         kernel<<<g, kBlock, 0, st>>>(pa, pb, (const Part *)cx.parts[ic].ptr, tl, ntl, q4[0], q4[1],
                                                      q4[2], q4[3], cl[0], cl[1], cl[2], wl, co[0], co[1], co[2],
-                                                     ws[wsn], n, bcnt, bw, bmin, fwd_out ? fwd_at(par ^ 1) : none,
+                                                     ws[wsn], B.span, bcnt, bw, bmin, fwd_out ? fwd_at(par ^ 1) : none,
                                                      skip_axis);
                     });
                 };
@@ -876,7 +884,7 @@ static bool run_levels(Context &cx, hipStream_t st, const BatchPlan &B, int wrap
                 timed(cx, st, COUPE_HIP_K_PARTITION, 2.0 * payload * (double)n, [&] {
                     k_partition_tiles<D, WS, Acc><<<g, kBlock, 0, st>>>(
                         parts, (const Part *)cx.parts[nxt].ptr, tiles, ntl, (const uint64_t *)cx.tile_left.ptr, ci[0],
-                        ci[1], ci[2], ws[wslot(level)], co[0], co[1], co[2], ws[wslot(level + 1)], n, bcnt, bw, bmin,
+                        ci[1], ci[2], ws[wslot(level)], co[0], co[1], co[2], ws[wslot(level + 1)], B.span, bcnt, bw, bmin,
                         (uint32_t *)cx.below.ptr);
                 });
             }
@@ -1025,7 +1033,7 @@ static void prologue(Context &cx, hipStream_t st, const BatchPlan &B, const doub
         int32_t *w32 = hint < 0 || hint == 1 ? (int32_t *)cx.w[0].ptr : nullptr;
         uint16_t *w16 = nullptr;
         if (cx.weights16 && hint <= 0) {
-            cx.w16.ensure(std::max<uint64_t>(B.n, 1) * sizeof(uint16_t));
+            cx.w16.ensure(std::max<uint64_t>(B.span, 1) * sizeof(uint16_t));
             w16 = (uint16_t *)cx.w16.ptr;
         }
         const double bytes =
@@ -1104,7 +1112,7 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
     const uint32_t copies = cells <= kMidCopied ? (uint32_t)kCopies : 1u;
     const uint32_t max_cells = 1u << B.max_levels;
     const bool fresh = cx.mid_cnt.bytes < copies * cells * 4 || cx.mid_w.bytes < copies * cells * 8;
-    cx.mid_code.ensure(n * 2);
+    cx.mid_code.ensure(B.span * 2);
     cx.mid_cnt.ensure(copies * cells * 4);
     cx.mid_w.ensure(copies * cells * 8);
     cx.mid_map.ensure(cells * 4);
@@ -1114,7 +1122,7 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
     cx.mid_lists.ensure(kMidClasses * cells * 4);
     cx.mid_slots.ensure(n * 2);
     cx.heap_split.ensure(std::max<uint64_t>(B.heap_total, 1) * sizeof(float));
-    cx.w[1].ensure(n * sizeof(WL));
+    cx.mid_points.ensure(n * sizeof(MidPoint<D, WL>));
     uint32_t *gcnt = (uint32_t *)cx.mid_cnt.ptr;
     Acc *gw = (Acc *)cx.mid_w.ptr;
     if (fresh || !cx.mid_clean) {   // k_mid_tree leaves them clear
@@ -1131,13 +1139,9 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
     uint32_t *lists = (uint32_t *)cx.mid_lists.ptr;
     uint16_t *code = (uint16_t *)cx.mid_code.ptr;
     float *heap = (float *)cx.heap_split.ptr;
-    const float *c[3], *g[3];
-    float *gc[3];
-    for (int k = 0; k < 3; k++) {
-        c[k] = k < D ? cx.coords0(k) : nullptr;
-        g[k] = gc[k] = k < D ? (float *)cx.cx[1][k].ptr : nullptr;
-    }
-    WL *gwt = (WL *)cx.w[1].ptr;
+    const float *c[3];
+    for (int k = 0; k < 3; k++) c[k] = k < D ? cx.coords0(k) : nullptr;
+    using Point = MidPoint<D, WL>;
     // workgroups of a kernel with `lds` bytes each: as many as fit the CUs
     auto grid_of = [&](auto kernel, uint64_t items, uint32_t lds) {
         const unsigned by_lds = (unsigned)cx.cu_count * std::max(1u, kSubLds / (lds + 4096));
@@ -1172,24 +1176,15 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
         timed(cx, st, COUPE_HIP_K_PARTITION, 0.0, [&] {
             const unsigned grid = persistent_grid(cx, k_mid_gather<D, WL>, nt);
             k_mid_gather<D, WL><<<grid, kBlock, 0, st>>>(tiles, nt, insts, minst, c[0], c[1], c[2], w, w_src, code,
-                                                        map, cursor, gc[0], gc[1], gc[2], gwt, mid);
+                                                        map, cursor, (Point *)cx.mid_points.ptr, mid);
         });
         timed(cx, st, COUPE_HIP_K_HIST, 0.0, [&] {
-            auto launch = [&](auto kernel, int tpb, int k, unsigned per_cu) {
-                const uint32_t lds = sub_lds(B.max_levels, tpb);
-                allow_lds(kernel, lds);
-                const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)cx.cu_count * per_cu, cells);
-                kernel<<<grid, tpb, lds, st>>>(open, lists + k * cells, &mid->of_class[k], insts, g[0], g[1], g[2],
-                                               (const WL *)gwt, wrap32, heap, mid);
-            };
-            launch(k_mid_subtrees<D, 256, 8, WL, Acc>, 256, 0, 2);
-            launch(k_mid_subtrees<D, 512, 16, WL, Acc>, 512, 1, 1);
-            const uint32_t lds = sub_lds(B.max_levels, kMidStreamThreads);
-            allow_lds(k_mid_streams<D, WL, Acc>, lds);
+            const uint32_t lds = sub_lds(B.max_levels, kMidThreads);
+            allow_lds(k_mid_search<D, WL, Acc>, lds);
             const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)cx.cu_count, cells);
-            k_mid_streams<D, WL, Acc><<<grid, kMidStreamThreads, lds, st>>>(
-                open, lists + 2 * cells, &mid->of_class[2], insts, g[0], g[1], g[2], gwt, (uint16_t *)cx.mid_slots.ptr,
-                wrap32, heap, mid);
+            k_mid_search<D, WL, Acc><<<grid, kMidThreads, lds, st>>>(open, lists, cells, insts,
+                                                                    (const Point *)cx.mid_points.ptr,
+                                                                    (uint16_t *)cx.mid_slots.ptr, wrap32, heap, mid);
         });
     };
     auto ids = [&] {
@@ -1201,7 +1196,8 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
             });
         };
         // non-temporal ids for calls the caches cannot hold (see run_levels' descent)
-        if ((4.0 * D + 8.0) * (double)n > cx.move_nt_bytes) launch(k_mid_ids<D, true>);
+        // (the instances of a batch start anywhere in the caller's ids)
+        if (n_inst == 1 && (4.0 * D + 8.0) * (double)n > cx.move_nt_bytes) launch(k_mid_ids<D, true>);
         else launch(k_mid_ids<D, false>);
     };
     auto wait = [&] {
@@ -1242,7 +1238,7 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
 template <int D, typename WIN>
 static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchPlan &B, const double *pts,
                       const WIN *win, int wkind, int spec_passes) {
-    const uint64_t n = B.n;
+    const uint64_t n = B.span;   // positions of the working arrays
     // Coordinate slots: 0 (prologue output, input order), 1 and 2 (levels).
     for (int b = cx.slot0[0] ? 1 : 0; b < 3; b++)
         for (int k = 0; k < D; k++) cx.cx[b][k].ensure(std::max<uint64_t>(n, 1) * sizeof(float));
@@ -1513,45 +1509,33 @@ static bool is_small(const Context &cx, uint64_t count, size_t levels) {
     return cx.small && count > 0 && count <= kSmallPoints && levels <= kSmallLevels;
 }
 
-// Points per workgroup of the three shapes: 256 threads of 8 points (several
-// workgroups per CU), 512 threads of 16, and 512 of 32.
-constexpr uint32_t kSmallShape[3] = {256 * 8, 512 * 16, 512 * 32};
-static_assert(kSmallShape[2] == kSmallPoints, "the last shape takes every small problem");
+constexpr uint32_t kSmallNarrow = 256 * 8;   // points of a workgroup of 256 threads
 
 template <int D, typename WIN>
 static void launch_small(Context &cx, hipStream_t st, const std::vector<SmallProblem> &problems,
                          const SmallProblem *table, const double *pts, const WIN *w, int wrap32, uint64_t *out,
                          uint32_t *report) {
-    // problems come sorted by shape; a shape's run is one launch
-    size_t at = 0;
-    for (int shape = 0; shape < 3; shape++) {
-        size_t end = at;
-        uint32_t levels = 1;
-        double points = 0.0;
-        while (end < problems.size() && problems[end].count <= kSmallShape[shape]) {
-            levels = std::max(levels, problems[end].levels);
-            points += problems[end].count;
-            end++;
-        }
-        if (end == at) continue;
-        Rotation rot;
-        memset(&rot, 0, sizeof rot);
-        if (cx.rot) rot = *cx.rot;
-        const float *c0 = cx.slot0[0], *c1 = cx.slot0[1], *c2 = cx.slot0[2];
-        auto launch = [&](auto kernel, int tpb) {
-            const uint32_t lds = sub_lds(levels, tpb);
-            allow_lds(kernel, lds);
-            // algorithmic bytes: points and weights read, ids written
-            timed(cx, st, COUPE_HIP_K_OTHER, points * (8.0 * D + sizeof(WIN) + 8.0), [&] {
-                kernel<<<(unsigned)(end - at), tpb, lds, st>>>(problems[at], table ? table + at : nullptr, pts, c0, c1,
-                                                              c2, w, wrap32, cx.rot ? 1 : 0, rot, out, report + at);
-            });
-        };
-        if (shape == 0) launch(k_small<D, 256, 8, WIN>, 256);
-        else if (shape == 1) launch(k_small<D, 512, 16, WIN>, 512);
-        else launch(k_small<D, 512, 32, WIN>, 512);
-        at = end;
+    // one launch for all sizes (a launch per size would run one after the
+    // other, each as long as its longest problem); narrow workgroups when no
+    // problem needs more (1021 points: 35 us, 41 in the wide ones)
+    uint32_t levels = 1;
+    double points = 0.0;
+    for (const SmallProblem &p : problems) {
+        levels = std::max(levels, p.levels);
+        points += p.count;
     }
+    SmallArrays<WIN> A{pts, cx.slot0[0], cx.slot0[1], cx.slot0[2], w, out, wrap32, cx.rot ? 1 : 0, {}};
+    if (cx.rot) A.rot = *cx.rot;
+    auto launch = [&](auto kernel, int tpb) {
+        const uint32_t lds = sub_lds(levels, tpb);
+        allow_lds(kernel, lds);
+        // algorithmic bytes: points and weights read, ids written
+        timed(cx, st, COUPE_HIP_K_OTHER, points * (8.0 * D + sizeof(WIN) + 8.0), [&] {
+            kernel<<<(unsigned)problems.size(), tpb, lds, st>>>(problems[0], table, A, report);
+        });
+    };
+    if (problems[0].count <= kSmallNarrow) launch(k_small<D, 256, WIN>, 256);
+    else launch(k_small<D, 512, WIN>, 512);
 }
 
 // Runs the small problems of a call and waits for them.  One problem is
@@ -1560,7 +1544,7 @@ static void launch_small(Context &cx, hipStream_t st, const std::vector<SmallPro
 static void run_small(Context &cx, hipStream_t st, std::vector<SmallProblem> &problems, size_t dim,
                       const double *pts, int wkind, const void *w, uint64_t *out) {
     std::stable_sort(problems.begin(), problems.end(),
-                     [](const SmallProblem &a, const SmallProblem &b) { return a.count < b.count; });
+                     [](const SmallProblem &a, const SmallProblem &b) { return a.count > b.count; });
     const bool one = problems.size() == 1;
     const bool pinned = one && !cx.borrowed_host;
     const SmallProblem *table = nullptr;
@@ -1942,7 +1926,7 @@ void Context::for_each_buf(F &&f) {
                      &tile_bins2, &tile4, &bcnt, &bw, &bmin, &xcnt, &xw, &xmin, &nchild, &ntiles, &bsum, &nodes, &leaf,
                      &heap_split, &instances, &tiles0, &below, &tile_left, &loads, &rib_moments, &tile_bins,
                      &gparts[0], &gparts[1], &gaxis, &gchunk, &gcount, &gctr, &gsat, &gcol, &grow, &gheap, &gscan,
-                     &mid_code, &mid_cnt, &mid_w, &mid_map, &mid_inst, &mid_open, &mid_cursor, &mid_lists, &mid_slots,
+                     &mid_code, &mid_cnt, &mid_w, &mid_map, &mid_inst, &mid_open, &mid_cursor, &mid_lists, &mid_slots, &mid_points,
                      &small_table, &small_report, &ired, &counters, &in_points, &in_weights, &out_ids};
     for (DevBuf *d : all) f(*d);
 }

@@ -35,49 +35,47 @@ namespace coupe_hip {
 // ---------------------------------------------------------------------------
 constexpr int kProPoints = kBlock * 4;   // points per prologue round (4 per thread)
 
-// Per-instance bounding box and weight sums, reduced over the workgroup and
-// added to the instance with one atomic per field.
+// Per-instance bounding box (as ordered keys) and weight sums, reduced over
+// the workgroup and added to the instance with one atomic per field.  The
+// wavefronts reduce by row shifts, not by shuffles through LDS (2^20 points
+// 2D: prologue 19.7 -> 15.5 us).
+struct FlushShared {
+    uint64_t mn[kBlock / 64][kMaxDim], mx[kBlock / 64][kMaxDim], su[kBlock / 64];
+    double sf[kBlock / 64];
+};
 template <int D>
 __device__ __forceinline__ void flush_instance(InstReduce *I, double (&mn)[D], double (&mx)[D], uint64_t &su,
-                                               double &sf, double *s_d, uint64_t *s_u) {
-    const int lane = lane_id(), wid = threadIdx.x >> 6;
+                                               double &sf, FlushShared &sh) {
+    const int wid = threadIdx.x >> 6;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            const double a = __shfl_xor(mn[k], o, 64);
-            const double b = __shfl_xor(mx[k], o, 64);
-            mn[k] = a < mn[k] ? a : mn[k];
-            mx[k] = mx[k] < b ? b : mx[k];
-        }
-        su += __shfl_xor(su, o, 64);
-        sf += __shfl_xor(sf, o, 64);
+    for (int k = 0; k < D; k++) {
+        const uint64_t l = wave_total_min64(f64_key(mn[k])), h = ~wave_total_min64(~f64_key(mx[k]));
+        if (lane_id() == 0) { sh.mn[wid][k] = l; sh.mx[wid][k] = h; }
     }
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < D; k++) { s_d[wid * 8 + k] = mn[k]; s_d[wid * 8 + 3 + k] = mx[k]; }
-        s_d[wid * 8 + 6] = sf;
-        s_u[wid] = su;
-    }
+    const uint64_t u = wave_total(su);
+    const double f = wave_total(sf);
+    if (lane_id() == 0) { sh.su[wid] = u; sh.sf[wid] = f; }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    const int t = (int)threadIdx.x;   // one field per lane
+    if (t < D) {
+        uint64_t l = sh.mn[0][t], h = sh.mx[0][t];
+#pragma unroll
         for (int v = 1; v < kBlock / 64; v++) {
-#pragma unroll
-            for (int k = 0; k < D; k++) {
-                const double a = s_d[v * 8 + k], b = s_d[v * 8 + 3 + k];
-                s_d[k] = a < s_d[k] ? a : s_d[k];
-                s_d[3 + k] = s_d[3 + k] < b ? b : s_d[3 + k];
-            }
-            s_d[6] += s_d[v * 8 + 6];
-            s_u[0] += s_u[v];
+            l = sh.mn[v][t] < l ? sh.mn[v][t] : l;
+            h = sh.mx[v][t] > h ? sh.mx[v][t] : h;
         }
+        atomicMin((unsigned long long *)&I->bmin[t], (unsigned long long)l);
+        atomicMax((unsigned long long *)&I->bmax[t], (unsigned long long)h);
+    } else if (t == D) {
+        uint64_t s = 0;
 #pragma unroll
-        for (int k = 0; k < D; k++) {
-            atomicMin((unsigned long long *)&I->bmin[k], (unsigned long long)f64_key(s_d[k]));
-            atomicMax((unsigned long long *)&I->bmax[k], (unsigned long long)f64_key(s_d[3 + k]));
-        }
-        atomicAdd((unsigned long long *)&I->sum_u64, (unsigned long long)s_u[0]);
-        atomicAdd(&I->sum_f64, s_d[6]);
+        for (int v = 0; v < kBlock / 64; v++) s += sh.su[v];
+        atomicAdd((unsigned long long *)&I->sum_u64, (unsigned long long)s);
+    } else if (t == D + 1) {
+        double s = 0.0;
+#pragma unroll
+        for (int v = 0; v < kBlock / 64; v++) s += sh.sf[v];
+        atomicAdd(&I->sum_f64, s);
     }
     __syncthreads();
 #pragma unroll
@@ -135,17 +133,13 @@ struct WeightScan {
 
     // the flags and |w| statistics of the whole call: the workgroup's, into
     // its XCD's copy of the flags (blockIdx mod kCopies; the host combines
-    // the copies).  Every thread; s_d holds kBlock / 64 * 8 doubles.
+    // the copies).  Every thread; s_d holds kBlock / 64 * 4 doubles.
     __device__ __forceinline__ void flush_flags(Prologue *out, double *s_d) {
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            sa += __shfl_xor(sa, o, 64);
-            const double m2 = __shfl_xor(ma, o, 64);
-            ma = m2 > ma ? m2 : ma;
-            nonint |= __shfl_xor(nonint, o, 64);
-            not32 |= __shfl_xor(not32, o, 64);
-            not16 |= __shfl_xor(not16, o, 64);
-        }
+        sa = wave_total(sa);
+        ma = key_f64(~wave_total_min64(~f64_key(ma)));   // (a maximum of non-negative numbers)
+        nonint = __ballot(nonint != 0) ? 1u : 0u;
+        not32 = __ballot(not32 != 0) ? 1u : 0u;
+        not16 = __ballot(not16 != 0) ? 1u : 0u;
         __syncthreads();   // s_d free
         const int wid = threadIdx.x >> 6;
         if (lane_id() == 0) {
@@ -186,8 +180,8 @@ k_prologue(const Tile *__restrict__ tiles, uint32_t n_tiles, const double *__res
     // w32, w16 (each optional): the weights as int32 and as 16-bit unsigned
     // integers; the latter are used when every weight is an integer in
     // [0, 65535] (not_u16 stays 0)
-    __shared__ double s_d[kBlock / 64 * 8];
-    __shared__ uint64_t s_u[kBlock / 64];
+    __shared__ double s_d[kBlock / 64 * 4];
+    __shared__ FlushShared s_f;
     const int tid = threadIdx.x;
     double mn[D], mx[D];
 #pragma unroll
@@ -201,7 +195,7 @@ k_prologue(const Tile *__restrict__ tiles, uint32_t n_tiles, const double *__res
     for (uint32_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
         const Tile T = tiles[t];
         if (T.part != cur) {
-            if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_d, s_u);
+            if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_f);
             cur = T.part;
             ipts = pts + insts[cur].src_pt;
             iwin = win + insts[cur].src;
@@ -257,7 +251,7 @@ k_prologue(const Tile *__restrict__ tiles, uint32_t n_tiles, const double *__res
             }
         }
     }
-    if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_d, s_u);
+    if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_f);
     ws.flush_flags(out, s_d);
 }
 
@@ -273,8 +267,8 @@ k_prologue_soa(const Tile *__restrict__ tiles, uint32_t n_tiles, const float *__
                const float *__restrict__ c1, const float *__restrict__ c2, const WIN *__restrict__ win,
                int32_t *__restrict__ w32, uint16_t *__restrict__ w16, Instance *__restrict__ insts, Prologue *out,
                InstReduce *red, uint32_t n_inst) {
-    __shared__ double s_d[kBlock / 64 * 8];
-    __shared__ uint64_t s_u[kBlock / 64];
+    __shared__ double s_d[kBlock / 64 * 4];
+    __shared__ FlushShared s_f;
     double mn[D], mx[D];
 #pragma unroll
     for (int k = 0; k < D; k++) { mn[k] = 1.7976931348623157e308; mx[k] = -1.7976931348623157e308; }
@@ -283,7 +277,7 @@ k_prologue_soa(const Tile *__restrict__ tiles, uint32_t n_tiles, const float *__
     for (uint32_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
         const Tile T = tiles[t];
         if (T.part != cur) {
-            if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_d, s_u);
+            if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_f);
             cur = T.part;
         }
         for (uint32_t p = threadIdx.x; p < T.count; p += kBlock) {
@@ -298,7 +292,7 @@ k_prologue_soa(const Tile *__restrict__ tiles, uint32_t n_tiles, const float *__
             ws.add(win[i], i, w32, w16);
         }
     }
-    if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_d, s_u);
+    if (cur != 0xffffffffu) flush_instance<D>(&red[(blockIdx.x % kCopies) * n_inst + cur], mn, mx, ws.su, ws.sf, s_f);
     ws.flush_flags(out, s_d);
 }
 

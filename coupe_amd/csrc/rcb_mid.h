@@ -27,7 +27,7 @@ namespace coupe_hip {
 constexpr uint32_t kMidLevels = 12;            // most levels: 4096 cells, two 16-bit halves of a map entry
 constexpr uint32_t kMidDone = 0xffffffffu;     // map: the cell's points are settled
 constexpr uint32_t kMidClasses = 3;            // open nodes of at most 2048 and 8192 points, and larger
-constexpr uint32_t kMidClass[2] = {256 * 8, 512 * 16};
+constexpr uint32_t kMidClass[2] = {512 * 4, 512 * 16};
 
 // An open node: its points are gathered at [begin, begin + count).
 struct MidOpen {
@@ -46,7 +46,7 @@ struct MidCounters {
     uint32_t of_class[kMidClasses];
     uint32_t big;                   // open nodes too large for a workgroup: the call takes the general path
     uint32_t error;                 // a subtree's search did not end
-    uint32_t pad;
+    uint32_t taken;                 // nodes taken from the queue
 };
 
 // An instance's figures on this path: its open nodes are
@@ -378,6 +378,15 @@ k_mid_tree(Instance *__restrict__ insts, const InstReduce *__restrict__ red, uin
     if (tid == 0) I.min_id = s_min == 0xffffffffu ? ~0ull : (uint64_t)s_min;   // (the subtrees lower it)
 }
 
+// One gathered point: a single store per point, whose address no neighbour
+// shares when the input is in random order (4096 instances 3D: gather 2.53 -> 1.62 ms
+// against one store per coordinate and weight).
+template <int D, typename WL>
+struct alignas(sizeof(WL) == 8 && D == 3 ? 8 : 16) MidPoint {
+    float x[D];
+    WL w;
+};
+
 // ---------------------------------------------------------------------------
 // The open nodes' points, gathered node by node (their order within a node is
 // free).  Workgroups take contiguous shares of the tiles: each counts its
@@ -389,8 +398,8 @@ __global__ void __launch_bounds__(kBlock)
 k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__restrict__ insts,
              const MidInstance *__restrict__ minst, const float *__restrict__ c0, const float *__restrict__ c1,
              const float *__restrict__ c2, const WL *__restrict__ w, int w_src, const uint16_t *__restrict__ code,
-             const uint32_t *__restrict__ map, uint32_t *__restrict__ cursor, float *__restrict__ o0,
-             float *__restrict__ o1, float *__restrict__ o2, WL *__restrict__ ow, const MidCounters *ctr) {
+             const uint32_t *__restrict__ map, uint32_t *__restrict__ cursor, MidPoint<D, WL> *__restrict__ gathered,
+             const MidCounters *ctr) {
     if (ctr->open == 0 || ctr->big) return;
     __shared__ uint16_t num[1 << kMidLevels];            // open node of a cell, 0xffff: settled
     __shared__ uint32_t place[1 << (kMidLevels - 1)];    // at most half as many open nodes as cells
@@ -420,22 +429,55 @@ k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *_
         for (uint32_t k = tid; k < M.n_open; k += kBlock) place[k] = 0;
         __syncthreads();
         const uint64_t begin = tiles[t].begin, end = tiles[e - 1].begin + tiles[e - 1].count;
-        for (uint64_t i = begin + tid; i < end; i += kBlock) {
-            const uint16_t o = num[code[i]];
-            if (o != 0xffffu) atomicAdd(&place[o], 1u);
+        // eight points of a thread at a time: their loads are issued together
+        constexpr int G = 8;
+        for (uint64_t i0 = begin; i0 < end; i0 += kBlock * G) {
+            uint16_t o[G];
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                const uint64_t i = i0 + (uint32_t)(k * kBlock) + tid;
+                o[k] = code[i < end ? i : end - 1];
+            }
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                const uint16_t m = num[o[k]];
+                if (m != 0xffffu && i0 + (uint32_t)(k * kBlock) + tid < end) atomicAdd(&place[m], 1u);
+            }
         }
         __syncthreads();
         for (uint32_t k = tid; k < M.n_open; k += kBlock)
             if (place[k]) place[k] = atomicAdd(&cursor[M.first_open + k], place[k]);
         __syncthreads();
-        for (uint64_t i = begin + tid; i < end; i += kBlock) {
-            const uint16_t o = num[code[i]];
-            if (o == 0xffffu) continue;
-            const uint32_t d = atomicAdd(&place[o], 1u);
-            o0[d] = c0[i];
-            o1[d] = c1[i];
-            if constexpr (D == 3) o2[d] = c2[i];
-            ow[d] = w[wbase + i];
+        for (uint64_t i0 = begin; i0 < end; i0 += kBlock * G) {
+            uint16_t o[G];
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                const uint64_t i = i0 + (uint32_t)(k * kBlock) + tid;
+                o[k] = code[i < end ? i : end - 1];
+            }
+            bool any = false;
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                o[k] = i0 + (uint32_t)(k * kBlock) + tid < end ? num[o[k]] : (uint16_t)0xffffu;
+                any |= o[k] != 0xffffu;
+            }
+            if (__ballot(any) == 0) continue;
+            MidPoint<D, WL> r[G];
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                const uint64_t i = i0 + (uint32_t)(k * kBlock) + tid;
+                if (o[k] != 0xffffu) {
+                    r[k].x[0] = c0[i];
+                    r[k].x[1] = c1[i];
+                    if constexpr (D == 3) r[k].x[2] = c2[i];
+                    r[k].w = w[wbase + i];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                if (o[k] == 0xffffu) continue;
+                gathered[atomicAdd(&place[o[k]], 1u)] = r[k];
+            }
         }
         t = e;
     }
@@ -473,101 +515,105 @@ struct MidSplits {
     }
 };
 
-// Points in registers: the nodes of one class.
+// A node whose points fit the workgroup's registers.
 template <int D, int TPB, int IT, typename WL, typename Acc>
-__global__ void __launch_bounds__(TPB)
-k_mid_subtrees(const MidOpen *__restrict__ open, const uint32_t *__restrict__ list, const uint32_t *n_list,
-               Instance *__restrict__ insts, const float *__restrict__ c0, const float *__restrict__ c1,
-               const float *__restrict__ c2, const WL *__restrict__ w, int wrap32, float *__restrict__ heap_split,
-               MidCounters *ctr) {
-    if (ctr->big) return;
-    SmallShared &sh = *(SmallShared *)sub_lds_base;
-    const uint32_t n = *n_list;
-    for (uint32_t g = blockIdx.x; g < n; g += gridDim.x) {
-        const MidOpen &O = open[list[g]];
-        Instance &I = insts[O.inst];
-        const uint32_t count = __builtin_amdgcn_readfirstlane(O.count), begin = __builtin_amdgcn_readfirstlane(O.begin);
-        const SubRoot R = mid_root<WL>(O, I, wrap32);
-        float x[IT][D];
-        small_points<D, TPB, IT>(count, x, [&](uint64_t i, float (&p)[D]) {
-            p[0] = c0[begin + i];
-            p[1] = c1[begin + i];
-            if constexpr (D == 3) p[2] = c2[begin + i];
-        });
-        __syncthreads();   // the last node's LDS is free
-        if (threadIdx.x == 0) sh.min_slot = 0xffffffffu;
-        const MidSplits out{heap_split + I.heap_base, O.node, R.levels, &sh.min_slot};
-        RegSlots<IT> slot;
-        const bool ok = reg_levels<D, TPB, IT, kWeightAcc, WL, Acc>(count, x, w + begin, R,
-                                                                    AccOps<Acc>::from_bits(O.sum), sh.ctr, slot, out);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            atomicMin((unsigned long long *)&I.min_id, (unsigned long long)sh.min_slot);
-            if (!ok) atomicOr(&ctr->error, 1u);
-        }
-    }
+__device__ __forceinline__ bool mid_registers(uint32_t count, const SubRoot &R, Acc sum,
+                                              const MidPoint<D, WL> *__restrict__ pts, uint32_t *ctr,
+                                              const MidSplits &out) {
+    float x[IT][D];
+    small_points<D, TPB, IT>(count, x, [&](uint64_t i, float (&p)[D]) {
+#pragma unroll
+        for (int a = 0; a < D; a++) p[a] = pts[i].x[a];
+    });
+    RegSlots<IT> slot;
+    return reg_levels<D, TPB, IT, kWeightAcc, WL, Acc>(count, x, [&](uint32_t i) { return pts[i].w; }, R, sum, ctr, slot,
+                                                       out);
 }
 
-// Larger nodes: the points stay in memory (a node's are read again per pass,
-// from the caches), their slots beside them.
-constexpr int kMidStreamThreads = 1024;
+// A larger node: its points stay in memory (read again per pass, from the
+// caches), their slots beside them.
+template <int D, int TPB, typename WL, typename Acc>
+__device__ __forceinline__ bool mid_memory(uint32_t count, const SubRoot &R, Acc sum,
+                                           const MidPoint<D, WL> *__restrict__ pts, uint16_t *__restrict__ slots,
+                                           uint32_t *ctr, const MidSplits &out) {
+    constexpr int B = kAhead;
+    const uint32_t tid = threadIdx.x;
+    SubTree<Acc, TPB> T(sub_slots(R.levels));
+    bool first = true;   // every point in slot 0: not read
+    return sub_levels<D, TPB, Acc>(
+        T, R, count, sum, ctr,
+        [&](int nb, int a) {
+            for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
+                uint32_t s[B];
+                float xa[B];
+                Acc wk[B];
+                bool valid[B];
+#pragma unroll
+                for (int j = 0; j < B; j++) {
+                    const uint32_t i = i0 + (uint32_t)(j * TPB) + tid, p = i < count ? i : count - 1;
+                    valid[j] = i < count;
+                    xa[j] = pts[p].x[a];
+                    wk[j] = AccOps<Acc>::of(pts[p].w);
+                    s[j] = first ? 0u : (uint32_t)slots[p];
+                }
+                sub_bin<B, TPB, Acc>(T, s, xa, wk, valid, nb, R.packed);
+            }
+        },
+        [&](int a) {
+            for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
+                uint32_t s[B];
+                float xa[B];
+#pragma unroll
+                for (int j = 0; j < B; j++) {   // (each thread its own points: no other touches their slots)
+                    const uint32_t i = i0 + (uint32_t)(j * TPB) + tid, p = i < count ? i : count - 1;
+                    xa[j] = pts[p].x[a];
+                    s[j] = first ? 0u : (uint32_t)slots[p];
+                }
+#pragma unroll
+                for (int j = 0; j < B; j++) {
+                    const uint32_t i = i0 + (uint32_t)(j * TPB) + tid;
+                    if (i < count) slots[i] = (uint16_t)(2 * s[j] + (xa[j] >= T.at(s[j]).win.x ? 1u : 0u));
+                }
+            }
+            first = false;
+        },
+        out);
+}
+
+// The workgroups take the nodes from a queue, the large ones first.
+constexpr int kMidThreads = 512;
 template <int D, typename WL, typename Acc>
-__global__ void __launch_bounds__(kMidStreamThreads)
-k_mid_streams(const MidOpen *__restrict__ open, const uint32_t *__restrict__ list, const uint32_t *n_list,
-              Instance *__restrict__ insts, const float *__restrict__ c0, const float *__restrict__ c1,
-              const float *__restrict__ c2, const WL *__restrict__ w, uint16_t *__restrict__ slots, int wrap32,
-              float *__restrict__ heap_split, MidCounters *ctr) {
+__global__ void __launch_bounds__(kMidThreads)
+k_mid_search(const MidOpen *__restrict__ open, const uint32_t *__restrict__ lists, uint64_t list_stride,
+             Instance *__restrict__ insts, const MidPoint<D, WL> *__restrict__ gathered,
+             uint16_t *__restrict__ slots, int wrap32, float *__restrict__ heap_split, MidCounters *ctr) {
     if (ctr->big) return;
-    constexpr int TPB = kMidStreamThreads, B = kAhead;
+    constexpr int TPB = kMidThreads;
     SmallShared &sh = *(SmallShared *)sub_lds_base;
-    const uint32_t n = *n_list, tid = threadIdx.x;
-    for (uint32_t g = blockIdx.x; g < n; g += gridDim.x) {
-        const MidOpen &O = open[list[g]];
+    const uint32_t n0 = ctr->of_class[0], n1 = ctr->of_class[1], n2 = ctr->of_class[2], tid = threadIdx.x;
+    for (;;) {
+        __syncthreads();   // the last node's LDS is free
+        if (tid == 0) {
+            sh.flags = atomicAdd(&ctr->taken, 1u);
+            sh.min_slot = 0xffffffffu;
+        }
+        __syncthreads();
+        uint32_t g = __builtin_amdgcn_readfirstlane(sh.flags);   // every workgroup gets past the end once, and leaves
+        if (g >= n0 + n1 + n2) return;
+        int k = 2;
+        if (g >= n2) { g -= n2; k = 1; }
+        if (k == 1 && g >= n1) { g -= n1; k = 0; }
+        const MidOpen &O = open[lists[(uint64_t)k * list_stride + g]];
         Instance &I = insts[O.inst];
         const uint32_t count = __builtin_amdgcn_readfirstlane(O.count), begin = __builtin_amdgcn_readfirstlane(O.begin);
         const SubRoot R = mid_root<WL>(O, I, wrap32);
-        __syncthreads();   // the last node's LDS is free
-        if (tid == 0) sh.min_slot = 0xffffffffu;
         const MidSplits out{heap_split + I.heap_base, O.node, R.levels, &sh.min_slot};
-        SubTree<Acc, TPB> T(sub_slots(R.levels));
-        uint16_t *sl = slots + begin;
-        const WL *wp = w + begin;
-        bool first = true;   // every point in slot 0: not read
-        const bool ok = sub_levels<D, TPB, Acc>(
-            T, R, count, AccOps<Acc>::from_bits(O.sum), sh.ctr,
-            [&](int nb, int a) {
-                const float *c = (a == 0 ? c0 : (a == 1 ? c1 : c2)) + begin;
-                for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
-                    uint32_t s[B];
-                    float xa[B];
-                    Acc wk[B];
-                    bool valid[B];
-#pragma unroll
-                    for (int j = 0; j < B; j++) {
-                        const uint32_t i = i0 + (uint32_t)(j * TPB) + tid, p = i < count ? i : count - 1;
-                        valid[j] = i < count;
-                        xa[j] = c[p];
-                        wk[j] = AccOps<Acc>::of(wp[p]);
-                        s[j] = first ? 0u : (uint32_t)sl[p];
-                    }
-                    sub_bin<B, TPB, Acc>(T, s, xa, wk, valid, nb, R.packed);
-                }
-            },
-            [&](int a) {
-                const float *c = (a == 0 ? c0 : (a == 1 ? c1 : c2)) + begin;
-                for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
-#pragma unroll
-                    for (int j = 0; j < B; j++) {
-                        const uint32_t i = i0 + (uint32_t)(j * TPB) + tid;
-                        if (i < count) {   // (each thread its own points: no other reads them)
-                            const uint32_t s = first ? 0u : (uint32_t)sl[i];
-                            sl[i] = (uint16_t)(2 * s + (c[i] >= T.at(s).win.x ? 1u : 0u));
-                        }
-                    }
-                }
-                first = false;
-            },
-            out);
+        const Acc sum = AccOps<Acc>::from_bits(O.sum);
+        const MidPoint<D, WL> *pts = gathered + begin;
+        bool ok;
+        if (k == 0) ok = mid_registers<D, TPB, 4, WL, Acc>(count, R, sum, pts, sh.ctr, out);
+        else if (k == 1) ok = mid_registers<D, TPB, 16, WL, Acc>(count, R, sum, pts, sh.ctr, out);
+        else ok = mid_memory<D, TPB, WL, Acc>(count, R, sum, pts, slots + begin, sh.ctr, out);
         __syncthreads();
         if (tid == 0) {
             atomicMin((unsigned long long *)&I.min_id, (unsigned long long)sh.min_slot);
@@ -588,12 +634,12 @@ k_mid_ids(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__re
           const float *__restrict__ c2, uint64_t *__restrict__ out, const MidCounters *ctr) {
     if (ctr->big) return;
     __shared__ uint16_t node[1 << kMidLevels];   // open node of a cell, 0xffff: settled
+    __shared__ float heap[1 << kMidLevels];      // the instance's splits
     const int tid = threadIdx.x;
     uint32_t t0, t1;
     tile_range(n_tiles, t0, t1);
     uint32_t cur = 0xffffffffu, levels = 0, leaf0 = 0;
     uint64_t off = 0, src = 0;
-    const float *heap = heap_split;
     bool any_open = false;
     for (uint32_t t = t0; t < t1; t++) {
         const Tile U = tiles[t];
@@ -604,40 +650,66 @@ k_mid_ids(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__re
             leaf0 = (1u << levels) - 1;
             off = I.min_id;
             src = I.src - I.begin;
-            heap = heap_split + I.heap_base;
             any_open = minst[cur].n_open != 0;
             if (any_open) {
-                const uint64_t cbase = mid_cell_base(I, cur);
+                const uint64_t cbase = mid_cell_base(I, cur), hb = I.heap_base;
                 __syncthreads();
-                for (uint32_t c = tid; c <= leaf0; c += kBlock) node[c] = (uint16_t)map[cbase + c];   // kMidDone: 0xffff
+                for (uint32_t c = tid; c <= leaf0; c += kBlock) {
+                    node[c] = (uint16_t)map[cbase + c];   // kMidDone: 0xffff
+                    if (c < leaf0) heap[c] = heap_split[hb + c];
+                }
                 __syncthreads();
             }
         }
-        uint32_t c[kItems];
+        uint32_t h[kItems];
+        uint64_t at[kItems];
 #pragma unroll
         for (int k = 0; k < kItems; k++) {
-            const uint64_t i = U.begin + min((uint32_t)(k * kBlock + tid), U.count - 1u);
-            if constexpr (NT) c[k] = __builtin_nontemporal_load(&code[i]);
-            else c[k] = code[i];
+            at[k] = U.begin + min((uint32_t)(k * kBlock + tid), U.count - 1u);
+            if constexpr (NT) h[k] = __builtin_nontemporal_load(&code[at[k]]);
+            else h[k] = code[at[k]];
+        }
+        if (!any_open) {
+#pragma unroll
+            for (int k = 0; k < kItems; k++) h[k] += leaf0;
+        } else {
+            bool walk = false;
+#pragma unroll
+            for (int k = 0; k < kItems; k++) {
+                const uint32_t o = node[h[k]];
+                h[k] = o != 0xffffu ? o : leaf0 + h[k];
+                walk |= h[k] < leaf0;
+            }
+            if (__ballot(walk)) {
+                float x[kItems][D];
+#pragma unroll
+                for (int k = 0; k < kItems; k++) {
+                    if (h[k] < leaf0) {
+                        x[k][0] = c0[at[k]];
+                        x[k][1] = c1[at[k]];
+                        if constexpr (D == 3) x[k][2] = c2[at[k]];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < kItems; k++) {
+                    if (h[k] < leaf0) {
+                        int a = (int)((31u - (uint32_t)__builtin_clz(h[k] + 1)) % D);
+                        do {
+                            const float xa = a == 0 ? x[k][0] : (a == 1 ? x[k][1] : x[k][D - 1]);
+                            h[k] = 2 * h[k] + (xa >= heap[h[k]] ? 2u : 1u);
+                            a = a + 1 == D ? 0 : a + 1;
+                        } while (h[k] < leaf0);
+                    }
+                }
+            }
         }
 #pragma unroll
         for (int k = 0; k < kItems; k++) {
             const uint32_t p = (uint32_t)(k * kBlock + tid);
-            if (p >= U.count) continue;
-            const uint64_t i = U.begin + p;
-            uint32_t h = leaf0 + c[k];
-            if (any_open && node[c[k]] != 0xffffu) {
-                h = node[c[k]];
-                uint32_t l = 31u - (uint32_t)__builtin_clz(h + 1);
-                const float x0 = c0[i], x1 = c1[i], x2 = D == 3 ? c2[i] : 0.0f;
-                int a = (int)(l % D);
-                for (; l < levels; l++) {
-                    h = 2 * h + (sel3(a, x0, x1, x2) >= heap[h] ? 2u : 1u);
-                    a = a + 1 == D ? 0 : a + 1;
-                }
+            if (p < U.count) {
+                if constexpr (NT) __builtin_nontemporal_store((uint64_t)h[k] - off, &out[src + U.begin + p]);
+                else out[src + U.begin + p] = (uint64_t)h[k] - off;
             }
-            if constexpr (NT) __builtin_nontemporal_store((uint64_t)h - off, &out[src + i]);
-            else out[src + i] = (uint64_t)h - off;
         }
     }
 }

@@ -73,8 +73,8 @@ enum : int { kWeightAcc, kWeight16, kWeightLoad };
 constexpr int kAhead = 4;   // points of a lane whose lookups are issued together
 constexpr int kLoad = 8;    // points of a lane loaded together
 
-// The levels of a subtree of `count` points in registers, their weights in
-// win; the slots two to a register.  Points are taken kAhead at a time, up to
+// The levels of a subtree of `count` points in registers, their weights
+// win(i); the slots two to a register.  Points are taken kAhead at a time, up to
 // the uniform end.
 template <int IT>
 struct RegSlots {
@@ -83,11 +83,12 @@ struct RegSlots {
         return k & 1 ? two[k / 2] >> 16 : two[k / 2] & 0xffffu;
     }
 };
-template <int D, int TPB, int IT, int KW, typename WIN, typename Acc, typename Split>
-__device__ __forceinline__ bool reg_levels(uint32_t count, const float (&x)[IT][D], const WIN *__restrict__ win,
+template <int D, int TPB, int IT, int KW, typename WIN, typename Acc, typename Weight, typename Split>
+__device__ __forceinline__ bool reg_levels(uint32_t count, const float (&x)[IT][D], Weight &&win,
                                            const SubRoot &R, Acc sum, uint32_t *ctr, RegSlots<IT> &slot,
                                            Split &&split_out) {
     constexpr int B = kAhead;
+    static_assert(IT % B == 0, "whole groups of points");
     const uint32_t tid = threadIdx.x;
     SubTree<Acc, TPB> T(sub_slots(R.levels));
     uint32_t w16[KW == kWeight16 ? IT / 2 : 1];
@@ -98,7 +99,7 @@ __device__ __forceinline__ bool reg_levels(uint32_t count, const float (&x)[IT][
 #pragma unroll
         for (int k = 0; k < IT; k++) {
             const uint32_t i = (uint32_t)(k * TPB) + tid;
-            const WIN v = win[i < count ? i : count - 1];
+            const WIN v = win(i < count ? i : count - 1);
             if constexpr (KW == kWeightAcc) wacc[k] = AccOps<Acc>::of(v);
             else w16[k / 2] = k & 1 ? w16[k / 2] | (uint32_t)v << 16 : (uint32_t)v;
         }
@@ -124,7 +125,7 @@ __device__ __forceinline__ bool reg_levels(uint32_t count, const float (&x)[IT][
                     s[j] = slot(k);   // opaque like the weights: nothing made of them is kept
                     asm volatile("" : "+v"(s[j]));
                     xa[j] = on(x[k]);
-                    if constexpr (KW == kWeightLoad) w[j] = AccOps<Acc>::of(win[valid[j] ? i : count - 1]);
+                    if constexpr (KW == kWeightLoad) w[j] = AccOps<Acc>::of(win(valid[j] ? i : count - 1));
                     else if constexpr (KW == kWeight16) {
                         uint32_t v = w16[k / 2];
                         asm volatile("" : "+v"(v));
@@ -164,8 +165,8 @@ __device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x
                                           uint64_t *__restrict__ out, uint32_t kind, uint32_t *report) {
     const uint32_t tid = threadIdx.x;
     RegSlots<IT> slot;
-    const bool ok = reg_levels<D, TPB, IT, KW, WIN, Acc>(P.count, x, win, R, sum, sh.ctr, slot,
-                                                        [](uint32_t, uint32_t, uint32_t, uint32_t, float) {});
+    const bool ok = reg_levels<D, TPB, IT, KW, WIN, Acc>(P.count, x, [&](uint32_t i) { return win[i]; }, R, sum, sh.ctr,
+                                                        slot, [](uint32_t, uint32_t, uint32_t, uint32_t, float) {});
     // ids: the leaf's path less the smallest one present (:589-601, :698-702)
     uint32_t m = 0xffffffffu;
 #pragma unroll
@@ -189,41 +190,47 @@ __device__ __forceinline__ void small_run(const SmallProblem &P, const float (&x
 // the end: from a resident working copy, mapped by a rotation (Rib), or as given.
 template <int D, int TPB, int IT, typename Load>
 __device__ __forceinline__ void small_points(uint32_t count, float (&x)[IT][D], Load &&load) {
+    constexpr int L = IT < kLoad ? IT : kLoad;
 #pragma unroll
-    for (int k0 = 0; k0 < IT; k0 += kLoad) {
+    for (int k0 = 0; k0 < IT; k0 += L) {
         if ((uint32_t)(k0 * TPB) >= count) {   // uniform: no point left
 #pragma unroll
-            for (int j = 0; j < kLoad; j++)
+            for (int j = 0; j < L; j++)
 #pragma unroll
                 for (int a = 0; a < D; a++) x[k0 + j][a] = 0.0f;
             continue;
         }
 #pragma unroll
-        for (int j = 0; j < kLoad; j++) {
+        for (int j = 0; j < L; j++) {
             const uint32_t i = (uint32_t)((k0 + j) * TPB) + threadIdx.x;
             load((uint64_t)(i < count ? i : count - 1), x[k0 + j]);
         }
     }
 }
 
-// Workgroup q: problem `one` (grid of one) or table[q].  c0 (non-null): the
-// f32 coordinates of a resident working copy replace the points; rot_on:
-// every point mapped by rot first (Rib).
+// What a launch of small problems reads and writes.  c0 (non-null): the f32
+// coordinates of a resident working copy replace the points; rot_on: every
+// point mapped by rot first (Rib).
+template <typename WIN>
+struct SmallArrays {
+    const double *pts;
+    const float *c0, *c1, *c2;
+    const WIN *win;
+    uint64_t *out;
+    int wrap32, rot_on;
+    Rotation rot;
+};
+
 template <int D, int TPB, int IT, typename WIN>
-__global__ void __launch_bounds__(TPB)
-k_small(SmallProblem one, const SmallProblem *__restrict__ table, const double *__restrict__ pts,
-        const float *__restrict__ c0, const float *__restrict__ c1, const float *__restrict__ c2,
-        const WIN *__restrict__ win, int wrap32, int rot_on, Rotation rot, uint64_t *__restrict__ out,
-        uint32_t *report) {
+__device__ __forceinline__ void small_problem(const SmallProblem &P, const SmallArrays<WIN> &A, uint32_t *report) {
     SmallShared &sh = *(SmallShared *)sub_lds_base;
-    SmallProblem P = one;
-    if (table) P = table[blockIdx.x];
-    P.levels = __builtin_amdgcn_readfirstlane(P.levels);   // uniform: kept in scalar registers
-    P.count = __builtin_amdgcn_readfirstlane(P.count);
+    const float *__restrict__ c0 = A.c0, *__restrict__ c1 = A.c1, *__restrict__ c2 = A.c2;
+    uint64_t *__restrict__ out = A.out;
+    const Rotation &rot = A.rot;
     const uint32_t tid = threadIdx.x;
     const int lane = lane_id(), wid = (int)(tid >> 6);
-    const double *p = pts + P.src_pt;
-    const WIN *w = win + P.src;
+    const double *__restrict__ p = A.pts + P.src_pt;
+    const WIN *__restrict__ w = A.win + P.src;
 
     // every point once: coordinates as f32 (:677), box (geometry.rs:42-76;
     // the cast is monotone, so the extremes of the f32 coordinates are the
@@ -236,7 +243,7 @@ k_small(SmallProblem one, const SmallProblem *__restrict__ table, const double *
             q[1] = c1[P.src + i];
             if constexpr (D == 3) q[2] = c2[P.src + i];
         });
-    } else if (rot_on) {
+    } else if (A.rot_on) {
         small_points<D, TPB, IT>(P.count, x, [&](uint64_t i, float (&q)[D]) {
             double v[D];
 #pragma unroll
@@ -260,17 +267,18 @@ k_small(SmallProblem one, const SmallProblem *__restrict__ table, const double *
     uint64_t su = 0;
     double sf = 0.0, sa = 0.0;
     uint32_t fl = 0;
+    constexpr int L = IT < kLoad ? IT : kLoad;
 #pragma unroll
-    for (int k0 = 0; k0 < IT; k0 += kLoad) {
+    for (int k0 = 0; k0 < IT; k0 += L) {
         if ((uint32_t)(k0 * TPB) >= P.count) continue;   // uniform: no point left
-        WIN v[kLoad];
+        WIN v[L];
 #pragma unroll
-        for (int j = 0; j < kLoad; j++) {
+        for (int j = 0; j < L; j++) {
             const uint32_t i = (uint32_t)((k0 + j) * TPB) + tid;
             v[j] = w[i < P.count ? i : P.count - 1];
         }
 #pragma unroll
-        for (int j = 0; j < kLoad; j++) {
+        for (int j = 0; j < L; j++) {
             const int k = k0 + j;
             const bool here = (uint32_t)(k * TPB) + tid < P.count;
 #pragma unroll
@@ -342,13 +350,12 @@ k_small(SmallProblem one, const SmallProblem *__restrict__ table, const double *
     R.axis = 0;
     R.levels = P.levels;
     R.tol = P.tol;
-    R.wrap32 = wrap32;
+    R.wrap32 = A.wrap32;
     // exact sums: integers, and integer-valued doubles whose sums stay exact
     const bool real = (all & kSmallReal) || (std::is_same<WIN, double>::value &&
                                             !(sa <= 9007199254740992.0 * (1.0 - 1e-6)));
     R.packed = !real && !(all & kSmallNegative) && sa < (double)(1ull << (kSubPack - 1));
     const uint32_t kind = (all & 7u) | (real ? kSmallReal : 0u);
-    report += blockIdx.x;
     if constexpr (IT <= 16) {
         if constexpr (std::is_same<WIN, double>::value) {
             if (real) {
@@ -370,5 +377,26 @@ k_small(SmallProblem one, const SmallProblem *__restrict__ table, const double *
             small_run<D, TPB, IT, kWeight16, WIN, uint64_t>(P, x, w, R, su, sh, out, kind, report);
     }
 }
+
+// Problem q of a launch: `one` (a launch of one) or table[q], largest first so
+// that the long ones start first.  Workgroups of 256 threads take 8 points per
+// thread; those of 512 threads 4, 16 or 32, by the problem's size.
+template <int D, int TPB, typename WIN>
+__global__ void __launch_bounds__(TPB)
+k_small(SmallProblem one, const SmallProblem *__restrict__ table, SmallArrays<WIN> A, uint32_t *report) {
+    SmallProblem P = one;
+    if (table) P = table[blockIdx.x];
+    P.levels = __builtin_amdgcn_readfirstlane(P.levels);   // uniform: kept in scalar registers
+    P.count = __builtin_amdgcn_readfirstlane(P.count);
+    report += blockIdx.x;
+    if constexpr (TPB == 256) {
+        small_problem<D, TPB, 8, WIN>(P, A, report);
+    } else {
+        if (P.count <= TPB * 4) small_problem<D, TPB, 4, WIN>(P, A, report);
+        else if (P.count <= TPB * 16) small_problem<D, TPB, 16, WIN>(P, A, report);
+        else small_problem<D, TPB, 32, WIN>(P, A, report);
+    }
+}
+static_assert(512 * 32 == kSmallPoints, "the last shape takes every small problem");
 
 }  // namespace coupe_hip
