@@ -87,6 +87,7 @@ struct Hints {
     std::vector<uint32_t> level_open;   // parts of each level still searching after the first decision
     uint64_t graph_key = 0;             // graph key of its last call (a key is captured when it repeats)
     int mid = -1;                       // the midpoint tree took its last call (-1: not tried, 0: no)
+    uint32_t front_rounds = 0;          // rounds the frontier took in its last call
     uint32_t mid_open = 1;              // open nodes the midpoint tree left (0: none)
     int moves_coherent = -1;            // its moved tiles went to few destinations (-1: not known)
 };
@@ -149,6 +150,7 @@ struct Context {
     uint32_t search_chunk = 2;       // consecutive tiles a workgroup takes at a time in the search passes
     bool small = true;               // problems of few points take one workgroup each (rcb_small.h)
     bool mid = true;                 // try the tree of box midpoints first (rcb_mid.h)
+    bool front = true;               // search one instance's levels without moving its points (rcb_front.h)
     double move_nt_bytes = 2.5e9;    // moves and id descents of more bytes than this go non-temporal
     int max_bins = kMaxBins;         // bins per part of the later search passes (16..256, a power of two)
     int wg_cap = 0;                  // workgroups per CU of the persistent kernels (0: as many as fit)
@@ -183,6 +185,7 @@ struct Context {
         return hints.back();
     }
     DevBuf mid_code, mid_cnt, mid_w, mid_map, mid_inst, mid_open, mid_cursor, mid_lists, mid_slots, mid_points;   // midpoint tree
+    DevBuf front_nodes[2], front_routes, front_rounds, front_w, front_c, front_m, front_h;   // frontier
     bool mid_clean = false;          // its cells are all zero
     DevBuf small_table, small_report;   // the small problems of a batch and what they report
     DevBuf loads;                    // per-part loads (imbalance)
@@ -293,6 +296,23 @@ inline bool mid_from_env() {
     return !(v && v[0] == '0');
 }
 
+// COUPE_HIP_FRONT=0: the points of every call past the midpoint tree are moved
+// level by level.
+inline bool front_from_env() {
+    const char *v = getenv("COUPE_HIP_FRONT");
+    return !(v && v[0] == '0');
+}
+
+// Whether a switch of the general path is set in the environment: such a
+// context runs that path, as the switches say.
+inline bool general_from_env() {
+    for (const char *name : {"COUPE_HIP_PAIRS", "COUPE_HIP_FORWARD", "COUPE_HIP_FULL_FIRST", "COUPE_HIP_BIN_COPIES",
+                             "COUPE_HIP_MOVE_NT_BYTES", "COUPE_HIP_SEARCH_CHUNK", "COUPE_HIP_GRAPHS", "COUPE_HIP_BINS",
+                             "COUPE_HIP_WG_PER_CU", "COUPE_HIP_SCAN_DIRECT", "COUPE_HIP_SEARCH_PASSES"})
+        if (getenv(name)) return true;
+    return false;
+}
+
 // COUPE_HIP_SEARCH_CHUNK=k: the later search passes hand k consecutive
 // tiles at a time to each workgroup (default 2, at most 64).
 inline uint32_t search_chunk_from_env() {
@@ -358,7 +378,8 @@ inline void configure_from_env(Context &c) {
     c.copy_parts = copy_parts_from_env();
     c.search_chunk = search_chunk_from_env();
     c.small = small_from_env();
-    c.mid = mid_from_env();
+    c.mid = mid_from_env() && !general_from_env();
+    c.front = front_from_env() && !general_from_env();
     c.move_nt_bytes = move_nt_bytes_from_env();
     c.max_bins = bins_from_env();
     c.wg_cap = wg_cap_from_env();

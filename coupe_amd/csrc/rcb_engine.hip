@@ -17,6 +17,7 @@
 #include "rcb_pairs.h"
 #include "rcb_small.h"
 #include "rcb_mid.h"
+#include "rcb_front.h"
 
 namespace coupe_hip {
 
@@ -1083,12 +1084,19 @@ constexpr uint64_t kMidCopied = 1ull << 16;       // cells kept in one copy per 
 // Whether a call takes it: its levels fit the cells, no switch asks for the
 // general path's passes or its graph, its buffers may grow, and the last call
 // of the shape did not end on the general path.
-static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
-    if (!cx.mid || !cx.pairs || !cx.forward || spec_passes <= 0 || cx.capturing || cx.graphs || t_arena) return false;
+static bool in_place_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
+    if (spec_passes <= 0 || cx.capturing || cx.graphs || t_arena) return false;
     if (!B.dense || B.max_levels == 0 || B.max_levels > kMidLevels) return false;
-    if (B.heap_total + B.inst.size() > kMidCells) return false;
+    return B.heap_total + B.inst.size() <= kMidCells;
+}
+static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
+    if (!cx.mid || !in_place_fits(cx, B, spec_passes)) return false;
     const Hints *seen = cx.hints_for(B.shape);
     return !seen || seen->mid != 0;
+}
+// And whether the frontier (rcb_front.h) takes it after that.
+static bool front_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
+    return cx.front && B.inst.size() == 1 && B.n <= kFrontPoints && in_place_fits(cx, B, spec_passes);
 }
 
 template <typename K>
@@ -1096,6 +1104,35 @@ static void allow_lds(K kernel, uint32_t lds) {
     if (lds > 65536)
         check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)lds));
+}
+
+// The open nodes' subtrees (k_mid_search), from the gathered points.
+template <int D, typename WL, typename Acc>
+static void search_nodes(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t cells,
+                         const uint32_t *gate) {
+    timed(cx, st, COUPE_HIP_K_HIST, 0.0, [&] {
+        const uint32_t lds = sub_lds(B.max_levels, kMidThreads);
+        allow_lds(k_mid_search<D, WL, Acc>, lds);
+        const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)cx.cu_count, cells);
+        k_mid_search<D, WL, Acc><<<grid, kMidThreads, lds, st>>>(
+            (const MidOpen *)cx.mid_open.ptr, (const uint32_t *)cx.mid_lists.ptr, cells, (Instance *)cx.instances.ptr,
+            (const MidPoint<D, WL> *)cx.mid_points.ptr, (uint16_t *)cx.mid_slots.ptr, wrap32,
+            (float *)cx.heap_split.ptr, (MidCounters *)((char *)cx.counters.ptr + offsetof(Counters, mid)), gate);
+    });
+}
+
+// Reads the call's counters back (and `more` bytes of `also` to the readback
+// area's end) and waits for the stream.
+constexpr size_t kFrontReadback = 53248;   // past the early prologue readback
+static MidCounters wait_counters(Context &cx, hipStream_t st, const void *also = nullptr, size_t more = 0) {
+    static_assert(kFrontReadback + kFrontRounds * sizeof(FrontRound) <= kHostScratch, "readback areas");
+    static_assert(kPrologueEarly + kCopies * sizeof(Prologue) <= kFrontReadback, "readback areas");
+    char *h_rb = (char *)cx.host_scratch + 256;
+    const size_t off = offsetof(Counters, swept);
+    check(hipMemcpyAsync(h_rb, (char *)cx.counters.ptr + off, offsetof(Counters, spec) - off, hipMemcpyDeviceToHost, st));
+    if (more) check(hipMemcpyAsync((char *)cx.host_scratch + kFrontReadback, also, more, hipMemcpyDeviceToHost, st));
+    check(hipStreamSynchronize(st));
+    return *(const MidCounters *)(h_rb + (offsetof(Counters, mid) - off));
 }
 
 // Runs a call on the midpoint tree after its prologue.  w: the stored weights,
@@ -1174,18 +1211,12 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
     });
     auto search_open = [&] {
         timed(cx, st, COUPE_HIP_K_PARTITION, 0.0, [&] {
-            const unsigned grid = persistent_grid(cx, k_mid_gather<D, WL>, nt);
-            k_mid_gather<D, WL><<<grid, kBlock, 0, st>>>(tiles, nt, insts, minst, c[0], c[1], c[2], w, w_src, code,
-                                                        map, cursor, (Point *)cx.mid_points.ptr, mid);
+            const unsigned grid = persistent_grid(cx, k_mid_gather<D, WL, false>, nt);
+            k_mid_gather<D, WL, false><<<grid, kBlock, 0, st>>>(tiles, nt, insts, minst, c[0], c[1], c[2], w, w_src,
+                                                               code, map, cursor, (Point *)cx.mid_points.ptr, mid,
+                                                               nullptr);
         });
-        timed(cx, st, COUPE_HIP_K_HIST, 0.0, [&] {
-            const uint32_t lds = sub_lds(B.max_levels, kMidThreads);
-            allow_lds(k_mid_search<D, WL, Acc>, lds);
-            const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)cx.cu_count, cells);
-            k_mid_search<D, WL, Acc><<<grid, kMidThreads, lds, st>>>(open, lists, cells, insts,
-                                                                    (const Point *)cx.mid_points.ptr,
-                                                                    (uint16_t *)cx.mid_slots.ptr, wrap32, heap, mid);
-        });
+        search_nodes<D, WL, Acc>(cx, st, B, wrap32, cells, nullptr);
     };
     auto ids = [&] {
         const double bytes = 10.0 * (double)n;
@@ -1200,25 +1231,18 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
         if (n_inst == 1 && (4.0 * D + 8.0) * (double)n > cx.move_nt_bytes) launch(k_mid_ids<D, true>);
         else launch(k_mid_ids<D, false>);
     };
-    auto wait = [&] {
-        char *h_rb = (char *)cx.host_scratch + 256;
-        const size_t off = offsetof(Counters, swept);
-        check(hipMemcpyAsync(h_rb, (char *)ctr + off, offsetof(Counters, spec) - off, hipMemcpyDeviceToHost, st));
-        check(hipStreamSynchronize(st));
-        return *(const MidCounters *)(h_rb + (offsetof(Counters, mid) - off));
-    };
     // a shape whose last call left no node open queues no search; open nodes
     // after all are searched once the counters are read
     const Hints *seen = cx.hints_for(B.shape);
     const bool expect = !seen || seen->mid < 0 || seen->mid_open > 0;
     if (expect) search_open();
     ids();
-    MidCounters m = wait();
+    MidCounters m = wait_counters(cx, st);
     if (!expect && m.open && !m.big) {
         cx.stats.reruns = 1;
         search_open();
         ids();
-        m = wait();
+        m = wait_counters(cx, st);
     }
     if (m.error) throw HipFailure{hipErrorUnknown};
     cx.mid_clean = true;
@@ -1233,6 +1257,118 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
     cx.stats.unit_points = kTile;
     cx.stats.bins = m.open ? (uint32_t)kSubMaxNb : 2u;
     return true;
+}
+
+// Runs a call of one instance on the frontier after its prologue (w, w_src as
+// for run_mid).  Waits for the stream and reads the call's counters.
+template <int D, typename WL, typename Acc>
+static void run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
+                      int w_src) {
+    const uint64_t n = B.n, cells = B.heap_total + 1;
+    const uint32_t nt = (uint32_t)B.tiles0;
+    // a workgroup has at least 16384 points: its bins are its own, and adding
+    // the workgroups' bins takes the decision longer than a second group of
+    // points takes the sweep (2^21 points: 13.6 + 19.5 us a round with 256
+    // workgroups, 16.6 + 13.3 with 128)
+    const unsigned grid = (unsigned)std::min<uint64_t>(std::min<uint64_t>(kFrontCopies, std::max(cx.cu_count, 1)),
+                                                       (n + 16383) / 16384);
+    const uint64_t bins = (uint64_t)kFrontCopies * kFrontBins;
+    const uint32_t small = (uint32_t)std::max<uint64_t>(kMidClass[1], (n + kFrontNodes - 1) / kFrontNodes);
+    cx.mid_code.ensure(n * 2);
+    cx.mid_open.ensure(cells * sizeof(MidOpen));
+    cx.mid_cursor.ensure(cells * 4);
+    cx.mid_lists.ensure(kMidClasses * cells * 4);
+    cx.mid_slots.ensure(n * 2);
+    cx.mid_points.ensure(n * sizeof(MidPoint<D, WL>));
+    cx.mid_inst.ensure(sizeof(MidInstance));
+    cx.heap_split.ensure(B.heap_total * sizeof(float));
+    for (int k = 0; k < 2; k++) cx.front_nodes[k].ensure(kFrontNodes * sizeof(FrontNode));
+    cx.front_routes.ensure(kFrontNodes * sizeof(FrontRoute));
+    cx.front_rounds.ensure(kFrontRounds * sizeof(FrontRound));
+    cx.front_w.ensure(bins * 8);
+    cx.front_c.ensure(bins * 4);
+    cx.front_m.ensure(bins * 4);
+    cx.front_h.ensure((uint64_t)kFrontCopies * kFrontNodes * 4);
+    MidCounters *mid = (MidCounters *)((char *)cx.counters.ptr + offsetof(Counters, mid));
+    FrontRound *rounds = (FrontRound *)cx.front_rounds.ptr;
+    FrontRoute *routes = (FrontRoute *)cx.front_routes.ptr;
+    Instance *insts = (Instance *)cx.instances.ptr;
+    const Tile *tiles = (const Tile *)cx.tiles0.ptr;
+    float *heap = (float *)cx.heap_split.ptr;
+    uint16_t *pid = (uint16_t *)cx.mid_code.ptr;
+    Acc *gw = (Acc *)cx.front_w.ptr;
+    uint32_t *gc = (uint32_t *)cx.front_c.ptr, *gm = (uint32_t *)cx.front_m.ptr, *gh = (uint32_t *)cx.front_h.ptr;
+    const float *c[3];
+    for (int k = 0; k < 3; k++) c[k] = k < D ? cx.coords0(k) : nullptr;
+    const WL *wp = w_src ? w + B.inst[0].src : w;
+    auto nodes = [&](int r) { return (FrontNode *)cx.front_nodes[r & 1].ptr; };
+    auto hist = [&](int r) {
+        allow_lds(k_front_hist<D, WL, Acc>, kFrontLds);
+        timed(cx, st, COUPE_HIP_K_HIST, (8.0 + sizeof(WL) + 2.0) * (double)n, [&] {
+            k_front_hist<D, WL, Acc><<<grid, kFrontThreads, kFrontLds, st>>>(r, rounds, nodes(r), routes, n, c[0], c[1],
+                                                                            c[2], wp, pid, gw, gc, gm, gh);
+        });
+    };
+    auto decide = [&](int r) {
+        const uint32_t lds = kSubMisc + sub_bins(kDecideThreads) * kSubBinBytes + 128 * kSubSlotBytes;
+        allow_lds(k_front_decide<D, WL, Acc>, lds + 16384);
+        timed(cx, st, COUPE_HIP_K_DECIDE, 0.0, [&] {
+            k_front_decide<D, WL, Acc><<<kFrontDecides, kDecideThreads, lds, st>>>(
+                r, rounds, nodes(r), nodes(r + 1), routes, grid, gw, gc, gm, gh, insts, wrap32, heap, small,
+                (MidOpen *)cx.mid_open.ptr, (uint32_t *)cx.mid_cursor.ptr, (uint32_t *)cx.mid_lists.ptr, cells, mid);
+        });
+    };
+    timed(cx, st, COUPE_HIP_K_OTHER, 0.0, [&] {
+        k_front_init<D, Acc><<<1, kBlock, 0, st>>>(insts, (const InstReduce *)cx.ired.ptr, nodes(0), rounds, mid);
+    });
+    hist(0);
+    // rounds queued without a look: what the shape's last call took and two
+    // more, or two per level; a call that takes longer goes on from there
+    const Hints *seen = cx.hints_for(B.shape);
+    int done = 0;
+    int queue = seen && seen->front_rounds ? (int)seen->front_rounds + 2 : 2 * (int)B.max_levels + 2;
+    MidCounters m;
+    const FrontRound *h = (const FrontRound *)((const char *)cx.host_scratch + kFrontReadback);
+    for (;;) {
+        const int to = std::min(done + queue, kFrontRounds - 2);
+        for (; done < to; done++) {
+            decide(done);
+            hist(done + 1);
+        }
+        const uint32_t *gate = &rounds[done].nodes;
+        timed(cx, st, COUPE_HIP_K_PARTITION, 0.0, [&] {
+            // (a workgroup takes places with one atomic per open node: few workgroups)
+            const unsigned g = std::min(persistent_grid(cx, k_mid_gather<D, WL, true>, (nt + 3) / 4), kFrontCopies);
+            k_mid_gather<D, WL, true><<<g, kBlock, 0, st>>>(tiles, nt, insts, (const MidInstance *)cx.mid_inst.ptr, c[0],
+                                                           c[1], c[2], w, w_src, pid, nullptr,
+                                                           (uint32_t *)cx.mid_cursor.ptr,
+                                                           (MidPoint<D, WL> *)cx.mid_points.ptr, mid, gate);
+        });
+        search_nodes<D, WL, Acc>(cx, st, B, wrap32, cells, gate);
+        const double bytes = (4.0 * D + 8.0) * (double)n;
+        timed(cx, st, COUPE_HIP_K_IDS, bytes, [&] {
+            const unsigned g = persistent_grid(cx, k_descend_dense<D, false>, B.tiles0);
+            k_descend_dense<D, false><<<g, kBlock, 0, st>>>(tiles, nt, insts, heap, c[0], c[1], c[2], d_out);
+        });
+        m = wait_counters(cx, st, rounds, kFrontRounds * sizeof(FrontRound));
+        if (m.error) throw HipFailure{hipErrorUnknown};
+        if (h[done].nodes == 0) break;
+        if (done >= kFrontRounds - 2) throw HipFailure{hipErrorUnknown};   // (never: f32 bisection ends long before)
+        cx.stats.reruns = 1;
+        queue = 8;
+    }
+    uint32_t used = 0;
+    while (used < (uint32_t)kFrontRounds && h[used].nodes) used++;
+    cx.pending.shape = B.shape;
+    Hints &e = cx.remember(B.shape);
+    e.front_rounds = used;
+    // the midpoint tree again when every level took one round
+    if (e.mid == 0 && used <= B.max_levels) e.mid = -1;
+    cx.stats.levels = B.max_levels;
+    cx.stats.passes = used;
+    cx.stats.max_passes = std::max(cx.stats.max_passes, 1u);
+    cx.stats.unit_points = kTile;
+    cx.stats.bins = kSubMaxNb;
 }
 
 template <int D, typename WIN>
@@ -1301,20 +1437,29 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
         }
         cx.pending.mode = mode;
         cx.pending.wkind = wkind;
-        if (mid_fits(cx, B, spec_passes)) {
+        // the midpoint tree, then the frontier, then the general path
+        const bool mid = mid_fits(cx, B, spec_passes), front = front_fits(cx, B, spec_passes);
+        if (mid || front) {
             cx.stats.weight_mode = mode == 3 ? 1 : 0;
             cx.stats.weight_bytes = weight_bytes(mode);
-            bool done;
-            if (mode == 0) done = run_mid<D, uint16_t, uint64_t>(cx, st, B, wrap32, d_out, (uint16_t *)cx.w16.ptr, 0);
-            else if (mode == 1) done = run_mid<D, int32_t, uint64_t>(cx, st, B, wrap32, d_out, (int32_t *)cx.w[0].ptr, 0);
-            else if (mode == 2) done = run_mid<D, WIN, uint64_t>(cx, st, B, wrap32, d_out, win, 1);
-            else if constexpr (std::is_same<WIN, double>::value)
-                done = run_mid<D, WIN, double>(cx, st, B, 0, d_out, win, 1);
-            else
-                done = false;   // (integers never need f64 sums)
+            auto in_place = [&](auto *w, auto acc, int w_src) {
+                using WL = typename std::remove_const<typename std::remove_pointer<decltype(w)>::type>::type;
+                using Acc = decltype(acc);
+                const int wrap = std::is_same<Acc, double>::value ? 0 : (int)wrap32;
+                if (mid) {
+                    if (run_mid<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src)) return true;
+                    cx.stats.reruns = 1;   // on, from the prologue's arrays
+                }
+                if (front) run_front<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
+                return front;
+            };
+            bool done = false;   // (integers never need f64 sums)
+            if (mode == 0) done = in_place((const uint16_t *)cx.w16.ptr, uint64_t{}, 0);
+            else if (mode == 1) done = in_place((const int32_t *)cx.w[0].ptr, uint64_t{}, 0);
+            else if (mode == 2) done = in_place(win, uint64_t{}, 1);
+            else if constexpr (std::is_same<WIN, double>::value) done = in_place(win, double{}, 1);
             if (!mode_held(cx)) continue;
             if (done) return false;
-            cx.stats.reruns = 1;   // on the general path, from the prologue's arrays
         }
         const bool unfinished = run_mode(mode);
         if (cx.capturing) return false;   // checked once the graph has run
@@ -1927,6 +2072,7 @@ void Context::for_each_buf(F &&f) {
                      &heap_split, &instances, &tiles0, &below, &tile_left, &loads, &rib_moments, &tile_bins,
                      &gparts[0], &gparts[1], &gaxis, &gchunk, &gcount, &gctr, &gsat, &gcol, &grow, &gheap, &gscan,
                      &mid_code, &mid_cnt, &mid_w, &mid_map, &mid_inst, &mid_open, &mid_cursor, &mid_lists, &mid_slots, &mid_points,
+                     &front_nodes[0], &front_nodes[1], &front_routes, &front_rounds, &front_w, &front_c, &front_m, &front_h,
                      &small_table, &small_report, &ired, &counters, &in_points, &in_weights, &out_ids};
     for (DevBuf *d : all) f(*d);
 }

@@ -39,6 +39,10 @@ struct MidOpen {
     uint32_t axis, levels;   // axis of its split, levels left
 };
 
+// A point's place in the frontier (rcb_front.h): a node of it, kFrontSmall + an
+// open node's number, or kFrontNone.
+constexpr uint32_t kFrontSmall = 0x8000u, kFrontNone = 0xffffu;
+
 // Counters of a call on this path (among the call's counters).
 struct MidCounters {
     uint32_t open;                  // open nodes
@@ -393,15 +397,17 @@ struct alignas(sizeof(WL) == 8 && D == 3 ? 8 : 16) MidPoint {
 // points per open node, takes places for them (one atomic per node) and
 // writes them, reading the 2-byte cells twice.
 // ---------------------------------------------------------------------------
-template <int D, typename WL>
+// FRONT: code holds the points' nodes of the frontier (rcb_front.h) instead of
+// cells, and gate the nodes it has left.
+template <int D, typename WL, bool FRONT>
 __global__ void __launch_bounds__(kBlock)
 k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__restrict__ insts,
              const MidInstance *__restrict__ minst, const float *__restrict__ c0, const float *__restrict__ c1,
              const float *__restrict__ c2, const WL *__restrict__ w, int w_src, const uint16_t *__restrict__ code,
              const uint32_t *__restrict__ map, uint32_t *__restrict__ cursor, MidPoint<D, WL> *__restrict__ gathered,
-             const MidCounters *ctr) {
-    if (ctr->open == 0 || ctr->big) return;
-    __shared__ uint16_t num[1 << kMidLevels];            // open node of a cell, 0xffff: settled
+             const MidCounters *ctr, const uint32_t *gate) {
+    if (ctr->open == 0 || ctr->big || (FRONT && *gate)) return;
+    __shared__ uint16_t num[FRONT ? 1 : 1 << kMidLevels];   // open node of a cell, 0xffff: settled
     __shared__ uint32_t place[1 << (kMidLevels - 1)];    // at most half as many open nodes as cells
     const int tid = threadIdx.x;
     uint32_t t0, t1;
@@ -414,7 +420,7 @@ k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *_
             const uint32_t last = I.tile_begin + (uint32_t)((I.count + kTile - 1) / kTile);
             e = last < t1 ? last : t1;
         }
-        const MidInstance M = minst[q];
+        const MidInstance M = FRONT ? MidInstance{0u, ctr->open} : minst[q];
         if (M.n_open == 0) {
             t = e;
             continue;
@@ -422,10 +428,15 @@ k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *_
         const uint32_t n_cells = 1u << I.levels;
         const uint64_t cbase = mid_cell_base(I, q), wbase = w_src ? I.src - I.begin : 0;
         __syncthreads();
-        for (uint32_t c = tid; c < n_cells; c += kBlock) {
-            const uint32_t m = map[cbase + c];
-            num[c] = m == kMidDone ? (uint16_t)0xffffu : (uint16_t)(m >> 16);
-        }
+        if constexpr (!FRONT)
+            for (uint32_t c = tid; c < n_cells; c += kBlock) {
+                const uint32_t m = map[cbase + c];
+                num[c] = m == kMidDone ? (uint16_t)0xffffu : (uint16_t)(m >> 16);
+            }
+        auto open_of = [&](uint16_t c) -> uint16_t {
+            if constexpr (FRONT) return c >= kFrontSmall && c != kFrontNone ? (uint16_t)(c - kFrontSmall) : (uint16_t)0xffffu;
+            else return num[c];
+        };
         for (uint32_t k = tid; k < M.n_open; k += kBlock) place[k] = 0;
         __syncthreads();
         const uint64_t begin = tiles[t].begin, end = tiles[e - 1].begin + tiles[e - 1].count;
@@ -440,7 +451,7 @@ k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *_
             }
 #pragma unroll
             for (int k = 0; k < G; k++) {
-                const uint16_t m = num[o[k]];
+                const uint16_t m = open_of(o[k]);
                 if (m != 0xffffu && i0 + (uint32_t)(k * kBlock) + tid < end) atomicAdd(&place[m], 1u);
             }
         }
@@ -458,7 +469,7 @@ k_mid_gather(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *_
             bool any = false;
 #pragma unroll
             for (int k = 0; k < G; k++) {
-                o[k] = i0 + (uint32_t)(k * kBlock) + tid < end ? num[o[k]] : (uint16_t)0xffffu;
+                o[k] = i0 + (uint32_t)(k * kBlock) + tid < end ? open_of(o[k]) : (uint16_t)0xffffu;
                 any |= o[k] != 0xffffu;
             }
             if (__ballot(any) == 0) continue;
@@ -556,7 +567,7 @@ __device__ __forceinline__ bool mid_memory(uint32_t count, const SubRoot &R, Acc
                     wk[j] = AccOps<Acc>::of(pts[p].w);
                     s[j] = first ? 0u : (uint32_t)slots[p];
                 }
-                sub_bin<B, TPB, Acc>(T, s, xa, wk, valid, nb, R.packed);
+                sub_bin<B>(T, s, [&](int j, uint32_t) { return xa[j]; }, wk, valid, nb, R.packed);
             }
         },
         [&](int a) {
@@ -586,8 +597,9 @@ template <int D, typename WL, typename Acc>
 __global__ void __launch_bounds__(kMidThreads)
 k_mid_search(const MidOpen *__restrict__ open, const uint32_t *__restrict__ lists, uint64_t list_stride,
              Instance *__restrict__ insts, const MidPoint<D, WL> *__restrict__ gathered,
-             uint16_t *__restrict__ slots, int wrap32, float *__restrict__ heap_split, MidCounters *ctr) {
-    if (ctr->big) return;
+             uint16_t *__restrict__ slots, int wrap32, float *__restrict__ heap_split, MidCounters *ctr,
+             const uint32_t *gate) {
+    if (ctr->big || (gate && *gate)) return;
     constexpr int TPB = kMidThreads;
     SmallShared &sh = *(SmallShared *)sub_lds_base;
     const uint32_t n0 = ctr->of_class[0], n1 = ctr->of_class[1], n2 = ctr->of_class[2], tid = threadIdx.x;

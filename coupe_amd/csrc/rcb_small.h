@@ -135,7 +135,7 @@ __device__ __forceinline__ bool reg_levels(uint32_t count, const float (&x)[IT][
                         asm volatile("" : "+v"(w[j]));
                     }
                 }
-                sub_bin<B, TPB, Acc>(T, s, xa, w, valid, nb, R.packed);
+                sub_bin<B>(T, s, [&](int j, uint32_t) { return xa[j]; }, w, valid, nb, R.packed);
             }
         },
         [&](int a) {

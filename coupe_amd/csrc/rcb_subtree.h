@@ -105,12 +105,16 @@ struct SubRoot {
 // estimate itself can be off; the other points (and all of a window that is
 // only a few ulps wide, or not finite) walk the midpoints par_rcb_split
 // computes (:472).
-template <int B, int TPB, typename Acc>
-__device__ __forceinline__ void sub_bin(const SubTree<Acc, TPB> &T, const uint32_t (&s)[B], const float (&x)[B],
-                                        const Acc (&w)[B], const bool (&valid)[B], int nb, bool packed) {
+// coord(j, flags): point j's coordinate on its window's axis.
+template <int B, typename Tree, typename Coord, typename Acc>
+__device__ __forceinline__ void sub_bin(const Tree &T, const uint32_t (&s)[B], Coord &&coord, const Acc (&w)[B],
+                                        const bool (&valid)[B], int nb, bool packed) {
     float4 v[B];
+    float x[B];
 #pragma unroll
     for (int j = 0; j < B; j++) v[j] = T.at(s[j]).win;
+#pragma unroll
+    for (int j = 0; j < B; j++) x[j] = coord(j, __builtin_bit_cast(uint32_t, v[j].w));
     bool in[B], any = false, mins = false;
 #pragma unroll
     for (int j = 0; j < B; j++) {
