@@ -1260,9 +1260,10 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
 }
 
 // Runs a call of one instance on the frontier after its prologue (w, w_src as
-// for run_mid).  Waits for the stream and reads the call's counters.
+// for run_mid).  Waits for the stream and reads the call's counters.  False:
+// its rounds are not enough.
 template <int D, typename WL, typename Acc>
-static void run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
+static bool run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
                       int w_src) {
     const uint64_t n = B.n, cells = B.heap_total + 1;
     const uint32_t nt = (uint32_t)B.tiles0;
@@ -1301,19 +1302,19 @@ static void run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap3
     const float *c[3];
     for (int k = 0; k < 3; k++) c[k] = k < D ? cx.coords0(k) : nullptr;
     const WL *wp = w_src ? w + B.inst[0].src : w;
+    const uint32_t decide_lds = kSubMisc + sub_bins(kDecideThreads) * kSubBinBytes + 128 * kSubSlotBytes;
+    allow_lds(k_front_hist<D, WL, Acc>, kFrontLds);
+    allow_lds(k_front_decide<D, WL, Acc>, decide_lds + 16384);
     auto nodes = [&](int r) { return (FrontNode *)cx.front_nodes[r & 1].ptr; };
     auto hist = [&](int r) {
-        allow_lds(k_front_hist<D, WL, Acc>, kFrontLds);
         timed(cx, st, COUPE_HIP_K_HIST, (8.0 + sizeof(WL) + 2.0) * (double)n, [&] {
             k_front_hist<D, WL, Acc><<<grid, kFrontThreads, kFrontLds, st>>>(r, rounds, nodes(r), routes, n, c[0], c[1],
                                                                             c[2], wp, pid, gw, gc, gm, gh);
         });
     };
     auto decide = [&](int r) {
-        const uint32_t lds = kSubMisc + sub_bins(kDecideThreads) * kSubBinBytes + 128 * kSubSlotBytes;
-        allow_lds(k_front_decide<D, WL, Acc>, lds + 16384);
         timed(cx, st, COUPE_HIP_K_DECIDE, 0.0, [&] {
-            k_front_decide<D, WL, Acc><<<kFrontDecides, kDecideThreads, lds, st>>>(
+            k_front_decide<D, WL, Acc><<<kFrontDecides, kDecideThreads, decide_lds, st>>>(
                 r, rounds, nodes(r), nodes(r + 1), routes, grid, gw, gc, gm, gh, insts, wrap32, heap, small,
                 (MidOpen *)cx.mid_open.ptr, (uint32_t *)cx.mid_cursor.ptr, (uint32_t *)cx.mid_lists.ptr, cells, mid);
         });
@@ -1353,8 +1354,8 @@ static void run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap3
         m = wait_counters(cx, st, rounds, kFrontRounds * sizeof(FrontRound));
         if (m.error) throw HipFailure{hipErrorUnknown};
         if (h[done].nodes == 0) break;
-        if (done >= kFrontRounds - 2) throw HipFailure{hipErrorUnknown};   // (never: f32 bisection ends long before)
         cx.stats.reruns = 1;
+        if (done >= kFrontRounds - 2) return false;   // (coordinates over all of f32's exponents)
         queue = 8;
     }
     uint32_t used = 0;
@@ -1369,6 +1370,7 @@ static void run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap3
     cx.stats.max_passes = std::max(cx.stats.max_passes, 1u);
     cx.stats.unit_points = kTile;
     cx.stats.bins = kSubMaxNb;
+    return true;
 }
 
 template <int D, typename WIN>
@@ -1450,8 +1452,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
                     if (run_mid<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src)) return true;
                     cx.stats.reruns = 1;   // on, from the prologue's arrays
                 }
-                if (front) run_front<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
-                return front;
+                return front && run_front<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
             };
             bool done = false;   // (integers never need f64 sums)
             if (mode == 0) done = in_place((const uint16_t *)cx.w16.ptr, uint64_t{}, 0);
