@@ -4,8 +4,9 @@
 // The grid is split level by level.  At level l every non-empty subgrid
 // (a box of cells) is cut across axis (1 + l) mod D at the weighted median
 // of its axis sums (the sums of its weights over the cross-section at each
-// index of that axis).  Two paths: the summed-area path further down (calls
-// of at most 20 levels whose weights are exactly summable) and the
+// index of that axis).  Three paths: for calls of at most 20 levels whose
+// weights are exactly summable the summed-area path further down, or, where
+// a large 2D grid makes its table the cost, the strips after it; else the
 // per-level path, which reads the weights at every level:
 //   k_grid_counts + scans  chunks of 4096 cells and axis-sum slots per subgrid
 //   k_grid_axis            one pass over the cells of every subgrid: axis sums
@@ -856,58 +857,31 @@ __device__ inline uint64_t sat_carrier(SatAcc<K> v) {
     else return __builtin_bit_cast(uint64_t, v);
 }
 
-// One wavefront per subgrid h of level l (2^l of them): weighted_median
-// (rcb.rs:52-99) with every chunk's prefix weight a lookup (the weight of
-// the subgrid's cross-sections before the chunk's start: coupe's
-// left_weight + prefix, the same integer; the first chunk's is the left
-// weight itself), the decisions by ballot in
-// coupe's order; then the split into the heap and the two halves into
-// slots 2h and 2h + 1 of the next level.
-template <int K, int D>
-__global__ void __launch_bounds__(kBlock)
-k_grid_level(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint32_t l,
-             const SatAcc<K> *__restrict__ S, uint64_t gx, uint64_t gy, uint64_t gz, uint32_t threads) {
+// weighted_median (rcb.rs:52-99) of m cross-sections by one wavefront: every
+// chunk's prefix weight is a lookup (`before(pos)`, pos >= 1: the weight of
+// the cross-sections before pos: coupe's left_weight + prefix, the same
+// integer; the first chunk's is the left weight itself), the decisions by
+// ballot in coupe's order.
+template <int K, typename Before>
+__device__ inline void median_rounds(uint64_t m, uint64_t total, uint32_t threads, uint64_t &pos_out,
+                                     uint64_t &left_out, Before &&before) {
     using Wt = GW<K>;
     const int lane = threadIdx.x & 63;
-    const uint64_t n = (uint64_t)1 << l;
-    const uint64_t h = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (h >= n) return;
-    const int coord = (int)((1 + l) % D);
-    GSlot P;   // level 0: the whole grid
-    if (l == 0) P = GSlot{{0, 0, 0}, {(uint32_t)gx, (uint32_t)gy, (uint32_t)gz}, 0};
-    else P = in[h];
-    if (P.size[0] == 0 || P.size[1] == 0 || P.size[2] == 0) {   // no cells: nothing below reaches a cell
-        if (lane == 0) {
-            out[2 * h] = P;
-            out[2 * h + 1] = P;
-            heap[n - 1 + h] = 0;
-        }
-        return;
-    }
-    uint64_t lo[3], hi[3];
-    for (int k = 0; k < 3; k++) {
-        lo[k] = P.off[k];
-        hi[k] = (uint64_t)P.off[k] + P.size[k];
-    }
-    const uint64_t total = l == 0 ? sat_carrier<K>(sat_box<D>(S, gx, gy, lo, hi)) : P.sum;
     const double ideal = Wt::f64(total) / 2.0;
     const uint64_t minp = Wt::from_f64(ideal * (1.0 - kGridTolerance));
     const uint64_t maxp = Wt::from_f64(ideal * (1.0 + kGridTolerance));
-    const uint64_t m = P.size[coord];
-    const SatAcc<K> f0 = sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord]);
-    uint64_t mn = 0, mx = m, left = 0, pos_out = 0, left_out = 0;
+    uint64_t mn = 0, mx = m, left = 0;
     for (;;) {
         uint64_t cs = (mx - mn) / threads;
         if (cs < 1) cs = 1;
         const uint64_t nch = (mx - mn + cs - 1) / cs;
         uint64_t nmin = mn, nmax = mx, nleft = left;
-        bool done = false;
         for (uint64_t base = 0; base < nch; base += 64) {
             const uint64_t k = base + lane;
             const bool valid = k < nch;
             const uint64_t pos = mn + k * cs;
             uint64_t c = left;   // the first chunk starts at the left weight's position
-            if (valid && k > 0) c = sat_carrier<K>(sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord] + pos) - f0);
+            if (valid && k > 0) c = sat_carrier<K>(before(pos));
             const bool stop = valid && !Wt::lt(c, minp);
             const uint64_t mask = __ballot(stop);
             if (mask == 0) {   // every chunk of this batch below the minimum
@@ -927,31 +901,391 @@ k_grid_level(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *__
             } else {
                 pos_out = pf;
                 left_out = cf;
-                done = true;
+                return;
             }
             break;
         }
-        if (!done && (nmin + 1 >= nmax || (nmin == mn && nmax == mx))) {
+        if (nmin + 1 >= nmax || (nmin == mn && nmax == mx)) {
             pos_out = nmin;
             left_out = nleft;
-            done = true;
+            return;
         }
-        if (done) break;
         mn = nmin;
         mx = nmax;
         left = nleft;
     }
-    if (lane == 0) {
-        GSlot A = P, B = P;
-        A.size[coord] = (uint32_t)pos_out;
-        A.sum = left_out;
-        B.off[coord] = P.off[coord] + (uint32_t)pos_out;
-        B.size[coord] = (uint32_t)(m - pos_out);
-        B.sum = Wt::sub(total, left_out);
-        out[2 * h] = A;
-        out[2 * h + 1] = B;
-        heap[n - 1 + h] = P.off[coord] + (uint32_t)pos_out;
+}
+
+// A subgrid without cells: nothing below reaches a cell.
+__device__ inline bool slot_empty(const GSlot &P, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint64_t n,
+                                  uint64_t h, bool writes) {
+    if (P.size[0] != 0 && P.size[1] != 0 && P.size[2] != 0) return false;
+    if (writes) {
+        out[2 * h] = P;
+        out[2 * h + 1] = P;
+        heap[n - 1 + h] = 0;
     }
+    return true;
+}
+// The split of subgrid h of the level's n into the heap and its two halves
+// into slots 2h and 2h + 1 of the next level.
+template <int K>
+__device__ inline void slot_split(const GSlot &P, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint64_t n,
+                                  uint64_t h, int coord, uint64_t total, uint64_t pos, uint64_t left) {
+    GSlot A = P, B = P;
+    A.size[coord] = (uint32_t)pos;
+    A.sum = left;
+    B.off[coord] = P.off[coord] + (uint32_t)pos;
+    B.size[coord] = P.size[coord] - (uint32_t)pos;
+    B.sum = GW<K>::sub(total, left);
+    out[2 * h] = A;
+    out[2 * h + 1] = B;
+    heap[n - 1 + h] = P.off[coord] + (uint32_t)pos;
+}
+
+// One wavefront per subgrid h of level l (2^l of them).
+template <int K, int D>
+__global__ void __launch_bounds__(kBlock)
+k_grid_level(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint32_t l,
+             const SatAcc<K> *__restrict__ S, uint64_t gx, uint64_t gy, uint64_t gz, uint32_t threads) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t n = (uint64_t)1 << l;
+    const uint64_t h = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (h >= n) return;
+    const int coord = (int)((1 + l) % D);
+    GSlot P;   // level 0: the whole grid
+    if (l == 0) P = GSlot{{0, 0, 0}, {(uint32_t)gx, (uint32_t)gy, (uint32_t)gz}, 0};
+    else P = in[h];
+    if (slot_empty(P, out, heap, n, h, lane == 0)) return;
+    uint64_t lo[3], hi[3];
+    for (int k = 0; k < 3; k++) {
+        lo[k] = P.off[k];
+        hi[k] = (uint64_t)P.off[k] + P.size[k];
+    }
+    const uint64_t total = l == 0 ? sat_carrier<K>(sat_box<D>(S, gx, gy, lo, hi)) : P.sum;
+    const SatAcc<K> f0 = sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord]);
+    uint64_t pos = 0, left = 0;
+    median_rounds<K>(P.size[coord], total, threads, pos, left,
+                     [&](uint64_t p) { return sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord] + p) - f0; });
+    if (lane == 0) slot_split<K>(P, out, heap, n, h, coord, total, pos, left);
+}
+
+// ---------------------------------------------------------------------------
+// 2D grids too large for the caches: no table.  The weights are read once,
+// for column sums of bands of 16 rows and row sums of groups of 16 columns,
+// scanned (an eighth of the table together).  A subgrid's axis sum at an index
+// is then the difference of two entries at band (group) boundaries, corrected
+// by the weights between the boundary and the subgrid's edge: at most 8 at
+// each edge, from the nearer boundary.  Per level k_strip_axis takes the axis
+// sums of all subgrids, spread over the device whatever their sizes (one
+// workgroup per subgrid is bound by what a CU reads: 25-35 us for a level of
+// few subgrids, against 10-13, and as much for a level with one that stays
+// large), and k_strip_median the splits, a wavefront per subgrid.
+// The scans of bands and groups are in two parts, so that no pass of their
+// own goes over all entries: k_strip_sums writes the prefix within 4 bands (a
+// workgroup's) and within 32 groups (a tile's), and the totals of those are
+// scanned (the last entry, past the axis, is the total).
+// The edges' strips grow by sqrt(2) a level (see strips_fit).
+// 10^8 cells, 12 levels, f64: 890 -> 610 us: the table's 345 us (weights read
+// again, table written) and 57 us of scans gone, 15 us of scans and 90 us of
+// axis sums instead.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kStripEdge = 8;                         // most weights at an edge
+constexpr uint32_t kStripBands = kBlock / 64;              // bands of a partial scan: a wavefront each
+constexpr uint32_t kStripGroups = kSatCols / kSatRows;     // groups of a partial scan: a tile's
+constexpr uint32_t kStripChunks = 64;                      // most chunks of an axis: a wavefront scans them
+
+// Sums over each 8 (16) consecutive lanes, in all of them.
+template <int Ctrl, typename Acc>
+__device__ inline Acc dpp_lanes(Acc v) {
+    return __builtin_bit_cast(Acc, dpp_row64<Ctrl>(__builtin_bit_cast(uint64_t, v)));
+}
+template <typename Acc>
+__device__ inline Acc lanes8_total(Acc v) {
+    v += dpp_lanes<0xb1>(v);    // quad_perm 1 0 3 2
+    v += dpp_lanes<0x4e>(v);    // quad_perm 2 3 0 1
+    v += dpp_lanes<0x141>(v);   // row_half_mirror
+    return v;
+}
+template <typename Acc>
+__device__ inline Acc lanes16_total(Acc v) {
+    v = lanes8_total(v);
+    return v + dpp_lanes<0x140>(v);   // row_mirror
+}
+template <typename Acc>
+__device__ inline Acc shfl_acc(Acc v, int lane) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(Acc, (uint64_t)(uint32_t)__shfl((int)(uint32_t)b, lane) |
+                                       (uint64_t)(uint32_t)__shfl((int)(uint32_t)(b >> 32), lane) << 32);
+}
+
+// The scanned sums.  col: (nb + 1) x gx, the prefix of the bands within their
+// kStripBands (rows at a multiple of it are 0 and not written); col_sup:
+// the totals per kStripBands.  row: (groups + 1) x gy and row_sup the same of
+// the groups.
+template <typename Acc>
+struct StripSums {
+    Acc *col, *col_sup, *row, *row_sup;
+};
+
+// One workgroup per kStripBands bands of a segment of columns, a tile per
+// wavefront; flags as in k_sat_sums.
+template <int K, typename WIN>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+k_strip_sums(const WIN *__restrict__ w, SatGeom g, StripSums<SatAcc<K>> out, GridSatFlags *flags) {
+    using Acc = SatAcc<K>;
+    static_assert(kSatRows == 16, "rows in 8 lanes, twice; a group of columns in 8 lanes");
+    __shared__ Acc cs[kStripBands][kSatCols];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t ng = (uint32_t)(g.gx / kSatRows + (g.gx % kSatRows != 0));
+    const uint64_t tiles = (uint64_t)((g.nb + kStripBands - 1) / kStripBands) * g.nseg;
+    double abs_sum = 0.0;
+    uint32_t bad = 0;
+    for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const uint32_t sup = (uint32_t)(t / g.nseg), band = sup * kStripBands + wave;
+        SatTile T;
+        T.z = 0;
+        T.b = band;
+        T.s = (uint32_t)(t - (uint64_t)sup * g.nseg);
+        T.xl = (uint64_t)T.s * kSatCols + 2 * lane;
+        T.whole = (uint64_t)(T.s + 1) * kSatCols <= g.gx;
+        T.y0 = (uint64_t)band * kSatRows;
+        T.nr = T.y0 < g.gy ? (uint32_t)std::min<uint64_t>(kSatRows, g.gy - T.y0) : 0;   // (past the grid: no rows)
+        Acc col[kSatPer], fine[kSatChunks][2];   // lane 8 g + j: rows j and j + 8 over the chunk's group g
+#pragma unroll
+        for (uint32_t j = 0; j < kSatPer; j++) col[j] = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < kSatChunks; c++) fine[c][0] = fine[c][1] = 0;
+        if (T.nr) {
+#pragma unroll
+            for (uint32_t i0 = 0; i0 < kSatRows; i0 += kSatGroup) {
+                WIN v[kSatGroup][kSatPer];
+                load_rows<kSatGroup, true>(w, g, T, i0, v);
+#pragma unroll
+                for (uint32_t b = 0; b < kSatGroup; b++) {
+                    const uint32_t i = i0 + b;
+                    if (i >= T.nr) continue;
+#pragma unroll
+                    for (uint32_t j = 0; j < kSatPer; j++) {
+                        col[j] += sat_of<K>(v[b][j]);
+                        if constexpr (K == 2) {
+                            const double d = (double)v[b][j];
+                            abs_sum += fabs(d);
+                            bad |= !(d == trunc(d) && fabs(d) < 0x1p53);
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t c = 0; c < kSatChunks; c++) {
+                        const Acc r = lanes8_total(sat_of<K>(v[b][2 * c]) + sat_of<K>(v[b][2 * c + 1]));
+                        if ((lane & 7) == i % 8) fine[c][i / 8] = r;
+                    }
+                }
+            }
+        }
+        // the bands' prefix within the workgroup
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < kSatPer; j++) cs[wave][j * 64 + lane] = col[j];
+        __syncthreads();
+        Acc ex[kSatPer];
+#pragma unroll
+        for (uint32_t j = 0; j < kSatPer; j++) {
+            ex[j] = 0;
+            for (uint32_t k = 0; k < wave; k++) ex[j] += cs[k][j * 64 + lane];
+        }
+        if (wave != 0 && band <= g.nb) store_lane(out.col + (uint64_t)band * g.gx, T, g.gx, g.vec_s, ex);
+        if (wave == kStripBands - 1) {
+#pragma unroll
+            for (uint32_t j = 0; j < kSatPer; j++) ex[j] += col[j];
+            store_lane(out.col_sup + (uint64_t)sup * g.gx, T, g.gx, g.vec_s, ex);
+        }
+        // the groups' prefix within the tile
+#pragma unroll
+        for (uint32_t k = 0; k < 2; k++) {
+            const uint32_t row = 8 * k + (lane & 7);
+            Acc carry = 0;
+#pragma unroll
+            for (uint32_t c = 0; c < kSatChunks; c++) {
+                const Acc v = fine[c][k];
+                Acc inc = v;
+#pragma unroll
+                for (uint32_t d = 8; d < 64; d *= 2) {
+                    const Acc below = shfl_acc(inc, (int)((lane - d) & 63));
+                    inc += lane >= d ? below : (Acc)0;
+                }
+                const uint32_t in = 8 * c + (lane >> 3), group = T.s * kStripGroups + in;
+                if (in != 0 && group <= ng && row < T.nr) out.row[group * g.gy + T.y0 + row] = carry + (inc - v);
+                carry += shfl_acc(inc, (int)(56 + (lane & 7)));
+            }
+            if (lane < 8 && row < T.nr) out.row_sup[T.s * g.gy + T.y0 + row] = carry;
+        }
+    }
+    if constexpr (K == 2) {
+        abs_sum = wave_total(abs_sum);
+        bad = wave_total(bad);
+        GridSatFlags *f = flags + blockIdx.x % kCopies;   // one copy per XCD
+        if (lane == 0) {
+            if (abs_sum != 0.0) atomicAdd(&f->abs_sum, abs_sum);
+            if (bad) atomicOr(&f->bad, 1u);
+        }
+    }
+}
+
+// An edge of a subgrid at index X of an axis of n cells: entry `blk` of the
+// scanned sums, plus (minus) the `count` cross-sections from `first` on.
+struct StripEdge {
+    uint32_t blk, first, count;
+    bool minus;
+};
+__device__ inline StripEdge strip_edge(uint32_t X, uint32_t n) {
+    const uint32_t q = X / kSatRows, r = X % kSatRows, nblk = n / kSatRows + (n % kSatRows != 0);
+    if (X == n) return {nblk, 0, 0, false};
+    const uint32_t end = (q + 1 < nblk ? (q + 1) * kSatRows : n), up = end - X;
+    if (r <= up) return {q, q * kSatRows, r, false};
+    return {q + 1, X, up, true};
+}
+
+// The subgrids of a level that share the decisions at splits of the other
+// axis (a path, its bits those of levels l - 1, l - 3, ..) are disjoint along
+// this one: one line per path holds their axis sums, each at its own place.
+__device__ inline uint32_t strip_path(uint32_t h, uint32_t l) {
+    uint32_t path = 0;
+    for (uint32_t k = l, j = 0; k >= 1; k = k >= 2 ? k - 2 : 0, j++) path |= ((h >> (l - k)) & 1u) << j;
+    return path;
+}
+__device__ inline GSlot strip_slot(const GSlot *__restrict__ in, uint64_t h, uint32_t l, uint64_t gx, uint64_t gy) {
+    return l == 0 ? GSlot{{0, 0, 0}, {(uint32_t)gx, (uint32_t)gy, 1}, 0} : in[h];   // level 0: the whole grid
+}
+
+// One workgroup per path and chunk of `len` indexes (a multiple of kBlock):
+// the axis sums and their prefix within the chunk into the path's line, the
+// chunk's total into totals.  Level l splits axis `COORD`.
+template <int K, typename WIN, int COORD>
+__global__ void __launch_bounds__(kBlock)
+k_strip_axis(const GSlot *__restrict__ in, const uint32_t *__restrict__ heap, uint32_t l, const WIN *__restrict__ w,
+             uint32_t gx, uint32_t gy, StripSums<SatAcc<K>> sums, SatAcc<K> *__restrict__ line,
+             SatAcc<K> *__restrict__ totals, uint32_t chunks, uint32_t len) {
+    using Acc = SatAcc<K>;
+    constexpr uint32_t W = kBlock / 64, part = COORD ? kStripGroups : kStripBands;
+    __shared__ uint32_t top[(1u << kFillTop) - 1];
+    __shared__ uint32_t edges[kBlock][2];
+    __shared__ Acc strip[kBlock], tot[2][W];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t path = blockIdx.x / chunks, chunk = blockIdx.x - path * chunks;
+    const uint32_t along = COORD ? gy : gx, other = COORD ? gx : gy;
+    const uint32_t lt = l < kFillTop ? l : kFillTop;
+    for (uint32_t i = tid; i < (1u << lt) - 1; i += kBlock) top[i] = heap[i];
+    __syncthreads();
+    const Acc *esup = COORD ? sums.row_sup : sums.col_sup, *ein = COORD ? sums.row : sums.col;
+    const uint32_t x1 = std::min<uint64_t>(along, (uint64_t)(chunk + 1) * len);
+    Acc carry = 0;
+    uint32_t it = 0;
+    for (uint32_t x0 = chunk * len; x0 < x1; x0 += kBlock, it++) {
+        const uint32_t x = std::min(x0 + tid, x1 - 1);
+        // the subgrid of index x on this path, and its edges on the other axis
+        uint32_t node = 0;
+        for (uint32_t k = 0; k < l; k++) {
+            const uint32_t at = k < lt ? top[node] : heap[node];
+            const uint32_t right = (1 + k) % 2 == COORD ? (uint32_t)(x >= at) : path >> ((l - 1 - k) / 2) & 1u;
+            node = 2 * node + 1 + right;
+        }
+        uint32_t o0 = 0, o1 = other;   // level 0: the whole grid
+        if (l) {
+            const GSlot &P = in[node + 1 - (1u << l)];
+            o0 = P.off[1 - COORD];
+            o1 = o0 + P.size[1 - COORD];
+        }
+        if (COORD == 1 && l) {
+            // rows: the 16 weights at both edges by 16 lanes, four rows per load
+            edges[tid][0] = o1;
+            edges[tid][1] = o0;
+            __syncthreads();
+            const uint32_t i = lane & 7;
+            constexpr uint32_t R = 8;   // loads in flight
+#pragma unroll
+            for (uint32_t u0 = 0; u0 < 16; u0 += R) {
+                WIN v[R];
+                uint32_t on = 0, minus = 0;
+#pragma unroll
+                for (uint32_t u = 0; u < R; u++) {
+                    const uint32_t p = wave * 64 + 4 * (u0 + u) + (lane >> 4);
+                    const StripEdge e = strip_edge(edges[p][(lane >> 3) & 1], other);
+                    // (all in flight: past the edge's count another cell of the row)
+                    v[u] = w[(uint64_t)std::min(x0 + p, x1 - 1) * gx + std::min(e.first + i, other - 1)];
+                    on |= (uint32_t)(i < e.count) << u;
+                    minus |= (uint32_t)(e.minus != ((lane & 8) != 0)) << u;
+                }
+                Acc keep = 0;
+#pragma unroll
+                for (uint32_t u = 0; u < R; u++) {
+                    const Acc a = on >> u & 1 ? sat_of<K>(v[u]) : (Acc)0;
+                    const Acc s = lanes16_total(minus >> u & 1 ? (Acc)0 - a : a);
+                    if ((lane & 15) == u) keep = s;
+                }
+                if ((lane & 15) < R) strip[wave * 64 + 4 * (u0 + (lane & 15)) + (lane >> 4)] = keep;
+            }
+            __syncthreads();
+        }
+        auto upto = [&](uint32_t X) -> Acc {   // the weight at index x before X on the other axis
+            const StripEdge e = strip_edge(X, other);
+            Acc s = esup[(uint64_t)(e.blk / part) * along + x];
+            if (e.blk % part) s += ein[(uint64_t)e.blk * along + x];
+            if constexpr (COORD == 0) {
+                WIN v[kStripEdge];
+                // (all in flight: past the edge's count its last again, a cell of the line either way)
+                const uint32_t last = e.count ? e.first + e.count - 1 : std::min(e.first, other - 1);
+#pragma unroll
+                for (uint32_t i = 0; i < kStripEdge; i++) v[i] = w[(uint64_t)std::min(e.first + i, last) * gx + x];
+                Acc a = 0;
+#pragma unroll
+                for (uint32_t i = 0; i < kStripEdge; i++) a += i < e.count ? sat_of<K>(v[i]) : (Acc)0;
+                s = e.minus ? s - a : s + a;
+            }
+            return s;
+        };
+        Acc raw = upto(o1);
+        if (o0) raw -= upto(o0);
+        if (COORD == 1 && l) raw += strip[tid];
+        if (x0 + tid >= x1) raw = 0;
+        const Acc inc = wave_scan(raw);
+        if (lane == 63) tot[it & 1][wave] = inc;
+        __syncthreads();
+        Acc before = carry;
+        for (uint32_t k = 0; k < W; k++) {
+            if (k < wave) before += tot[it & 1][k];
+            carry += tot[it & 1][k];
+        }
+        if (x0 + tid < x1) line[(uint64_t)path * along + x] = before + inc;
+    }
+    if (tid == 0) totals[blockIdx.x] = carry;
+}
+
+// The splits of level l, a wavefront per subgrid.
+template <int K>
+__global__ void __launch_bounds__(kBlock)
+k_strip_median(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint32_t l,
+               uint64_t gx, uint64_t gy, const SatAcc<K> *__restrict__ line, const SatAcc<K> *__restrict__ totals,
+               uint32_t chunks, uint32_t len, uint32_t threads) {
+    using Acc = SatAcc<K>;
+    __shared__ Acc before[kBlock / 64][kStripChunks];   // weight of the line's chunks before
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t n = (uint64_t)1 << l, h = (uint64_t)blockIdx.x * (kBlock / 64) + wave;
+    if (h >= n) return;
+    const int coord = (int)((1 + l) % 2);
+    const GSlot P = strip_slot(in, h, l, gx, gy);
+    if (slot_empty(P, out, heap, n, h, lane == 0)) return;
+    const uint32_t path = strip_path((uint32_t)h, l);
+    const Acc t = lane < chunks ? totals[(uint64_t)path * chunks + lane] : (Acc)0;
+    before[wave][lane] = wave_scan(t) - t;   // (a wavefront's own row: in order)
+    __builtin_amdgcn_wave_barrier();
+    const Acc *mine = line + (uint64_t)path * (coord ? gy : gx);
+    auto upto = [&](uint64_t x) -> Acc { return x ? mine[x - 1] + before[wave][(uint32_t)(x - 1) / len] : (Acc)0; };
+    const uint32_t off = P.off[coord], m = P.size[coord];
+    const Acc f0 = upto(off);
+    const uint64_t total = l == 0 ? sat_carrier<K>(upto(m)) : P.sum;
+    uint64_t pos = 0, left = 0;
+    median_rounds<K>(m, total, threads, pos, left, [&](uint64_t q) { return upto(off + q) - f0; });
+    if (lane == 0) slot_split<K>(P, out, heap, n, h, coord, total, pos, left);
 }
 
 // part_of (rcb.rs:21-42) from the heap of splits: at level l the cell goes
@@ -1214,6 +1548,43 @@ void colscan(Context &cx, hipStream_t st, Acc *a, uint64_t W, uint32_t rows, uin
     ck(hipGetLastError());
 }
 
+// The ids from the heap of splits; false when f64 weights turned out not to be
+// exactly summable.  Waits for the stream.
+template <int K>
+bool grid_ids(Context &cx, hipStream_t st, size_t dim, const SatGeom &g, const uint32_t *heap, size_t L,
+              const GridSatFlags *flags, uint64_t *out) {
+    const uint64_t cells = g.gx * g.gy * g.gz;
+    const uint64_t fill_chunks = (cells + kBlock * kFillCells - 1) / (kBlock * kFillCells);
+    const double inv_gx = 1.0 / (double)g.gx, inv_gy = 1.0 / (double)g.gy;
+    const int r = cx.prof.begin(st, COUPE_HIP_K_IDS, (double)cells * 8.0);
+    if (dim == 2)
+        k_grid_fill_heap<2><<<fill_grid(cx, k_grid_fill_heap<2>, fill_chunks), kBlock, 0, st>>>(heap, (uint32_t)L, g.gx, g.gy,
+                                                                                        cells, inv_gx, inv_gy, out);
+    else
+        k_grid_fill_heap<3><<<fill_grid(cx, k_grid_fill_heap<3>, fill_chunks), kBlock, 0, st>>>(heap, (uint32_t)L, g.gx, g.gy,
+                                                                                        cells, inv_gx, inv_gy, out);
+    ck(hipGetLastError());
+    cx.prof.end(st, r);
+    if (K != 2) {
+        ck(hipStreamSynchronize(st));
+        return true;
+    }
+    if (!cx.host_scratch) ck(hipHostMalloc(&cx.host_scratch, kHostScratch, hipHostMallocDefault));
+    GridSatFlags *hf = (GridSatFlags *)cx.host_scratch;
+    ck(hipMemcpyAsync(hf, flags, kCopies * sizeof(GridSatFlags), hipMemcpyDeviceToHost, st));
+    ck(hipStreamSynchronize(st));
+    double abs_sum = 0.0;
+    uint32_t bad = 0;
+    for (int c = 0; c < kCopies; c++) {
+        abs_sum += hf[c].abs_sum;
+        bad |= hf[c].bad;
+    }
+    // Every partial sum is an integer of magnitude at most sum |w|; the f64
+    // sum of the magnitudes, over at most 2^36 terms, is within a factor
+    // 1 + 2^-17 of the exact one, so this bound keeps the exact sum <= 2^53.
+    return bad == 0 && cells <= (1ull << 36) && abs_sum <= 0x1p53 * (1.0 - 0x1p-15);
+}
+
 // The summed-area path.  Returns false when f64 weights are not exactly
 // summable (then nothing it wrote is a result and the caller runs the
 // per-level path).
@@ -1290,35 +1661,98 @@ bool grid_run_sat(Context &cx, hipStream_t st, size_t dim, const uint64_t *size,
     }
     cx.prof.end(st, r);
 
-    const uint64_t fill_chunks = (cells + kBlock * kFillCells - 1) / (kBlock * kFillCells);
-    const double inv_gx = 1.0 / (double)g.gx, inv_gy = 1.0 / (double)g.gy;
-    r = cx.prof.begin(st, COUPE_HIP_K_IDS, (double)cells * 8.0);
-    if (dim == 2)
-        k_grid_fill_heap<2><<<fill_grid(cx, k_grid_fill_heap<2>, fill_chunks), kBlock, 0, st>>>(heap, (uint32_t)L, g.gx, g.gy,
-                                                                                        cells, inv_gx, inv_gy, out);
-    else
-        k_grid_fill_heap<3><<<fill_grid(cx, k_grid_fill_heap<3>, fill_chunks), kBlock, 0, st>>>(heap, (uint32_t)L, g.gx, g.gy,
-                                                                                        cells, inv_gx, inv_gy, out);
+    return grid_ids<K>(cx, st, dim, g, heap, L, flags, out);
+}
+
+// Lines of level l: the splits of the other axis above it.
+uint32_t strip_paths(size_t l) { return 1u << (l % 2 ? (l + 1) / 2 : l / 2); }
+
+// Whether a 2D call goes by strips instead of the table.  They save the
+// table's write and the second read of the weights (8 + 8 bytes a cell at
+// about 4.6 TB/s); a cross-section of a level costs about 110 bytes along x
+// (two entries, 8 to 16 weights, the prefix) and, in whole lines, 400 along
+// y, at about 2 TB/s, and a level a few microseconds more than the wavefronts
+// on the table take.  (COUPE_HIP_GRID_STRIPS=1, 0: always, never.)
+bool strips_fit(size_t dim, const uint64_t *size, size_t L, size_t wbytes, uint64_t &line) {
+    const char *e = getenv("COUPE_HIP_GRID_STRIPS");
+    line = 1;
+    if (dim != 2 || L == 0 || std::max(size[0], size[1]) >> 31 || (e && e[0] == '0')) return false;
+    double cost = 0.0;   // nanoseconds
+    for (size_t l = 0; l < L; l++) {
+        const bool y = l % 2 == 0;
+        const uint64_t along = y ? size[1] : size[0], paths = strip_paths(l);
+        cost += (double)along * (double)paths * (y ? 0.2 : 0.055) + 5000.0;
+        line = std::max(line, along * paths);
+    }
+    if (e && e[0] == '1') return true;
+    return cost < (double)size[0] * (double)size[1] * (double)(wbytes + 8) / 4600.0;
+}
+
+// The path of strips (line: cross-sections of the prefixes' buffer).  False
+// as for the table.
+template <int K, typename WIN>
+bool grid_run_strips(Context &cx, hipStream_t st, const uint64_t *size, const WIN *w, size_t L, uint32_t T,
+                     uint64_t line, uint64_t *out) {
+    using Acc = SatAcc<K>;
+    SatGeom g;
+    g.gx = size[0];
+    g.gy = size[1];
+    g.gz = 1;
+    g.nb = (uint32_t)((g.gy + kSatRows - 1) / kSatRows);
+    g.nseg = (uint32_t)((g.gx + kSatCols - 1) / kSatCols);
+    g.vec_w = g.gx % 2 == 0 && (uintptr_t)w % (2 * sizeof(WIN)) == 0;
+    g.vec_s = g.gx % 2 == 0;
+    const uint64_t cells = g.gx * g.gy;
+    const uint32_t groups = (uint32_t)((g.gx + kSatRows - 1) / kSatRows);
+    const uint32_t sups = (g.nb + kStripBands - 1) / kStripBands;
+    const uint64_t col_sup = (g.nb + 1) * g.gx, row_sup = (groups + 1) * g.gy;
+    auto chunks = [](uint64_t r) { return (r + kScanChunk - 1) / kScanChunk; };
+    cx.gsat.ensure((line + (uint64_t)kStripChunks * strip_paths(L - 1)) * 8);   // the prefixes, and totals of chunks
+    cx.gcol.ensure((col_sup + (sups + 1) * g.gx) * 8);
+    cx.grow.ensure((row_sup + (g.nseg + 1) * g.gy) * 8);
+    cx.gscan.ensure(std::max(chunks(sups + 1) * g.gx, chunks(g.nseg + 1) * g.gy) * 8);
+    const uint64_t slots = (uint64_t)1 << L;
+    cx.gparts[0].ensure(slots * sizeof(GSlot));
+    cx.gparts[1].ensure(slots * sizeof(GSlot));
+    cx.gheap.ensure(slots * 4);
+    cx.gctr.ensure(kCopies * sizeof(GridSatFlags));
+    GridSatFlags *flags = (GridSatFlags *)cx.gctr.ptr;
+    Acc *col = (Acc *)cx.gcol.ptr, *row = (Acc *)cx.grow.ptr, *tmp = (Acc *)cx.gscan.ptr;
+    const StripSums<Acc> sums{col, col + col_sup, row, row + row_sup};
+    uint32_t *heap = (uint32_t *)cx.gheap.ptr;
+    if (K == 2) ck(hipMemsetAsync(flags, 0, kCopies * sizeof(GridSatFlags), st));
+    int r = cx.prof.begin(st, COUPE_HIP_K_PROLOGUE, (double)cells * (sizeof(WIN) + 16.0 / kSatRows));
+    const unsigned tile_grid = (unsigned)std::min<uint64_t>((uint64_t)sups * g.nseg, 1u << 24);
+    k_strip_sums<K, WIN><<<tile_grid, kBlock, 0, st>>>(w, g, sums, flags);
     ck(hipGetLastError());
+    // (an entry past the last one: the totals)
+    colscan<Acc>(cx, st, sums.col_sup, g.gx, sups + 1, 1, tmp);
+    colscan<Acc>(cx, st, sums.row_sup, g.gy, g.nseg + 1, 1, tmp);
     cx.prof.end(st, r);
-    if (K != 2) {
-        ck(hipStreamSynchronize(st));
-        return true;
+    r = cx.prof.begin(st, COUPE_HIP_K_DECIDE, 0.0);
+    Acc *prefix = (Acc *)cx.gsat.ptr, *totals = prefix + line;
+    int cur = 0;
+    for (size_t l = 0; l < L; l++) {
+        const GSlot *in = (const GSlot *)cx.gparts[cur].ptr;
+        GSlot *nx = (GSlot *)cx.gparts[cur ^ 1].ptr;
+        const uint64_t along = l % 2 ? g.gx : g.gy;
+        const uint32_t paths = strip_paths(l);
+        const uint32_t len = (uint32_t)((along + kBlock * kStripChunks - 1) / (kBlock * kStripChunks)) * kBlock;
+        const uint32_t nch = (uint32_t)((along + len - 1) / len);
+        auto axis = [&](auto kernel) {
+            kernel<<<paths * nch, kBlock, 0, st>>>(in, heap, (uint32_t)l, w, (uint32_t)g.gx, (uint32_t)g.gy, sums,
+                                                   prefix, totals, nch, len);
+            ck(hipGetLastError());
+        };
+        if (l % 2) axis(k_strip_axis<K, WIN, 0>);
+        else axis(k_strip_axis<K, WIN, 1>);
+        const unsigned blocks = ((1u << l) + kBlock / 64 - 1) / (kBlock / 64);
+        k_strip_median<K><<<blocks, kBlock, 0, st>>>(in, nx, heap, (uint32_t)l, g.gx, g.gy, prefix, totals, nch, len, T);
+        ck(hipGetLastError());
+        cur ^= 1;
     }
-    if (!cx.host_scratch) ck(hipHostMalloc(&cx.host_scratch, kHostScratch, hipHostMallocDefault));
-    GridSatFlags *hf = (GridSatFlags *)cx.host_scratch;
-    ck(hipMemcpyAsync(hf, flags, kCopies * sizeof(GridSatFlags), hipMemcpyDeviceToHost, st));
-    ck(hipStreamSynchronize(st));
-    double abs_sum = 0.0;
-    uint32_t bad = 0;
-    for (int c = 0; c < kCopies; c++) {
-        abs_sum += hf[c].abs_sum;
-        bad |= hf[c].bad;
-    }
-    // Every partial sum is an integer of magnitude at most sum |w|; the f64
-    // sum of the magnitudes, over at most 2^36 terms, is within a factor
-    // 1 + 2^-17 of the exact one, so this bound keeps the exact sum <= 2^53.
-    return bad == 0 && cells <= (1ull << 36) && abs_sum <= 0x1p53 * (1.0 - 0x1p-15);
+    cx.prof.end(st, r);
+    return grid_ids<K>(cx, st, 2, g, heap, L, flags, out);
 }
 
 }  // namespace
@@ -1344,18 +1778,24 @@ enum coupe_err grid_rcb(Context &cx, hipStream_t st, size_t dim, const uint64_t 
             ck(hipDeviceGetAttribute(&cx.cu_count, hipDeviceAttributeMultiprocessorCount, cx.device));
             if (cx.cu_count <= 0) cx.cu_count = 1;
         }
-        // the summed-area path up to kDenseGridLevels levels (COUPE_HIP_GRID_SAT=0: never)
+        // the summed-area path or the strips up to kDenseGridLevels levels (COUPE_HIP_GRID_SAT=0: never)
         const char *e = getenv("COUPE_HIP_GRID_SAT");
         const bool sat = iter_count <= kDenseGridLevels && !(e && e[0] == '0');
+        auto run = [&](auto kind, auto *wp) {
+            constexpr int K = decltype(kind)::value;
+            using WIN = typename std::remove_const<typename std::remove_pointer<decltype(wp)>::type>::type;
+            uint64_t line;
+            const bool strips = sat && strips_fit(dim, size, iter_count, sizeof(WIN), line);
+            if (strips && grid_run_strips<K, WIN>(cx, st, size, wp, iter_count, T, line, out)) return;
+            if (!strips && sat && grid_run_sat<K, WIN>(cx, st, dim, size, wp, iter_count, T, out)) return;
+            grid_run<K, WIN>(cx, st, dim, size, wp, iter_count, T, out);
+        };
         if (wkind == COUPE_INT) {
-            if (!sat || !grid_run_sat<0, int32_t>(cx, st, dim, size, (const int32_t *)w, iter_count, T, out))
-                grid_run<0, int32_t>(cx, st, dim, size, (const int32_t *)w, iter_count, T, out);
+            run(std::integral_constant<int, 0>{}, (const int32_t *)w);
         } else if (wkind == COUPE_INT64) {
-            if (!sat || !grid_run_sat<1, int64_t>(cx, st, dim, size, (const int64_t *)w, iter_count, T, out))
-                grid_run<1, int64_t>(cx, st, dim, size, (const int64_t *)w, iter_count, T, out);
+            run(std::integral_constant<int, 1>{}, (const int64_t *)w);
         } else {
-            if (!sat || !grid_run_sat<2, double>(cx, st, dim, size, (const double *)w, iter_count, T, out))
-                grid_run<2, double>(cx, st, dim, size, (const double *)w, iter_count, T, out);
+            run(std::integral_constant<int, 2>{}, (const double *)w);
         }
         cx.prof.collect();
     } catch (const HipFailure &f) {
