@@ -343,7 +343,7 @@ k_grid_fill(const GridPart *__restrict__ parts, const uint32_t *n_parts, const u
 //   k_sat_linescan    inclusive scans along rows of the row carries
 //   k_sat_tiles       per tile: the table from the weights and the carries
 //   k_sat_zsum/zapply 3D: the scan along z, in bands of 16 planes
-//   k_grid_level      one wavefront per subgrid of a level: weighted_median
+//   k_grid_level      one wavefront per subgrid, five levels a launch: weighted_median
 //                     on lookups, the split into a dense heap, the children
 //   k_grid_fill_heap  each cell walks the heap to its part id (part_of)
 // ---------------------------------------------------------------------------
@@ -916,58 +916,70 @@ __device__ inline void median_rounds(uint64_t m, uint64_t total, uint32_t thread
     }
 }
 
-// A subgrid without cells: nothing below reaches a cell.
-__device__ inline bool slot_empty(const GSlot &P, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint64_t n,
-                                  uint64_t h, bool writes) {
+// A subgrid without cells: nothing below reaches a cell.  two: its halves
+// (slots 2h and 2h + 1 of the next level); n, h: the level's subgrids, this one.
+__device__ inline bool slot_empty(const GSlot &P, GSlot *two, uint32_t *__restrict__ heap, uint64_t n, uint64_t h,
+                                  bool writes) {
     if (P.size[0] != 0 && P.size[1] != 0 && P.size[2] != 0) return false;
     if (writes) {
-        out[2 * h] = P;
-        out[2 * h + 1] = P;
+        two[0] = P;
+        two[1] = P;
         heap[n - 1 + h] = 0;
     }
     return true;
 }
-// The split of subgrid h of the level's n into the heap and its two halves
-// into slots 2h and 2h + 1 of the next level.
+// The split of subgrid h into the heap, and its two halves.
 template <int K>
-__device__ inline void slot_split(const GSlot &P, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint64_t n,
-                                  uint64_t h, int coord, uint64_t total, uint64_t pos, uint64_t left) {
+__device__ inline void slot_split(const GSlot &P, GSlot *two, uint32_t *__restrict__ heap, uint64_t n, uint64_t h,
+                                  int coord, uint64_t total, uint64_t pos, uint64_t left) {
     GSlot A = P, B = P;
     A.size[coord] = (uint32_t)pos;
     A.sum = left;
     B.off[coord] = P.off[coord] + (uint32_t)pos;
     B.size[coord] = P.size[coord] - (uint32_t)pos;
     B.sum = GW<K>::sub(total, left);
-    out[2 * h] = A;
-    out[2 * h + 1] = B;
+    two[0] = A;
+    two[1] = B;
     heap[n - 1 + h] = P.off[coord] + (uint32_t)pos;
 }
 
-// One wavefront per subgrid h of level l (2^l of them).
+// Levels l0 .. l0 + nl - 1 of the subgrids of level l0, a workgroup of
+// 2^(nl - 1) wavefronts each: a wavefront per subgrid of a level, the slots
+// between the levels in LDS.  A level is a chain of a few lookups, so a launch
+// of its own costs as much as its rounds (1000 x 700 cells, 10 levels: 69 us
+// one by one, 41 in two launches).
+constexpr uint32_t kLevelRun = 5;   // most levels: 16 wavefronts
 template <int K, int D>
-__global__ void __launch_bounds__(kBlock)
-k_grid_level(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint32_t l,
-             const SatAcc<K> *__restrict__ S, uint64_t gx, uint64_t gy, uint64_t gz, uint32_t threads) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t n = (uint64_t)1 << l;
-    const uint64_t h = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (h >= n) return;
-    const int coord = (int)((1 + l) % D);
-    GSlot P;   // level 0: the whole grid
-    if (l == 0) P = GSlot{{0, 0, 0}, {(uint32_t)gx, (uint32_t)gy, (uint32_t)gz}, 0};
-    else P = in[h];
-    if (slot_empty(P, out, heap, n, h, lane == 0)) return;
-    uint64_t lo[3], hi[3];
-    for (int k = 0; k < 3; k++) {
-        lo[k] = P.off[k];
-        hi[k] = (uint64_t)P.off[k] + P.size[k];
+__global__ void __launch_bounds__(64 << (kLevelRun - 1))
+k_grid_level(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *__restrict__ heap, uint32_t l0,
+             uint32_t nl, const SatAcc<K> *__restrict__ S, uint64_t gx, uint64_t gy, uint64_t gz, uint32_t threads) {
+    __shared__ GSlot slots[2][1u << kLevelRun];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x == 0) {   // level 0: the whole grid
+        if (l0 == 0) slots[0][0] = GSlot{{0, 0, 0}, {(uint32_t)gx, (uint32_t)gy, (uint32_t)gz}, 0};
+        else slots[0][0] = in[blockIdx.x];
     }
-    const uint64_t total = l == 0 ? sat_carrier<K>(sat_box<D>(S, gx, gy, lo, hi)) : P.sum;
-    const SatAcc<K> f0 = sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord]);
-    uint64_t pos = 0, left = 0;
-    median_rounds<K>(P.size[coord], total, threads, pos, left,
-                     [&](uint64_t p) { return sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord] + p) - f0; });
-    if (lane == 0) slot_split<K>(P, out, heap, n, h, coord, total, pos, left);
+    for (uint32_t k = 0; k < nl; k++) {
+        __syncthreads();
+        if (wave >> k) continue;
+        const uint32_t l = l0 + k;
+        const uint64_t n = (uint64_t)1 << l, h = ((uint64_t)blockIdx.x << k) + wave;
+        const int coord = (int)((1 + l) % D);
+        const GSlot P = slots[k & 1][wave];
+        GSlot *two = k + 1 < nl ? &slots[(k + 1) & 1][2 * wave] : &out[2 * h];
+        if (slot_empty(P, two, heap, n, h, lane == 0)) continue;
+        uint64_t lo[3], hi[3];
+        for (int a = 0; a < 3; a++) {
+            lo[a] = P.off[a];
+            hi[a] = (uint64_t)P.off[a] + P.size[a];
+        }
+        const uint64_t total = l == 0 ? sat_carrier<K>(sat_box<D>(S, gx, gy, lo, hi)) : P.sum;
+        const SatAcc<K> f0 = sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord]);
+        uint64_t pos = 0, left = 0;
+        median_rounds<K>(P.size[coord], total, threads, pos, left,
+                         [&](uint64_t p) { return sat_face<D>(S, gx, gy, lo, hi, coord, lo[coord] + p) - f0; });
+        if (lane == 0) slot_split<K>(P, two, heap, n, h, coord, total, pos, left);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1273,7 +1285,7 @@ k_strip_median(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *
     if (h >= n) return;
     const int coord = (int)((1 + l) % 2);
     const GSlot P = strip_slot(in, h, l, gx, gy);
-    if (slot_empty(P, out, heap, n, h, lane == 0)) return;
+    if (slot_empty(P, &out[2 * h], heap, n, h, lane == 0)) return;
     const uint32_t path = strip_path((uint32_t)h, l);
     const Acc t = lane < chunks ? totals[(uint64_t)path * chunks + lane] : (Acc)0;
     before[wave][lane] = wave_scan(t) - t;   // (a wavefront's own row: in order)
@@ -1285,7 +1297,7 @@ k_strip_median(const GSlot *__restrict__ in, GSlot *__restrict__ out, uint32_t *
     const uint64_t total = l == 0 ? sat_carrier<K>(upto(m)) : P.sum;
     uint64_t pos = 0, left = 0;
     median_rounds<K>(m, total, threads, pos, left, [&](uint64_t q) { return upto(off + q) - f0; });
-    if (lane == 0) slot_split<K>(P, out, heap, n, h, coord, total, pos, left);
+    if (lane == 0) slot_split<K>(P, &out[2 * h], heap, n, h, coord, total, pos, left);
 }
 
 // part_of (rcb.rs:21-42) from the heap of splits: at level l the cell goes
@@ -1648,14 +1660,15 @@ bool grid_run_sat(Context &cx, hipStream_t st, size_t dim, const uint64_t *size,
 
     int cur = 0;
     r = cx.prof.begin(st, COUPE_HIP_K_DECIDE, 0.0);
-    for (size_t l = 0; l < L; l++) {
+    for (size_t l = 0; l < L; l += kLevelRun) {
         const GSlot *in = (const GSlot *)cx.gparts[cur].ptr;
         GSlot *nx = (GSlot *)cx.gparts[cur ^ 1].ptr;
-        const unsigned blocks = (unsigned)((((uint64_t)1 << l) + kBlock / 64 - 1) / (kBlock / 64));
-        if (dim == 2)
-            k_grid_level<K, 2><<<blocks, kBlock, 0, st>>>(in, nx, heap, (uint32_t)l, S, g.gx, g.gy, g.gz, T);
-        else
-            k_grid_level<K, 3><<<blocks, kBlock, 0, st>>>(in, nx, heap, (uint32_t)l, S, g.gx, g.gy, g.gz, T);
+        const uint32_t nl = (uint32_t)std::min<size_t>(kLevelRun, L - l);
+        auto launch = [&](auto kernel) {
+            kernel<<<1u << l, 64u << (nl - 1), 0, st>>>(in, nx, heap, (uint32_t)l, nl, S, g.gx, g.gy, g.gz, T);
+        };
+        if (dim == 2) launch(k_grid_level<K, 2>);
+        else launch(k_grid_level<K, 3>);
         ck(hipGetLastError());
         cur ^= 1;
     }
@@ -1669,10 +1682,13 @@ uint32_t strip_paths(size_t l) { return 1u << (l % 2 ? (l + 1) / 2 : l / 2); }
 
 // Whether a 2D call goes by strips instead of the table.  They save the
 // table's write and the second read of the weights (8 + 8 bytes a cell at
-// about 4.6 TB/s); a cross-section of a level costs about 110 bytes along x
-// (two entries, 8 to 16 weights, the prefix) and, in whole lines, 400 along
-// y, at about 2 TB/s, and a level a few microseconds more than the wavefronts
-// on the table take.  (COUPE_HIP_GRID_STRIPS=1, 0: always, never.)
+// about 4.6 TB/s); a level costs about 8 us more than the wavefronts on the
+// table take, and 30 ps per cross-section along x (two entries, 8 to 16
+// weights, the prefix), 100 along y (each edge's weights a line of their own).
+// Fitted over 12 shapes of 10^6 to 10^8 cells and 4 to 16 levels: where it
+// says strips the table took 1.02 to 1.9 times as long, where it says the table
+// the strips 0.78 to 3.
+// (COUPE_HIP_GRID_STRIPS=1, 0: always, never.)
 bool strips_fit(size_t dim, const uint64_t *size, size_t L, size_t wbytes, uint64_t &line) {
     const char *e = getenv("COUPE_HIP_GRID_STRIPS");
     line = 1;
@@ -1681,7 +1697,7 @@ bool strips_fit(size_t dim, const uint64_t *size, size_t L, size_t wbytes, uint6
     for (size_t l = 0; l < L; l++) {
         const bool y = l % 2 == 0;
         const uint64_t along = y ? size[1] : size[0], paths = strip_paths(l);
-        cost += (double)along * (double)paths * (y ? 0.2 : 0.055) + 5000.0;
+        cost += (double)along * (double)paths * (y ? 0.1 : 0.03) + 8000.0;
         line = std::max(line, along * paths);
     }
     if (e && e[0] == '1') return true;
