@@ -120,6 +120,10 @@ struct GraphEntry {
 
 constexpr size_t kGraphs = 8;           // graphs a context keeps
 
+// The paths that leave the points in place (rcb_mid.h, rcb_front.h).
+constexpr uint64_t kMidCells = 1ull << 21;        // cells of a call, at most
+constexpr uint64_t kMidCopied = 1ull << 16;       // cells kept in one copy per XCD up to here
+
 struct Context {
     int device = 0;
     std::mutex lock;                 // one call at a time per context
@@ -149,6 +153,7 @@ struct Context {
     uint32_t copy_parts = 256;       // levels of at most this many parts flush into per-XCD copies
     uint32_t search_chunk = 2;       // consecutive tiles a workgroup takes at a time in the search passes
     bool small = true;               // problems of few points take one workgroup each (rcb_small.h)
+    bool in_place = true;            // false: calls that leave the points in place are not taken (a bound on bytes)
     bool mid = true;                 // try the tree of box midpoints first (rcb_mid.h)
     bool front = true;               // search one instance's levels without moving its points (rcb_front.h)
     double move_nt_bytes = 2.5e9;    // moves and id descents of more bytes than this go non-temporal

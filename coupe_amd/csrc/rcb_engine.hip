@@ -1078,14 +1078,12 @@ static void prologue(Context &cx, hipStream_t st, const BatchPlan &B, const doub
 // ---------------------------------------------------------------------------
 // The midpoint tree (rcb_mid.h).
 // ---------------------------------------------------------------------------
-constexpr uint64_t kMidCells = 1ull << 21;        // cells of a call, at most
-constexpr uint64_t kMidCopied = 1ull << 16;       // cells kept in one copy per XCD up to here
 
 // Whether a call takes it: its levels fit the cells, no switch asks for the
 // general path's passes or its graph, its buffers may grow, and the last call
 // of the shape did not end on the general path.
 static bool in_place_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
-    if (spec_passes <= 0 || cx.capturing || cx.graphs || t_arena) return false;
+    if (!cx.in_place || spec_passes <= 0 || cx.capturing || cx.graphs || t_arena) return false;
     if (!B.dense || B.max_levels == 0 || B.max_levels > kMidLevels) return false;
     return B.heap_total + B.inst.size() <= kMidCells;
 }

@@ -105,6 +105,19 @@ uint64_t batch_bytes(uint64_t n, uint64_t dim, uint64_t wsize, uint64_t parts, u
     return b + b / 8;
 }
 
+// What the paths that leave the points in place hold besides (points gathered,
+// cells and slots; the tables of at most kMidCells cells; the frontier's
+// bins).  A batch that fits the budget only without runs on the general path.
+uint64_t in_place_bytes(uint64_t n, uint64_t dim, uint64_t wsize, uint64_t requests, uint64_t levels) {
+    if (levels > 12) return 0;
+    const uint64_t record = dim == 3 && wsize == 8 ? 24 : 16;
+    const uint64_t cells = std::min<uint64_t>(coupe_hip::kMidCells, requests << levels);
+    uint64_t b = n * (2 + 2 + record);
+    b += cells * ((cells <= coupe_hip::kMidCopied ? 8 : 1) * 12 + 4 + 64 + 4 + 3 * 4 + 4);   // counts, map, open nodes, cursors, lists, splits
+    if (requests == 1 && n > 16384) b += 256ull * (5376 * 16 + 1024 * 4) + (1ull << 20);   // the frontier's bins
+    return b + b / 8;
+}
+
 uint64_t parts_bound(uint64_t n, uint64_t levels) {
     uint64_t p = 1;
     for (uint64_t l = 1; l < levels && p < n; l++) p = std::min<uint64_t>(2 * p, n);
@@ -291,8 +304,11 @@ bool pick_batch(coupe_hip_server *S, Worker *W, std::vector<Req *> &batch) {
     }
     // admission: what W will hold for this batch (at least what it holds now,
     // its buffers only grow), against what the others and the meshes hold now
-    const uint64_t need = batch_bytes(pts, dim, wsize, parts, levels, !first->mesh);
+    uint64_t need = batch_bytes(pts, dim, wsize, parts, levels, !first->mesh);
     const uint64_t others = S->held() - W->held;
+    const uint64_t more = in_place_bytes(pts, dim, wsize, take.size() + 1, levels);
+    W->cx.in_place = others + std::max(need + more, W->held) <= S->cfg.memory_budget;
+    if (W->cx.in_place) need += more;
     if (others + std::max(need, W->held) > S->cfg.memory_budget) {
         S->memory_wanted = true;
         return false;
