@@ -1186,11 +1186,17 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
         // 16-bit weights share a word with the count (unless a workgroup's share is large)
         const bool one_word = packable<WL, Acc>() && n / (uint64_t)cx.cu_count < (1ull << 23);
         const uint32_t lds = max_cells * (one_word ? 8u : 12u);
-        const unsigned grid = grid_of(k_mid_count<D, WL, Acc>, nt, lds);
-        timed(cx, st, COUPE_HIP_K_HIST, (4.0 * D + sizeof(WL) + 2.0) * (double)n, [&] {
-            k_mid_count<D, WL, Acc><<<grid, kBlock, lds, st>>>(tiles, nt, insts, red, n_inst, c[0], c[1], c[2], w,
-                                                              w_src, code, gcnt, gw, cells, copies);
-        });
+        auto launch = [&](auto kernel, int tpb) {
+            const unsigned grid = grid_of(kernel, nt, lds);
+            timed(cx, st, COUPE_HIP_K_HIST, (4.0 * D + sizeof(WL) + 2.0) * (double)n, [&] {
+                kernel<<<grid, tpb, lds, st>>>(tiles, nt, insts, red, n_inst, c[0], c[1], c[2], w, w_src, code, gcnt,
+                                               gw, cells, copies);
+            });
+        };
+        // the cells' LDS bounds the workgroups of a CU: more wavefronts in each
+        // (2^27 points, 4096 cells: 569 us with 256 threads, 553 with 512)
+        if (lds > 16384) launch(k_mid_count<D, 512, WL, Acc>, 512);
+        else launch(k_mid_count<D, 256, WL, Acc>, 256);
     }
     // An open node past the register classes is searched by one workgroup from
     // memory, about 0.55 ns per point and level; the general path takes about

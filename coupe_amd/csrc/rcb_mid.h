@@ -96,7 +96,7 @@ __device__ __forceinline__ void mid_tables(MidTables &T, uint32_t levels) {
     constexpr float nan = __builtin_nanf("");
     for (int a = 0; a < D; a++) {
         const uint32_t la = mid_axis_levels(levels, a, D), n = 1u << la;
-        for (uint32_t r = threadIdx.x; r < n; r += kBlock) {
+        for (uint32_t r = threadIdx.x; r < n; r += blockDim.x) {
             uint32_t bits = 0;
             for (uint32_t j = 0; j < la; j++)
                 bits |= ((r >> (la - 1 - j)) & 1u) << (levels - 1 - (uint32_t)a - j * D);
@@ -123,16 +123,21 @@ __device__ __forceinline__ uint32_t mid_rank(const float4 *rank, int n, float x,
     return __builtin_bit_cast(uint32_t, t.z);
 }
 
+// Runs of a wavefront's cells up to which they are added run by run (a random
+// cloud has about 60; 2^27 points in mesh order: 553 us without, 505 with).
+constexpr int kMidRuns = 14;
+
 // w: the stored weights (w_src 0) or the caller's (w_src 1, 64-bit weights
 // are not stored on this path).  cells: per copy (copies of them), the count
 // and weight of every instance's cells.  code: each point's cell.
-template <int D, typename WL, typename Acc>
-__global__ void __launch_bounds__(kBlock)
+template <int D, int TPB, typename WL, typename Acc>
+__global__ void __launch_bounds__(TPB)
 k_mid_count(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__restrict__ insts,
             const InstReduce *__restrict__ red, uint32_t n_inst, const float *__restrict__ c0,
             const float *__restrict__ c1, const float *__restrict__ c2, const WL *__restrict__ w, int w_src,
             uint16_t *__restrict__ code, uint32_t *__restrict__ gcnt, Acc *__restrict__ gw, uint64_t cells,
             uint32_t copies) {
+    constexpr int IT = kTile / TPB;
     __shared__ MidTables T;
     extern __shared__ __align__(16) char mid_lds[];
     uint32_t t0, t1;
@@ -143,13 +148,13 @@ k_mid_count(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__
     const bool packed = packable<WL, Acc>() && (uint64_t)(t1 - t0) * kTile < (1ull << 24);
     Acc *sw = (Acc *)mid_lds;
     uint32_t *sc = nullptr;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     uint32_t cur = 0xffffffffu, levels = 0, n_cells = 0;
     uint64_t gbase = 0, wbase = 0;
     float lo[D], scale[D];
     int ranks[D];
     auto flush = [&]() {
-        for (uint32_t c = tid; c < n_cells; c += kBlock) {
+        for (uint32_t c = tid; c < n_cells; c += TPB) {
             uint32_t cnt;
             Acc sum = sw[c];
             if (packed) {
@@ -183,7 +188,7 @@ k_mid_count(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__
             if (tid < D) mid_box<D>(red, n_inst, cur, tid, T.lo[tid], T.hi[tid]);
             __syncthreads();
             mid_tables<D>(T, levels);
-            for (uint32_t c = tid; c < n_cells; c += kBlock) {
+            for (uint32_t c = tid; c < n_cells; c += TPB) {
                 sw[c] = (Acc)0;
                 if (!packed) sc[c] = 0;
             }
@@ -196,22 +201,44 @@ k_mid_count(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__
             __syncthreads();
         }
         // every load of the tile issued first (clamped, unconditional)
-        float x[kItems][D];
-        WL wk[kItems];
+        float x[IT][D];
+        WL wk[IT];
 #pragma unroll
-        for (int k = 0; k < kItems; k++) {
-            const uint64_t i = U.begin + min((uint32_t)(k * kBlock + tid), U.count - 1u);
+        for (int k = 0; k < IT; k++) {
+            const uint64_t i = U.begin + min((uint32_t)(k * TPB + tid), U.count - 1u);
             x[k][0] = c0[i];
             x[k][1] = c1[i];
             if constexpr (D == 3) x[k][2] = c2[i];
             wk[k] = w[wbase + i];
         }
 #pragma unroll
-        for (int k = 0; k < kItems; k++) {
+        for (int k = 0; k < IT; k++) {
             uint32_t c = 0;
 #pragma unroll
             for (int a = 0; a < D; a++) c |= mid_rank(T.rank[a], ranks[a], x[k][a], lo[a], scale[a]);
-            const uint32_t p = (uint32_t)(k * kBlock + tid);
+            const uint32_t p = (uint32_t)(k * TPB + tid);
+            if constexpr (packable<WL, Acc>()) {
+                // Points in a mesh's order share cells with their neighbours, and
+                // atomics of a wavefront on one address are done one by one: where
+                // the lanes' cells form few runs (within rows of 16 lanes), a run
+                // adds its prefix at its end and takes off the prefix before it at
+                // its start (modulo 2^64: exact)
+                const uint64_t heads = __ballot(c != dpp_row<0x111, true>(0u, c) || (tid & 15) == 0);
+                if (packed && __popcll(heads) <= kMidRuns && (uint32_t)(k * TPB) + (tid | 63) < U.count) {
+                    uint32_t s = (uint32_t)wk[k];
+                    s += dpp_row<0x111, true>(0u, s);
+                    s += dpp_row<0x112, true>(0u, s);
+                    s += dpp_row<0x114, true>(0u, s);
+                    s += dpp_row<0x118, true>(0u, s);
+                    code[U.begin + p] = (uint16_t)c;
+                    const uint64_t tails = heads >> 1 | 1ull << 63;
+                    const unsigned long long upto = ((unsigned long long)((tid & 15) + 1) << kPackShift) + s;
+                    const unsigned long long own = (1ull << kPackShift) + (uint32_t)wk[k];
+                    if (tails >> lane & 1) atomicAdd((unsigned long long *)&sw[c], upto);
+                    if ((heads >> lane & 1) && (tid & 15) != 0) atomicAdd((unsigned long long *)&sw[c], own - upto);
+                    continue;
+                }
+            }
             if (p >= U.count) continue;
             code[U.begin + p] = (uint16_t)c;
             if (packed) {
@@ -547,45 +574,67 @@ template <int D, int TPB, typename WL, typename Acc>
 __device__ __forceinline__ bool mid_memory(uint32_t count, const SubRoot &R, Acc sum,
                                            const MidPoint<D, WL> *__restrict__ pts, uint16_t *__restrict__ slots,
                                            uint32_t *ctr, const MidSplits &out) {
-    constexpr int B = kAhead;
+    // G points of a thread in flight: a CU has this workgroup alone (2^27 jittered
+    // points, nodes of up to 131072: 356 us with B in flight, 278 with G)
+    constexpr int B = kAhead, G = 16;
     const uint32_t tid = threadIdx.x;
     SubTree<Acc, TPB> T(sub_slots(R.levels));
     bool first = true;   // every point in slot 0: not read
     return sub_levels<D, TPB, Acc>(
         T, R, count, sum, ctr,
         [&](int nb, int a) {
-            for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
-                uint32_t s[B];
-                float xa[B];
-                Acc wk[B];
-                bool valid[B];
+            auto points = [&](uint32_t i0, auto many) {
+                constexpr int M = decltype(many)::value;
+                uint16_t sg[M];
+                float xg[M];
+                WL wg[M];
 #pragma unroll
-                for (int j = 0; j < B; j++) {
-                    const uint32_t i = i0 + (uint32_t)(j * TPB) + tid, p = i < count ? i : count - 1;
-                    valid[j] = i < count;
-                    xa[j] = pts[p].x[a];
-                    wk[j] = AccOps<Acc>::of(pts[p].w);
-                    s[j] = first ? 0u : (uint32_t)slots[p];
+                for (int g = 0; g < M; g++) {
+                    const uint32_t i = i0 + (uint32_t)(g * TPB) + tid, p = i < count ? i : count - 1;
+                    xg[g] = pts[p].x[a];
+                    wg[g] = pts[p].w;
+                    sg[g] = first ? (uint16_t)0 : slots[p];
                 }
-                sub_bin<B>(T, s, [&](int j, uint32_t) { return xa[j]; }, wk, valid, nb, R.packed);
-            }
+#pragma unroll
+                for (int g = 0; g < M; g += B) {
+                    uint32_t s[B];
+                    float xa[B];
+                    Acc wk[B];
+                    bool valid[B];
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        valid[j] = i0 + (uint32_t)((g + j) * TPB) + tid < count;
+                        xa[j] = xg[g + j];
+                        wk[j] = AccOps<Acc>::of(wg[g + j]);
+                        s[j] = sg[g + j];
+                    }
+                    sub_bin<B>(T, s, [&](int j, uint32_t) { return xa[j]; }, wk, valid, nb, R.packed);
+                }
+            };
+            uint32_t i0 = 0;
+            for (; i0 + TPB * G <= count; i0 += TPB * G) points(i0, std::integral_constant<int, G>{});
+            for (; i0 < count; i0 += TPB * B) points(i0, std::integral_constant<int, B>{});
         },
         [&](int a) {
-            for (uint32_t i0 = 0; i0 < count; i0 += TPB * B) {
-                uint32_t s[B];
-                float xa[B];
+            auto points = [&](uint32_t i0, auto many) {
+                constexpr int M = decltype(many)::value;
+                uint32_t s[M];
+                float xa[M];
 #pragma unroll
-                for (int j = 0; j < B; j++) {   // (each thread its own points: no other touches their slots)
+                for (int j = 0; j < M; j++) {   // (each thread its own points: no other touches their slots)
                     const uint32_t i = i0 + (uint32_t)(j * TPB) + tid, p = i < count ? i : count - 1;
                     xa[j] = pts[p].x[a];
                     s[j] = first ? 0u : (uint32_t)slots[p];
                 }
 #pragma unroll
-                for (int j = 0; j < B; j++) {
+                for (int j = 0; j < M; j++) {
                     const uint32_t i = i0 + (uint32_t)(j * TPB) + tid;
                     if (i < count) slots[i] = (uint16_t)(2 * s[j] + (xa[j] >= T.at(s[j]).win.x ? 1u : 0u));
                 }
-            }
+            };
+            uint32_t i0 = 0;
+            for (; i0 + TPB * G <= count; i0 += TPB * G) points(i0, std::integral_constant<int, G>{});
+            for (; i0 < count; i0 += TPB * B) points(i0, std::integral_constant<int, B>{});
             first = false;
         },
         out);
