@@ -69,9 +69,8 @@ def algo_bytes_per_point(dim: int, levels: int) -> int:
     return (12 * dim + 20) + 12 * levels + (levels - 1) * (8 * dim + 24) + 12
 
 
-TRAFFIC_PROFILES = {("jgrid512", "partition"): "profiles/rcb_jgrid512_hbm_traffic.md",
-                    ("gauss3d", "hist"): "profiles/rcb_gauss3d_hbm_traffic.md",
-                    ("gauss3d", "partition"): "profiles/rcb_gauss3d_hbm_traffic.md"}
+TRAFFIC_PROFILES = {("jgrid512", "prologue"): "profiles/rcb_jgrid512_hbm_traffic.md",
+                    ("gauss3d", "hist"): "profiles/rcb_gauss3d_hbm_traffic.md"}
 
 
 def measured_traffic(workload: str, kernel: str):
@@ -271,9 +270,9 @@ def main():
         "unit": "GB/s",
         "frac": round(dk["GBps"] / HBM_PEAK_GBS, 4),
         "traffic": measured_traffic(args.workload, dominant),
-        "basis": "engine: the bytes the move must read and write in this layout (f32 coordinates, 16-bit "
-                 "weights, no index stream; two levels per launch), checked against FETCH_SIZE/WRITE_SIZE "
-                 "(traffic); frac_s8d prices the same launches at the survey's (8D+24) B/pt per level",
+        "basis": "engine: the bytes the kernel must read and write in this layout (f32 coordinates, 16-bit "
+                 "weights, no index stream), checked against FETCH_SIZE/WRITE_SIZE where traffic is given; "
+                 "frac_s8d prices moves at (8D+24) B/pt per level",
         "frac_engine": round(dk["GBps"] / HBM_PEAK_GBS, 4),
         "achieved_s8d": round(s8d_gbs, 1) if s8d_gbs else None,
         "frac_s8d": round(s8d_gbs / HBM_PEAK_GBS, 4) if s8d_gbs else None,
