@@ -1381,9 +1381,14 @@ template <int D, typename WIN>
 static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchPlan &B, const double *pts,
                       const WIN *win, int wkind, int spec_passes) {
     const uint64_t n = B.span;   // positions of the working arrays
-    // Coordinate slots: 0 (prologue output, input order), 1 and 2 (levels).
-    for (int b = cx.slot0[0] ? 1 : 0; b < 3; b++)
-        for (int k = 0; k < D; k++) cx.cx[b][k].ensure(std::max<uint64_t>(n, 1) * sizeof(float));
+    // Coordinate slots: 0 (prologue output, input order), 1 and 2 (levels of
+    // the general path: a call in place has no use for them unless it ends there).
+    const bool in_place_first = mid_fits(cx, B, spec_passes) || front_fits(cx, B, spec_passes);
+    auto slots = [&](int from, int to) {
+        for (int b = from; b < to; b++)
+            for (int k = 0; k < D; k++) cx.cx[b][k].ensure(std::max<uint64_t>(n, 1) * sizeof(float));
+    };
+    slots(cx.slot0[0] ? 1 : 0, in_place_first ? 1 : 3);
     cx.w[0].ensure(std::max<uint64_t>(n, 1) * sizeof(int32_t));
     cx.ired.ensure(kCopies * std::max<size_t>(B.inst.size(), 1) * sizeof(InstReduce));
     cx.counters.ensure(sizeof(Counters));
@@ -1403,6 +1408,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
     auto run_mode = [&](int mode) {
         cx.stats.weight_mode = mode == 3 ? 1 : 0;
         cx.stats.weight_bytes = weight_bytes(mode);
+        slots(1, 3);
         cx.w[1].ensure(std::max<uint64_t>(n, 1) * weight_bytes(mode));
         if (mode == 0)
             return run_levels<D, uint16_t, uint64_t>(cx, st, B, wrap32, d_out, (uint16_t *)cx.w16.ptr, spec_passes);
@@ -1435,7 +1441,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
         // buffers for the expected mode before anything is queued (a buffer
         // that grows is freed and allocated again)
         cx.w[0].ensure(std::max<uint64_t>(n, 1) * (hint >= 2 ? 8u : 4u));
-        if (hint >= 0) cx.w[1].ensure(std::max<uint64_t>(n, 1) * weight_bytes(hint));
+        if (hint >= 0 && !in_place_first) cx.w[1].ensure(std::max<uint64_t>(n, 1) * weight_bytes(hint));
         prologue<D, WIN>(cx, st, B, pts, win, hp, hint < 0, hint);
         if (hint < 0) {
             mode = best_mode(combine_flags(hp));
