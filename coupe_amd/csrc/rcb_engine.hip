@@ -1005,6 +1005,14 @@ static bool mode_held(Context &cx) {
     return (mode == 3) == (best == 3) && mode >= best;
 }
 
+// The weight mode expected of a call: its shape's last one, or the context's
+// for a shape not seen (-1: not known, the call waits for its flags).
+// Integers never need f64 sums: after a call with real weights they start anew.
+static int expected_mode(const Context &cx, const Hints *seen, int wkind) {
+    const int hint = seen ? seen->weight_hint : cx.weight_hint;
+    return hint == 3 && wkind != COUPE_DOUBLE ? -1 : hint;
+}
+
 template <int D, typename WIN>
 static void prologue(Context &cx, hipStream_t st, const BatchPlan &B, const double *pts, const WIN *win,
                      Prologue *h, bool wait, int hint) {
@@ -1414,20 +1422,22 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
             return run_levels<D, uint16_t, uint64_t>(cx, st, B, wrap32, d_out, (uint16_t *)cx.w16.ptr, spec_passes);
         if (mode == 1)
             return run_levels<D, int32_t, uint64_t>(cx, st, B, wrap32, d_out, (int32_t *)cx.w[0].ptr, spec_passes);
-        if (mode == 2) {
-            timed(cx, st, COUPE_HIP_K_OTHER, 0.0, [&] {
-                k_store_weights<WIN, int64_t><<<tgrid, kBlock, 0, st>>>(
-                    (const Tile *)cx.tiles0.ptr, (uint32_t)B.tiles0, (const Instance *)cx.instances.ptr, win,
-                    (int64_t *)cx.w[0].ptr);
-            });
-            return run_levels<D, int64_t, uint64_t>(cx, st, B, wrap32, d_out, (int64_t *)cx.w[0].ptr, spec_passes);
+        if constexpr (std::is_same<WIN, double>::value) {   // (integers never need f64 sums)
+            if (mode == 3) {
+                timed(cx, st, COUPE_HIP_K_OTHER, 0.0, [&] {
+                    k_store_weights<WIN, double><<<tgrid, kBlock, 0, st>>>(
+                        (const Tile *)cx.tiles0.ptr, (uint32_t)B.tiles0, (const Instance *)cx.instances.ptr, win,
+                        (double *)cx.w[0].ptr);
+                });
+                return run_levels<D, double, double>(cx, st, B, 0, d_out, (double *)cx.w[0].ptr, spec_passes);
+            }
         }
         timed(cx, st, COUPE_HIP_K_OTHER, 0.0, [&] {
-            k_store_weights<WIN, double><<<tgrid, kBlock, 0, st>>>(
+            k_store_weights<WIN, int64_t><<<tgrid, kBlock, 0, st>>>(
                 (const Tile *)cx.tiles0.ptr, (uint32_t)B.tiles0, (const Instance *)cx.instances.ptr, win,
-                (double *)cx.w[0].ptr);
+                (int64_t *)cx.w[0].ptr);
         });
-        return run_levels<D, double, double>(cx, st, B, 0, d_out, (double *)cx.w[0].ptr, spec_passes);
+        return run_levels<D, int64_t, uint64_t>(cx, st, B, wrap32, d_out, (int64_t *)cx.w[0].ptr, spec_passes);
     };
     // The mode of this context's last call is taken as this call's: the
     // prologue's flags are then read with the call's last counters, without a
@@ -1435,8 +1445,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
     // runs again in its own.  A new context waits for the flags first.
     Prologue *hp = prologue_early(cx);
     for (;;) {
-        const Hints *seen = cx.hints_for(B.shape);
-        const int hint = seen ? seen->weight_hint : cx.weight_hint;
+        const int hint = expected_mode(cx, cx.hints_for(B.shape), wkind);
         int mode = hint;
         // buffers for the expected mode before anything is queued (a buffer
         // that grows is freed and allocated again)
@@ -1447,6 +1456,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
             mode = best_mode(combine_flags(hp));
             if (mode >= 2) cx.w[0].ensure(std::max<uint64_t>(n, 1) * 8u);
         }
+        cx.pending.shape = B.shape;
         cx.pending.mode = mode;
         cx.pending.wkind = wkind;
         // the midpoint tree, then the frontier, then the general path
@@ -1781,7 +1791,7 @@ static enum coupe_err rcb_general(Context &cx, hipStream_t st, uint64_t *d_out, 
         // 2 not run that way (or its data needs another weight mode).
         int how = 2;
         if (cx.graphs && !rot && !cx.prof.enabled && !t_arena && spec > 0 && cx.bins_clean && seen &&
-            seen->weight_hint >= 0 && seen->level_passes.size() == B.max_levels)
+            expected_mode(cx, seen, wkind) >= 0 && seen->level_passes.size() == B.max_levels)
             how = run_captured(cx, st, B, dim, wkind, d_out, d_points, d_weights, spec, run);
         if (how == 3) how = 2;   // first sight of the graph key: eager
         const bool unfinished = how == 1 || (how == 2 && run(spec, st));
