@@ -144,7 +144,7 @@ k_front_hist(int r, const FrontRound *__restrict__ rounds, const FrontNode *__re
     for (uint32_t s = tid; s < H.nodes; s += TPB) {
         const FrontNode &N = nodes[s];
         const uint32_t f = N.flags | (nb <= 4 ? (uint32_t)kSubMin : 0u) | s | N.axis << kFrontAxis;
-        T.at(s).win = make_float4(N.lo, N.hi, __builtin_amdgcn_rcpf(N.hi - N.lo), __builtin_bit_cast(float, f));
+        T.at(s).win = make_float4(N.lo, N.hi, window_scale(N.lo, N.hi), __builtin_bit_cast(float, f));
         T.at(s).nhi = 0xffffffffu;
     }
     for (uint32_t s = tid; s < before; s += TPB) T.route(s) = routes[s];

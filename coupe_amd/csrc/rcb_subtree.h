@@ -35,10 +35,20 @@ enum : uint32_t { kCandCount = (1u << 29) - 1, kCandLeft = 1u << 29, kCandStop =
 // when compiling, so that the accesses need no base registers.
 extern __shared__ __align__(16) char sub_lds_base[];
 
+// 1 / (hi - lo) of a window, for sub_bin's estimate; NaN (no estimate: every
+// point walks the midpoints) where an end is 2^124 or more.  Below, every sum
+// of two values of the window is finite, so the midpoints are evenly spaced,
+// and the reciprocal is a normal number (one below 2^-126 is flushed to 0,
+// which would put every point into bin 0).
+__device__ __forceinline__ float window_scale(float lo, float hi) {
+    const float r = __builtin_amdgcn_rcpf(hi - lo);
+    return fmaxf(fabsf(lo), fabsf(hi)) < 0x1p124f ? r : __builtin_nanf("");
+}
+
 // One part of the level.
 template <typename Acc>
 struct SubSlot {
-    float4 win;       // lo, hi (par_rcb_split's min, max; lo is the split once closed), 1 / (hi - lo), flags
+    float4 win;       // lo, hi (par_rcb_split's min, max; lo is the split once closed), window_scale, flags
     Acc sum;          // weight of the part
     Acc bw;           // weight below the window; of the left side once closed
     uint32_t n;       // points of the part
@@ -103,8 +113,8 @@ struct SubRoot {
 // further from a whole number than the candidates (midpoints taken in f32,
 // within a few ulps of the window's magnitude of even spacing) and the
 // estimate itself can be off; the other points (and all of a window that is
-// only a few ulps wide, or not finite) walk the midpoints par_rcb_split
-// computes (:472).
+// only a few ulps wide, or that has no estimate: window_scale) walk the
+// midpoints par_rcb_split computes (:472).
 // coord(j, flags): point j's coordinate on its window's axis.
 template <int B, typename Tree, typename Coord, typename Acc>
 __device__ __forceinline__ void sub_bin(const Tree &T, const uint32_t (&s)[B], Coord &&coord, const Acc (&w)[B],
@@ -405,7 +415,7 @@ __device__ __forceinline__ void sub_decide(const SubTree<Acc, TPB> &T, const Sub
             T.at(s).prev = prev;
             const uint32_t k = atomicAdd(n_next, 1u);
             next[k] = (uint16_t)s;
-            T.at(s).win = make_float4(lo, hi, __builtin_amdgcn_rcpf(hi - lo), __builtin_bit_cast(float, f | k));
+            T.at(s).win = make_float4(lo, hi, window_scale(lo, hi), __builtin_bit_cast(float, f | k));
         } else {
             T.at(s).bc = stop >= 0 ? T.binc(e0 + stop) & kCandCount : T.at(s).n;
             T.at(s).bw = stop >= 0 ? T.binw(e0 + stop) : T.at(s).sum;
@@ -430,7 +440,7 @@ __device__ __forceinline__ void sub_start(const SubTree<Acc, TPB> &T, uint32_t s
         list[k] = (uint16_t)s;
         f = kSubOpen | k;
     }
-    T.at(s).win = make_float4(lo, hi, __builtin_amdgcn_rcpf(hi - lo), __builtin_bit_cast(float, f));
+    T.at(s).win = make_float4(lo, hi, window_scale(lo, hi), __builtin_bit_cast(float, f));
 }
 
 // Splits a subtree of n points of weight `sum` level by level.
