@@ -105,6 +105,7 @@ struct PendingCall {
     double ws_bytes = 0.0;              // bytes of one stored weight
     int mode = -1;                      // weight mode the call ran in
     int wkind = 0;                      // caller's weight type
+    bool in_place = false;              // it left the points in place (rcb_mid.h, rcb_front.h)
 };
 
 // A captured call: the graph of every launch and copy of one call of a

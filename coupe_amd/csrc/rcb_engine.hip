@@ -1142,11 +1142,13 @@ static MidCounters wait_counters(Context &cx, hipStream_t st, const void *also =
 }
 
 // Runs a call on the midpoint tree after its prologue.  w: the stored weights,
-// or the caller's (w_src).  Waits for the stream and reads the call's
-// counters.  False when an open node is too large for a workgroup: nothing
-// was written then, and the call goes on on the general path.
+// or the caller's (w_src).  Waits for the stream and returns the call's
+// counters; where `big` is set (an open node is too large for a workgroup)
+// nothing was written, and the call goes on on another path.  The shape's
+// hints are left to the caller: the call may have run on weights of a mode
+// that did not hold.
 template <int D, typename WL, typename Acc>
-static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
+static MidCounters run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
                     int w_src) {
     Counters *ctr = (Counters *)cx.counters.ptr;
     MidCounters *mid = (MidCounters *)((char *)ctr + offsetof(Counters, mid));
@@ -1258,24 +1260,14 @@ static bool run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32,
     }
     if (m.error) throw HipFailure{hipErrorUnknown};
     cx.mid_clean = true;
-    cx.pending.shape = B.shape;
-    Hints &h = cx.remember(B.shape);
-    h.mid = m.big ? 0 : 1;
-    h.mid_open = m.open;
-    if (m.big) return false;
-    cx.stats.levels = B.max_levels;
-    cx.stats.passes = B.max_levels;
-    cx.stats.max_passes = std::max(cx.stats.max_passes, 1u);
-    cx.stats.unit_points = kTile;
-    cx.stats.bins = m.open ? (uint32_t)kSubMaxNb : 2u;
-    return true;
+    return m;
 }
 
 // Runs a call of one instance on the frontier after its prologue (w, w_src as
-// for run_mid).  Waits for the stream and reads the call's counters.  False:
-// its rounds are not enough.
+// for run_mid).  Waits for the stream and reads the call's counters.  Returns
+// the rounds it took, 0 when they are not enough; the hints as for run_mid.
 template <int D, typename WL, typename Acc>
-static bool run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
+static uint32_t run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap32, uint64_t *d_out, const WL *w,
                       int w_src) {
     const uint64_t n = B.n, cells = B.heap_total + 1;
     const uint32_t nt = (uint32_t)B.tiles0;
@@ -1367,22 +1359,12 @@ static bool run_front(Context &cx, hipStream_t st, const BatchPlan &B, int wrap3
         if (m.error) throw HipFailure{hipErrorUnknown};
         if (h[done].nodes == 0) break;
         cx.stats.reruns = 1;
-        if (done >= kFrontRounds - 2) return false;   // (coordinates over all of f32's exponents)
+        if (done >= kFrontRounds - 2) return 0;   // (coordinates over all of f32's exponents)
         queue = 8;
     }
     uint32_t used = 0;
     while (used < (uint32_t)kFrontRounds && h[used].nodes) used++;
-    cx.pending.shape = B.shape;
-    Hints &e = cx.remember(B.shape);
-    e.front_rounds = used;
-    // the midpoint tree again when every level took one round
-    if (e.mid == 0 && used <= B.max_levels) e.mid = -1;
-    cx.stats.levels = B.max_levels;
-    cx.stats.passes = used;
-    cx.stats.max_passes = std::max(cx.stats.max_passes, 1u);
-    cx.stats.unit_points = kTile;
-    cx.stats.bins = kSubMaxNb;
-    return true;
+    return used;
 }
 
 template <int D, typename WIN>
@@ -1459,28 +1441,57 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
         cx.pending.shape = B.shape;
         cx.pending.mode = mode;
         cx.pending.wkind = wkind;
+        cx.pending.in_place = false;
         // the midpoint tree, then the frontier, then the general path
         const bool mid = mid_fits(cx, B, spec_passes), front = front_fits(cx, B, spec_passes);
         if (mid || front) {
             cx.stats.weight_mode = mode == 3 ? 1 : 0;
             cx.stats.weight_bytes = weight_bytes(mode);
-            auto in_place = [&](auto *w, auto acc, int w_src) {
+            enum Outcome { kDone, kAgain, kGeneral };
+            auto finish = [&](uint32_t passes, uint32_t bins) {
+                cx.pending.in_place = true;
+                cx.stats.levels = B.max_levels;
+                cx.stats.passes = passes;
+                cx.stats.max_passes = 1;
+                cx.stats.unit_points = kTile;
+                cx.stats.bins = bins;
+                return kDone;
+            };
+            // the shape's hints only from a run whose weights were the call's
+            // (one in a mode that did not hold weighed points with what the
+            // buffers held before)
+            auto in_place = [&](auto *w, auto acc, int w_src) -> Outcome {
                 using WL = typename std::remove_const<typename std::remove_pointer<decltype(w)>::type>::type;
                 using Acc = decltype(acc);
                 const int wrap = std::is_same<Acc, double>::value ? 0 : (int)wrap32;
                 if (mid) {
-                    if (run_mid<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src)) return true;
+                    const MidCounters m = run_mid<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
+                    if (!mode_held(cx)) return kAgain;
+                    Hints &h = cx.remember(B.shape);
+                    h.mid = m.big ? 0 : 1;
+                    h.mid_open = m.open;
+                    if (!m.big) return finish(B.max_levels, m.open ? (uint32_t)kSubMaxNb : 2u);
                     cx.stats.reruns = 1;   // on, from the prologue's arrays
                 }
-                return front && run_front<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
+                if (front) {
+                    const uint32_t rounds = run_front<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
+                    if (!mode_held(cx)) return kAgain;
+                    if (rounds == 0) return kGeneral;
+                    Hints &h = cx.remember(B.shape);
+                    h.front_rounds = rounds;
+                    // the midpoint tree again when every level took one round
+                    if (h.mid == 0 && rounds <= B.max_levels) h.mid = -1;
+                    return finish(rounds, kSubMaxNb);
+                }
+                return kGeneral;
             };
-            bool done = false;   // (integers never need f64 sums)
-            if (mode == 0) done = in_place((const uint16_t *)cx.w16.ptr, uint64_t{}, 0);
-            else if (mode == 1) done = in_place((const int32_t *)cx.w[0].ptr, uint64_t{}, 0);
-            else if (mode == 2) done = in_place(win, uint64_t{}, 1);
-            else if constexpr (std::is_same<WIN, double>::value) done = in_place(win, double{}, 1);
-            if (!mode_held(cx)) continue;
-            if (done) return false;
+            Outcome end = kGeneral;   // (integers never need f64 sums)
+            if (mode == 0) end = in_place((const uint16_t *)cx.w16.ptr, uint64_t{}, 0);
+            else if (mode == 1) end = in_place((const int32_t *)cx.w[0].ptr, uint64_t{}, 0);
+            else if (mode == 2) end = in_place(win, uint64_t{}, 1);
+            else if constexpr (std::is_same<WIN, double>::value) end = in_place(win, double{}, 1);
+            if (end == kAgain) continue;
+            if (end == kDone) return false;
         }
         const bool unfinished = run_mode(mode);
         if (cx.capturing) return false;   // checked once the graph has run
@@ -1803,7 +1814,8 @@ static enum coupe_err rcb_general(Context &cx, hipStream_t st, uint64_t *d_out, 
             cx.stats.reruns = 1;
             run(0, st);
         }
-        cx.remember(B.shape).passes_hint = (int)cx.stats.max_passes;
+        // (calls in place say nothing of the general path's searches)
+        if (!cx.pending.in_place) cx.remember(B.shape).passes_hint = (int)cx.stats.max_passes;
     } catch (const HipFailure &f) {
         cx.bins_clean = false;
         (void)hipGetLastError();

@@ -59,3 +59,36 @@ def test_weights_of_another_type_between_other_shapes(oracle_mod, monkeypatch, o
                   f"graphs {graphs}, {order}: call {k} {call}")
     finally:
         ctx.close()
+
+
+def path_of(ctx):
+    """The path of the context's last call (profiling enabled)."""
+    t = ctx.kernel_times()
+    if t["prologue"]["launches"] == 0:
+        return "small"
+    if t["partition"]["algo_bytes"] > 0:
+        return "general"
+    return "mid" if t["decide"]["launches"] == 1 else "front"
+
+
+@pytest.mark.parametrize("n", [50_000, 400_000])
+@pytest.mark.parametrize("kinds", ["unit real real", "whole real real", "real whole real", "unit int64 real", "int64 real unit"])
+def test_a_change_of_weights_leaves_the_shape_its_path(oracle_mod, n, kinds):
+    """Points that split at the midpoints: a call whose expected weight mode
+    does not hold runs again, and neither it nor the next one ends on another path."""
+    pytest.importorskip("torch")
+    rng = np.random.default_rng(n)
+    iters, tol = 8, 0.25
+    ctx = coupe_amd.DeviceContext(0)
+    try:
+        ctx.set_profiling(True)
+        for k, kind in enumerate(kinds.split()):
+            for again in range(2):
+                _call(oracle_mod, ctx, rng.random((n, 3)), _weights(rng, kind, n), iters, tol,
+                      f"n={n} {kinds}: call {k}.{again} {kind}")
+                st = ctx.stats()
+                assert st["passes"] == iters, st
+                if again:
+                    assert path_of(ctx) == "mid", ctx.kernel_times()
+    finally:
+        ctx.close()
