@@ -108,13 +108,15 @@ uint64_t batch_bytes(uint64_t n, uint64_t dim, uint64_t wsize, uint64_t parts, u
 // What the paths that leave the points in place hold besides (points gathered,
 // cells and slots; the tables of at most kMidCells cells; the frontier's
 // bins).  A batch that fits the budget only without runs on the general path.
-uint64_t in_place_bytes(uint64_t n, uint64_t dim, uint64_t wsize, uint64_t requests, uint64_t levels) {
-    if (levels > 12) return 0;
+// large: requests that do not run as one workgroup.  Where there is one it is
+// the only instance left for these paths, and may take the frontier.
+uint64_t in_place_bytes(uint64_t n, uint64_t dim, uint64_t wsize, uint64_t requests, uint64_t large, uint64_t levels) {
+    if (levels > 12 || large == 0) return 0;
     const uint64_t record = dim == 3 && wsize == 8 ? 24 : 16;
     const uint64_t cells = std::min<uint64_t>(coupe_hip::kMidCells, requests << levels);
     uint64_t b = n * (2 + 2 + record);
     b += cells * ((cells <= coupe_hip::kMidCopied ? 8 : 1) * 12 + 4 + 64 + 4 + 3 * 4 + 4);   // counts, map, open nodes, cursors, lists, splits
-    if (requests == 1 && n > 16384) b += 256ull * (5376 * 16 + 1024 * 4) + (1ull << 20);   // the frontier's bins
+    if (large == 1) b += 256ull * (5376 * 16 + 1024 * 4) + (1ull << 20);   // the frontier's bins
     return b + b / 8;
 }
 
@@ -286,6 +288,9 @@ bool pick_batch(coupe_hip_server *S, Worker *W, std::vector<Req *> &batch) {
     const uint64_t room = S->cfg.memory_budget - std::min(S->cfg.memory_budget, S->mesh_bytes);
     uint64_t pts = n_of(first), parts = parts_bound(pts, first->r.iter_count);
     uint64_t levels = first->r.iter_count;
+    // (COUPE_HIP_SMALL=0: none runs as one workgroup)
+    auto is_large = [&](const Req *q) { return !W->cx.small || n_of(q) > 16384 || q->r.iter_count > 12; };
+    uint64_t large = is_large(first) ? 1 : 0;
     std::vector<std::deque<Req *>::iterator> take;
     if (!alone(first)) {
         for (auto it = head + 1; it != S->queue.end() && take.size() + 1 < S->cfg.max_batch_requests; ++it) {
@@ -300,13 +305,14 @@ bool pick_batch(coupe_hip_server *S, Worker *W, std::vector<Req *> &batch) {
             pts += q->r.n;
             parts = p2;
             levels = l2;
+            large += is_large(q) ? 1 : 0;
         }
     }
     // admission: what W will hold for this batch (at least what it holds now,
     // its buffers only grow), against what the others and the meshes hold now
     uint64_t need = batch_bytes(pts, dim, wsize, parts, levels, !first->mesh);
     const uint64_t others = S->held() - W->held;
-    const uint64_t more = in_place_bytes(pts, dim, wsize, take.size() + 1, levels);
+    const uint64_t more = in_place_bytes(pts, dim, wsize, take.size() + 1, large, levels);
     W->cx.in_place = others + std::max(need + more, W->held) <= S->cfg.memory_budget;
     if (W->cx.in_place) need += more;
     if (others + std::max(need, W->held) > S->cfg.memory_budget) {
