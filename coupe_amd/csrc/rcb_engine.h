@@ -230,10 +230,14 @@ struct Context {
         weight_hint = h.weight_hint;
     }
     uint64_t device_bytes() const;
+    uint64_t in_place_bytes() const;   // of them, the paths' that leave the points in place
+    void release_in_place();
     void release_all();
     void forget_all();               // every buffer dropped without freeing (arena contexts)
     template <typename F>
     void for_each_buf(F &&f);
+    template <typename F>
+    void for_each_in_place(F &&f);
 };
 
 enum coupe_err map_hip_error(hipError_t e);

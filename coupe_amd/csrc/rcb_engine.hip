@@ -2104,9 +2104,16 @@ void Context::for_each_buf(F &&f) {
                      &tile_bins2, &tile4, &bcnt, &bw, &bmin, &xcnt, &xw, &xmin, &nchild, &ntiles, &bsum, &nodes, &leaf,
                      &heap_split, &instances, &tiles0, &below, &tile_left, &loads, &rib_moments, &tile_bins,
                      &gparts[0], &gparts[1], &gaxis, &gchunk, &gcount, &gctr, &gsat, &gcol, &grow, &gheap, &gscan,
-                     &mid_code, &mid_cnt, &mid_w, &mid_map, &mid_inst, &mid_open, &mid_cursor, &mid_lists, &mid_slots, &mid_points,
-                     &front_nodes[0], &front_nodes[1], &front_routes, &front_rounds, &front_w, &front_c, &front_m, &front_h,
                      &small_table, &small_report, &ired, &counters, &in_points, &in_weights, &out_ids};
+    for (DevBuf *d : all) f(*d);
+    for_each_in_place(f);
+}
+
+template <typename F>
+void Context::for_each_in_place(F &&f) {
+    DevBuf *all[] = {&mid_code, &mid_cnt, &mid_w, &mid_map, &mid_inst, &mid_open, &mid_cursor, &mid_lists, &mid_slots,
+                     &mid_points, &front_nodes[0], &front_nodes[1], &front_routes, &front_rounds, &front_w, &front_c,
+                     &front_m, &front_h};
     for (DevBuf *d : all) f(*d);
 }
 
@@ -2130,6 +2137,17 @@ uint64_t Context::device_bytes() const {
     uint64_t b = 0;
     const_cast<Context *>(this)->for_each_buf([&](DevBuf &d) { b += d.bytes; });
     return b;
+}
+
+uint64_t Context::in_place_bytes() const {
+    uint64_t b = 0;
+    const_cast<Context *>(this)->for_each_in_place([&](DevBuf &d) { b += d.bytes; });
+    return b;
+}
+
+void Context::release_in_place() {
+    for_each_in_place([](DevBuf &d) { d.release(); });
+    mid_clean = false;
 }
 
 void Context::release_all() {

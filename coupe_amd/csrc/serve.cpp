@@ -80,6 +80,8 @@ struct Worker {
     DevBuf pts, w, ids;
     std::thread th;
     uint64_t held = 0;                // device bytes this worker holds (accounted)
+    uint64_t held_in_place = 0;       // of them, the buffers of the paths in place
+    bool drop_in_place = false;       // those are given back before the next batch
     uint64_t bytes() { return cx.device_bytes() + pts.bytes + w.bytes + ids.bytes; }
     void trim() {
         cx.release_all();
@@ -308,24 +310,30 @@ bool pick_batch(coupe_hip_server *S, Worker *W, std::vector<Req *> &batch) {
             large += is_large(q) ? 1 : 0;
         }
     }
-    // admission: what W will hold for this batch (at least what it holds now,
-    // its buffers only grow), against what the others and the meshes hold now
-    uint64_t need = batch_bytes(pts, dim, wsize, parts, levels, !first->mesh);
+    // admission: what W will hold for this batch, against what the others and
+    // the meshes hold now.  W's buffers only grow, and those of the paths in
+    // place lie beside the others: a batch of one kind keeps what one of the
+    // other kind left, unless there is no room for it.
     const uint64_t others = S->held() - W->held;
-    const uint64_t more = in_place_bytes(pts, dim, wsize, take.size() + 1, large, levels);
-    W->cx.in_place = others + std::max(need + more, W->held) <= S->cfg.memory_budget;
-    if (W->cx.in_place) need += more;
-    if (others + std::max(need, W->held) > S->cfg.memory_budget) {
+    const uint64_t core = std::max(batch_bytes(pts, dim, wsize, parts, levels, !first->mesh),
+                                   W->held - W->held_in_place);
+    uint64_t in_place = std::max(in_place_bytes(pts, dim, wsize, take.size() + 1, large, levels), W->held_in_place);
+    auto fits = [&](uint64_t bytes) { return others + core + bytes <= S->cfg.memory_budget; };
+    W->cx.in_place = fits(in_place);
+    if (!W->cx.in_place) in_place = fits(W->held_in_place) ? W->held_in_place : 0;
+    if (!fits(in_place)) {
         S->memory_wanted = true;
         return false;
     }
+    W->drop_in_place = in_place < W->held_in_place;
     batch.push_back(first);
     for (auto it : take) batch.push_back(*it);
     for (Req *q : batch) q->started = true;
     S->queue.erase(std::remove_if(S->queue.begin(), S->queue.end(), [](const Req *q) { return q->started; }),
                    S->queue.end());
     if (first->mesh) first->mesh->busy = true;
-    W->held = std::max(need, W->held);   // accounted until the batch's real figure is known
+    W->held = core + in_place;   // accounted until the batch's real figure is known
+    W->held_in_place = in_place;
     S->note_peak();
     return true;
 }
@@ -342,7 +350,7 @@ void worker_main(coupe_hip_server *S, Worker *W) {
                 lk.unlock();
                 W->trim();
                 lk.lock();
-                W->held = 0;
+                W->held = W->held_in_place = 0;
                 S->cv_work.notify_all();
                 continue;
             }
@@ -351,11 +359,13 @@ void worker_main(coupe_hip_server *S, Worker *W) {
         S->memory_wanted = false;
         S->running += (uint32_t)batch.size();
         lk.unlock();
+        if (W->drop_in_place) W->cx.release_in_place();
         run_batch(W, batch);
         if (batch[0]->err == COUPE_ERR_ALLOC) W->trim();   // nothing left behind by a failed growth
-        const uint64_t real = W->bytes();
+        const uint64_t real = W->bytes(), real_in_place = W->cx.in_place_bytes();
         lk.lock();
         W->held = real;
+        W->held_in_place = real_in_place;
         S->note_peak();
         S->running -= (uint32_t)batch.size();
         for (Req *q : batch) {

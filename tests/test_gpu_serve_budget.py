@@ -42,3 +42,27 @@ def test_one_larger_request_among_small_ones(oracle_mod):
         assert st["peak_device_bytes"] <= budget, st
     finally:
         srv.close()
+
+
+def test_buffers_of_both_kinds_of_paths(oracle_mod):
+    """A batch in place, then, with a mesh created meanwhile, one for which
+    only the general path's buffers have room: those of the first are given back."""
+    rng = np.random.default_rng(6)
+    budget, n, iters = 420_000_000, 2_000_000, 10
+    srv = coupe_amd.Server(slots=1, memory_budget=budget)
+    try:
+        # (the frontier: its bins are held too)
+        pts, w, out = rng.normal(0, 1, (n, 3)) ** 5, rng.integers(1, 100, n).astype(np.float64), np.zeros(n, dtype=np.uint64)
+        for call in range(3):
+            srv.wait(srv.submit(out, pts, w, iters, 0.05))
+            _same(oracle_mod, out, pts, w, iters, 0.05, f"call {call}")
+            st = srv.stats()
+            assert st["peak_device_bytes"] <= budget, st
+            if call == 0:   # 28 bytes a point
+                mesh = srv.create_mesh(rng.random((6_857_000, 3)), np.ones(6_857_000))
+        mesh.destroy()
+        srv.wait(srv.submit(out, pts, w, iters, 0.05))
+        _same(oracle_mod, out, pts, w, iters, 0.05, "after the mesh")
+        assert srv.stats()["peak_device_bytes"] <= budget
+    finally:
+        srv.close()
