@@ -313,16 +313,6 @@ inline bool front_from_env() {
     return !(v && v[0] == '0');
 }
 
-// Whether a switch of the general path is set in the environment: such a
-// context runs that path, as the switches say.
-inline bool general_from_env() {
-    for (const char *name : {"COUPE_HIP_PAIRS", "COUPE_HIP_FORWARD", "COUPE_HIP_FULL_FIRST", "COUPE_HIP_BIN_COPIES",
-                             "COUPE_HIP_MOVE_NT_BYTES", "COUPE_HIP_SEARCH_CHUNK", "COUPE_HIP_GRAPHS", "COUPE_HIP_BINS",
-                             "COUPE_HIP_WG_PER_CU", "COUPE_HIP_SCAN_DIRECT", "COUPE_HIP_SEARCH_PASSES"})
-        if (getenv(name)) return true;
-    return false;
-}
-
 // COUPE_HIP_SEARCH_CHUNK=k: the later search passes hand k consecutive
 // tiles at a time to each workgroup (default 2, at most 64).
 inline uint32_t search_chunk_from_env() {
@@ -387,12 +377,23 @@ inline void configure_from_env(Context &c) {
     c.graphs = graphs_from_env();
     c.copy_parts = copy_parts_from_env();
     c.search_chunk = search_chunk_from_env();
-    c.small = small_from_env();
-    c.mid = mid_from_env() && !general_from_env();
-    c.front = front_from_env() && !general_from_env();
     c.move_nt_bytes = move_nt_bytes_from_env();
     c.max_bins = bins_from_env();
     c.wg_cap = wg_cap_from_env();
+    // a context with a switch of the general path off its default runs that
+    // path, and so does one that asks for a part of it by name, on or off
+    auto named = [](const char *name) {
+        const char *v = getenv(name);
+        return v && *v;
+    };
+    const Context d{};
+    const bool general = named("COUPE_HIP_PAIRS") || named("COUPE_HIP_FORWARD") || named("COUPE_HIP_FULL_FIRST") ||
+                         c.search_passes != d.search_passes || c.scan_direct != d.scan_direct ||
+                         c.graphs != d.graphs || c.copy_parts != d.copy_parts || c.search_chunk != d.search_chunk ||
+                         c.move_nt_bytes != d.move_nt_bytes || c.max_bins != d.max_bins || c.wg_cap != d.wg_cap;
+    c.small = small_from_env() && !general;
+    c.mid = mid_from_env() && !general;
+    c.front = front_from_env() && !general;
 }
 
 // The context's switches as a tuning record, and back.

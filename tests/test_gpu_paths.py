@@ -1,0 +1,88 @@
+"""Which path a call takes: switches of the general path count where they differ
+from their defaults (those of its parts wherever they are set), and each path
+gives the oracle's ids where it is the one that runs."""
+import numpy as np
+import pytest
+
+import coupe_amd
+from tests import cases
+from tests.test_gpu_hints import path_of
+from tests.test_gpu_mid import _same
+
+pytestmark = pytest.mark.gpu
+
+PARTS = ("PAIRS", "FORWARD", "FULL_FIRST")
+DEFAULTS = {"PAIRS": "1", "FORWARD": "1", "FULL_FIRST": "1", "BIN_COPIES": "256", "MOVE_NT_BYTES": "2.5e9",
+            "SEARCH_CHUNK": "2", "GRAPHS": "0", "BINS": "256", "WG_PER_CU": "0", "SCAN_DIRECT": "2048",
+            "SEARCH_PASSES": "3"}
+OTHERS = {"PAIRS": "0", "FORWARD": "0", "FULL_FIRST": "0", "BIN_COPIES": "0", "MOVE_NT_BYTES": "0", "SEARCH_CHUNK": "1",
+          "GRAPHS": "1", "BINS": "64", "WG_PER_CU": "2", "SCAN_DIRECT": "64", "SEARCH_PASSES": "2"}
+
+
+def _call(oracle_mod, ctx, pts, w, iters, tol, label):
+    import torch
+
+    print(f"[gpu] {label}", flush=True)
+    out = torch.full((len(w),), -1, dtype=torch.int64, device="cuda")
+    coupe_amd.Rcb(iters, tol).partition(out, (torch.from_numpy(pts).cuda(), torch.from_numpy(w).cuda()), context=ctx)
+    err, exp, _ = oracle_mod.rcb(pts, w, iters, tol, parallel=True, nthreads=8)
+    assert err == 0
+    _same(out.cpu().numpy().astype(np.uint64), exp, w, label)
+    return path_of(ctx)
+
+
+@pytest.mark.parametrize("name", sorted(DEFAULTS))
+def test_switches_at_and_off_their_defaults(oracle_mod, monkeypatch, name):
+    pytest.importorskip("torch")
+    rng = np.random.default_rng(2)
+    in_place, general = ("small", "mid"), ("general", "general")
+    for value, expect in ((DEFAULTS[name], general if name in PARTS else in_place), ("", in_place),
+                          (OTHERS[name], general)):
+        monkeypatch.setenv(f"COUPE_HIP_{name}", value)
+        ctx = coupe_amd.DeviceContext(0)
+        try:
+            ctx.set_profiling(True)
+            for n, path in zip((5000, 60_000), expect):
+                got = _call(oracle_mod, ctx, rng.random((n, 3)), rng.integers(1, 50, n).astype(np.float64), 6, 0.2,
+                            f"{name}={value!r} n={n}")
+                assert got == path, f"{name}={value!r} n={n}: {got}"
+        finally:
+            ctx.close()
+
+
+@pytest.mark.parametrize("path", ["default", "front", "general"])
+@pytest.mark.parametrize("seed", range(3))
+def test_each_path_where_it_runs(oracle_mod, monkeypatch, path, seed):
+    """Clouds for every path; with the tree off the frontier takes them, with
+    both (and the small problems) off the general path."""
+    pytest.importorskip("torch")
+    if path != "default":
+        for name in ("SMALL", "MID") + (("FRONT",) if path == "general" else ()):
+            monkeypatch.setenv(f"COUPE_HIP_{name}", "0")
+    rng = np.random.default_rng(seed)
+    ctx = coupe_amd.DeviceContext(0)
+    try:
+        ctx.set_profiling(True)
+        for n, dim, expect in ((3000, 3, "small"), (70_001, 2, "mid"), (300_000, 3, "mid"), (120_000, 3, "front")):
+            even = expect != "front"
+            pts = rng.random((n, dim)) if even else rng.normal(0, 1, (n, dim)) ** 5
+            w = rng.integers(1, 50, n).astype([np.float64, np.int32, np.int64][seed])
+            for call in range(2):
+                got = _call(oracle_mod, ctx, pts, w, 7, 0.05 if even else 0.01, f"{path} n={n} d={dim} call {call}")
+                assert got == (expect if path == "default" else path), got
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_general_path_on_small_cases(oracle_mod, monkeypatch, seed):
+    """The general path on inputs the one-workgroup kernel takes by default."""
+    pytest.importorskip("torch")
+    for name in ("SMALL", "MID", "FRONT"):
+        monkeypatch.setenv(f"COUPE_HIP_{name}", "0")
+    pts, w, iters, tol = cases.random_case(700 + seed, 3000)
+    ctx = coupe_amd.DeviceContext(0)
+    try:
+        _call(oracle_mod, ctx, pts, w, iters, tol, f"seed {seed}")
+    finally:
+        ctx.close()
