@@ -39,6 +39,16 @@ struct ArenaScope {
     ~ArenaScope();
 };
 
+// A bound on the device bytes of a context's buffers, while it is installed on
+// the calling thread (COUPE_HIP_MEMORY_LIMIT): an allocation past it fails like
+// one the device has no memory for.
+struct MemoryScope {
+    uint64_t limit, held;
+    MemoryScope *prev;
+    MemoryScope(uint64_t limit_, uint64_t held_);
+    ~MemoryScope();
+};
+
 // A grow-only device allocation (or, under an ArenaScope, a carve of the
 // arena: `borrowed` buffers are never freed).
 struct DevBuf {
@@ -89,6 +99,7 @@ struct Hints {
     int mid = -1;                       // the midpoint tree took its last call (-1: not tried, 0: no)
     uint32_t front_rounds = 0;          // rounds the frontier took in its last call
     uint32_t mid_open = 1;              // open nodes the midpoint tree left (0: none)
+    bool no_room = false;               // the paths in place could not have their buffers
     int moves_coherent = -1;            // its moved tiles went to few destinations (-1: not known)
 };
 
@@ -154,6 +165,7 @@ struct Context {
     uint32_t copy_parts = 256;       // levels of at most this many parts flush into per-XCD copies
     uint32_t search_chunk = 2;       // consecutive tiles a workgroup takes at a time in the search passes
     bool small = true;               // problems of few points take one workgroup each (rcb_small.h)
+    uint64_t memory_limit = 0;       // most device bytes of its buffers (0: no bound but the device's)
     bool in_place = true;            // false: calls that leave the points in place are not taken (a bound on bytes)
     bool mid = true;                 // try the tree of box midpoints first (rcb_mid.h)
     bool front = true;               // search one instance's levels without moving its points (rcb_front.h)
@@ -313,6 +325,14 @@ inline bool front_from_env() {
     return !(v && v[0] == '0');
 }
 
+// COUPE_HIP_MEMORY_LIMIT=b: a context's buffers take at most b bytes of device
+// memory; a call that needs more fails as when the device has no more.
+inline uint64_t memory_limit_from_env() {
+    const char *v = getenv("COUPE_HIP_MEMORY_LIMIT");
+    const double b = v && *v ? atof(v) : 0.0;
+    return b > 0.0 ? (uint64_t)b : 0;
+}
+
 // COUPE_HIP_SEARCH_CHUNK=k: the later search passes hand k consecutive
 // tiles at a time to each workgroup (default 2, at most 64).
 inline uint32_t search_chunk_from_env() {
@@ -377,6 +397,7 @@ inline void configure_from_env(Context &c) {
     c.graphs = graphs_from_env();
     c.copy_parts = copy_parts_from_env();
     c.search_chunk = search_chunk_from_env();
+    c.memory_limit = memory_limit_from_env();
     c.move_nt_bytes = move_nt_bytes_from_env();
     c.max_bins = bins_from_env();
     c.wg_cap = wg_cap_from_env();

@@ -39,6 +39,13 @@ static thread_local bool t_capturing = false;   // a stream capture is running o
 ArenaScope::ArenaScope(Arena *a) : prev(t_arena) { t_arena = a; }
 ArenaScope::~ArenaScope() { t_arena = prev; }
 
+static thread_local MemoryScope *t_memory = nullptr;
+
+MemoryScope::MemoryScope(uint64_t limit_, uint64_t held_) : limit(limit_), held(held_), prev(t_memory) {
+    t_memory = limit ? this : nullptr;
+}
+MemoryScope::~MemoryScope() { t_memory = prev; }
+
 void DevBuf::ensure(size_t need) {
     if (need <= bytes) return;
     // a capture records no allocation: the caller gives it up and runs eagerly
@@ -55,14 +62,18 @@ void DevBuf::ensure(size_t need) {
         return;
     }
     if (ptr && !borrowed) check(hipFree(ptr));
+    if (t_memory) t_memory->held -= bytes;
     ptr = nullptr;
     bytes = 0;
     borrowed = false;
+    if (t_memory && t_memory->held + sz > t_memory->limit) throw HipFailure{hipErrorOutOfMemory};
     check(hipMalloc(&ptr, sz));
     bytes = sz;
+    if (t_memory) t_memory->held += sz;
 }
 
 void DevBuf::release() {
+    if (t_memory) t_memory->held -= bytes;
     if (ptr && !borrowed) (void)hipFree(ptr);
     ptr = nullptr;
     bytes = 0;
@@ -1093,6 +1104,8 @@ static void prologue(Context &cx, hipStream_t st, const BatchPlan &B, const doub
 static bool in_place_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
     if (!cx.in_place || spec_passes <= 0 || cx.capturing || cx.graphs || t_arena) return false;
     if (!B.dense || B.max_levels == 0 || B.max_levels > kMidLevels) return false;
+    const Hints *seen = cx.hints_for(B.shape);
+    if (seen && seen->no_room) return false;
     return B.heap_total + B.inst.size() <= kMidCells;
 }
 static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
@@ -1782,9 +1795,36 @@ static enum coupe_err rcb_general(Context &cx, hipStream_t st, uint64_t *d_out, 
             check(hipDeviceGetAttribute(&cx.cu_count, hipDeviceAttributeMultiprocessorCount, cx.device));
             if (cx.cu_count <= 0) cx.cu_count = 1;
         }
-        auto run = [&](int spec, hipStream_t s) {
+        auto run_once = [&](int spec, hipStream_t s) {
             return dim == 2 ? run_dim<2>(cx, s, d_out, B, d_points, wkind, d_weights, spec)
                             : run_dim<3>(cx, s, d_out, B, d_points, wkind, d_weights, spec);
+        };
+        // The paths in place have buffers of their own, beside the general
+        // path's.  Where they cannot be had, or leave no room for the general
+        // path's, they are given back, and the call (and the shape's later
+        // ones) runs on the general path.
+        auto run = [&](int spec, hipStream_t s) {
+            try {
+                return run_once(spec, s);
+            } catch (const HipFailure &f) {
+                if (map_hip_error(f.err) != COUPE_ERR_ALLOC || cx.capturing ||
+                    (cx.in_place_bytes() == 0 && !in_place_fits(cx, B, spec)))
+                    throw;
+            }
+            (void)hipGetLastError();
+            check(hipStreamSynchronize(s));
+            cx.release_in_place();
+            cx.bins_clean = false;
+            Hints h = {};
+            if (const Hints *seen = cx.hints_for(B.shape)) h = *seen;
+            else h.weight_hint = cx.weight_hint;
+            h.shape = B.shape;
+            h.no_room = true;
+            cx.remember(B.shape) = h;
+            cx.stats = coupe_hip_stats{};
+            cx.stats.points = B.n;
+            cx.stats.reruns = 1;
+            return run_once(spec, s);
         };
         // Passes queued per level: the configured depth, or fewer (never
         // under 2) when this context's last call needed fewer (its deepest
@@ -1874,6 +1914,7 @@ enum coupe_err rcb_batch(Context &cx, hipStream_t st, uint64_t *d_out, size_t di
             for (int k = 0; k < 3; k++) c.slot0[k] = nullptr;
         }
     } call_scope(cx, rot, src);
+    MemoryScope memory_scope(cx.memory_limit, cx.memory_limit ? cx.device_bytes() : 0);
     cx.swept_bytes = 0.0;
     // switches of the call: the autotuner's for its class, if any
     struct TuneScope {   // the context's own switches come back after the call
