@@ -1154,6 +1154,12 @@ static MidCounters wait_counters(Context &cx, hipStream_t st, const void *also =
     return *(const MidCounters *)(h_rb + (offsetof(Counters, mid) - off));
 }
 
+// A shape of this many points or more that the midpoint tree has not taken
+// before is looked at first: the buffers of gathered points (20 to 28 bytes a
+// point) only once its open nodes are known, at the cost of one more wait of
+// the host (10 to 20 us, of more than 300).
+constexpr uint64_t kMidLook = 1ull << 22;
+
 // Runs a call on the midpoint tree after its prologue.  w: the stored weights,
 // or the caller's (w_src).  Waits for the stream and returns the call's
 // counters; where `big` is set (an open node is too large for a workgroup)
@@ -1178,9 +1184,17 @@ static MidCounters run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int 
     cx.mid_open.ensure(cells * sizeof(MidOpen));
     cx.mid_cursor.ensure(cells * 4);
     cx.mid_lists.ensure(kMidClasses * cells * 4);
-    cx.mid_slots.ensure(n * 2);
     cx.heap_split.ensure(std::max<uint64_t>(B.heap_total, 1) * sizeof(float));
-    cx.mid_points.ensure(n * sizeof(MidPoint<D, WL>));
+    auto hold_points = [&] {
+        cx.mid_slots.ensure(n * 2);
+        cx.mid_points.ensure(n * sizeof(MidPoint<D, WL>));
+    };
+    // a shape whose last call left no node open queues no search; open nodes
+    // after all are searched once the counters are read
+    const Hints *seen = cx.hints_for(B.shape);
+    const bool known = seen && seen->mid >= 0, look = !known && n >= kMidLook;
+    const bool expect = known ? seen->mid_open > 0 : !look;
+    if (expect) hold_points();
     uint32_t *gcnt = (uint32_t *)cx.mid_cnt.ptr;
     Acc *gw = (Acc *)cx.mid_w.ptr;
     if (fresh || !cx.mid_clean) {   // k_mid_tree leaves them clear
@@ -1258,16 +1272,15 @@ static MidCounters run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int 
         if (n_inst == 1 && (4.0 * D + 8.0) * (double)n > cx.move_nt_bytes) launch(k_mid_ids<D, true>);
         else launch(k_mid_ids<D, false>);
     };
-    // a shape whose last call left no node open queues no search; open nodes
-    // after all are searched once the counters are read
-    const Hints *seen = cx.hints_for(B.shape);
-    const bool expect = !seen || seen->mid < 0 || seen->mid_open > 0;
     if (expect) search_open();
-    ids();
+    if (!look) ids();
     MidCounters m = wait_counters(cx, st);
-    if (!expect && m.open && !m.big) {
-        cx.stats.reruns = 1;
-        search_open();
+    if (!m.big && (look || (!expect && m.open))) {
+        if (m.open) {
+            if (known) cx.stats.reruns = 1;
+            hold_points();
+            search_open();
+        }
         ids();
         m = wait_counters(cx, st);
     }
@@ -1485,6 +1498,10 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
                     h.mid_open = m.open;
                     if (!m.big) return finish(B.max_levels, m.open ? (uint32_t)kSubMaxNb : 2u);
                     cx.stats.reruns = 1;   // on, from the prologue's arrays
+                    if (!front && B.n >= kMidLook) {   // the gathered points give way to the moved ones
+                        cx.mid_points.release();
+                        cx.mid_slots.release();
+                    }
                 }
                 if (front) {
                     const uint32_t rounds = run_front<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);

@@ -93,3 +93,44 @@ def test_no_room_at_all(monkeypatch):
             assert e.value.code == _native.ALLOC
     finally:
         ctx.close()
+
+
+def test_what_a_call_that_leaves_the_tree_holds(oracle_mod, monkeypatch):
+    """A large call that the midpoint tree gives up holds no gathered points
+    beside the general path's buffers; one that it takes gives the oracle's ids
+    on the first call, and its gathered points go when other points end elsewhere."""
+    torch = pytest.importorskip("torch")
+    n, pieces = 1 << 20, 5   # a batch: no frontier
+    rng = np.random.default_rng(4)
+    held = {}
+    clouds = {"cluster": rng.normal(0, 1, (n * pieces, 3)) ** 5, "uniform": rng.random((n * pieces, 3))}
+    w = rng.integers(1, 50, n * pieces).astype(np.float64)
+    out = torch.zeros(n * pieces, dtype=torch.int64, device="cuda")
+    for path in ("general", "default"):
+        if path == "general":
+            for name in ("SMALL", "MID", "FRONT"):
+                monkeypatch.setenv(f"COUPE_HIP_{name}", "0")
+        else:
+            for name in ("SMALL", "MID", "FRONT"):
+                monkeypatch.delenv(f"COUPE_HIP_{name}")
+        ctx = coupe_amd.DeviceContext(0)
+        ctx.set_profiling(True)
+        order = ["cluster", "uniform", "uniform", "cluster"] if path == "default" else ["cluster"]
+        for k, cloud in enumerate(order):
+            print(f"[gpu] {path} call {k}: {cloud}", flush=True)
+            iters = 8 if k == 0 else 7   # another shape after the first call
+            out.fill_(-1)
+            coupe_amd.partition_batch(out, torch.from_numpy(clouds[cloud]).cuda(), torch.from_numpy(w).cuda(),
+                                      [(n, iters, TOL)] * pieces, context=ctx)
+            got = out.cpu().numpy().astype(np.uint64)
+            for q in range(pieces):
+                s = slice(q * n, (q + 1) * n)
+                err, exp, _ = oracle_mod.rcb(clouds[cloud][s], w[s], iters, TOL, parallel=True, nthreads=8)
+                assert err == 0 and np.array_equal(got[s], exp), f"{path} call {k} {cloud} piece {q}"
+            st = ctx.stats()
+            held[path, k] = st["device_bytes"] / (n * pieces)
+            if path == "default" and cloud == "uniform":
+                assert path_of(ctx) == "mid" and st["reruns"] == 0, st
+        ctx.close()
+    for k in (0, 3):   # cells and tables: 2 bytes a point and a few more
+        assert held["default", k] < held["general", 0] + 4, held
