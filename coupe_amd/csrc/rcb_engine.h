@@ -117,6 +117,7 @@ struct PendingCall {
     int mode = -1;                      // weight mode the call ran in
     int wkind = 0;                      // caller's weight type
     bool in_place = false;              // it left the points in place (rcb_mid.h, rcb_front.h)
+    bool mid_skipped = false;           // the midpoint tree is not tried: it left the last new shapes' calls
 };
 
 // A captured call: the graph of every launch and copy of one call of a
@@ -183,6 +184,8 @@ struct Context {
     uint64_t layout() ;              // hash of every buffer's address and size
     void drop_graphs();
     int weight_hint = -1;            // weight mode of the last call, for a shape not seen before
+    uint32_t mid_misses = 0;         // new shapes in a row whose calls the midpoint tree left to the general path
+    uint32_t mid_wait = 0;           // new shapes that pass it by from now on
     std::vector<Hints> hints;        // per shape, the most recent last
     const Hints *hints_for(uint64_t shape) const {
         for (const Hints &h : hints)

@@ -226,7 +226,11 @@ static bool finish_levels(Context &cx) {
         e.level_passes = used;
         e.level_open = open1;
         // the midpoint tree again when every part of the first levels split at its midpoint
-        if (e.mid == 0 && P.levels >= 3 && open1[0] == 0 && open1[1] == 0 && open1[2] == 0) e.mid = -1;
+        if (e.mid == 0 || P.mid_skipped) {
+            const bool midpoints = P.levels >= 3 && open1[0] == 0 && open1[1] == 0 && open1[2] == 0;
+            e.mid = midpoints ? -1 : 0;
+            if (midpoints) cx.mid_misses = cx.mid_wait = 0;
+        }
     }
     return h->unfinished != 0;
 }
@@ -1108,14 +1112,31 @@ static bool in_place_fits(const Context &cx, const BatchPlan &B, int spec_passes
     if (seen && seen->no_room) return false;
     return B.heap_total + B.inst.size() <= kMidCells;
 }
-static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
-    if (!cx.mid || !in_place_fits(cx, B, spec_passes)) return false;
-    const Hints *seen = cx.hints_for(B.shape);
-    return !seen || seen->mid != 0;
-}
 // And whether the frontier (rcb_front.h) takes it after that.
 static bool front_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
     return cx.front && B.inst.size() == 1 && B.n <= kFrontPoints && in_place_fits(cx, B, spec_passes);
+}
+static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
+    if (!cx.mid || cx.pending.mid_skipped || !in_place_fits(cx, B, spec_passes)) return false;
+    const Hints *seen = cx.hints_for(B.shape);
+    return !seen || seen->mid != 0;
+}
+// The tree's sweep is for nothing where it leaves a call to the general path:
+// 5 to 8% of such a call (64 Gaussian meshes of 200000 points, another shape each
+// call: 1.72 ms without the tree, 1.83 with it).  A shape not seen before tries
+// it all the same, since where it takes the call it saves up to a half; after
+// kMidMisses new shapes in a row that it left, the next 2, 4, 8, then 16 pass it by.
+constexpr uint32_t kMidMisses = 3;
+static bool mid_passed_by(Context &cx, const BatchPlan &B, int spec_passes) {
+    if (cx.mid_wait == 0 || cx.hints_for(B.shape) || !cx.mid || !in_place_fits(cx, B, spec_passes) ||
+        front_fits(cx, B, spec_passes))
+        return false;
+    cx.mid_wait--;
+    return true;
+}
+static void mid_tried(Context &cx, bool left) {   // a new shape's call that had only the general path besides
+    cx.mid_misses = left ? cx.mid_misses + 1 : 0;
+    cx.mid_wait = cx.mid_misses >= kMidMisses ? 2u << std::min(cx.mid_misses - kMidMisses, 3u) : 0;
 }
 
 template <typename K>
@@ -1494,6 +1515,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
                     const MidCounters m = run_mid<D, WL, Acc>(cx, st, B, wrap, d_out, w, w_src);
                     if (!mode_held(cx)) return kAgain;
                     Hints &h = cx.remember(B.shape);
+                    if (!front && h.mid < 0) mid_tried(cx, m.big != 0);
                     h.mid = m.big ? 0 : 1;
                     h.mid_open = m.open;
                     if (!m.big) return finish(B.max_levels, m.open ? (uint32_t)kSubMaxNb : 2u);
@@ -1852,6 +1874,8 @@ static enum coupe_err rcb_general(Context &cx, hipStream_t st, uint64_t *d_out, 
         int spec = cx.search_passes;
         const Hints *seen = cx.hints_for(B.shape);
         const int passes_hint = seen ? seen->passes_hint : 0;
+        cx.pending.mid_skipped = false;
+        cx.pending.mid_skipped = mid_passed_by(cx, B, spec);
         if (passes_hint > 0 && spec > 0)
             spec = std::max(2, std::min(16, passes_hint + (B.n >= kSparePoints ? 2 : 0)));
         // A shape this context has run (hints known, buffers sized) runs as

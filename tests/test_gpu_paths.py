@@ -86,3 +86,37 @@ def test_general_path_on_small_cases(oracle_mod, monkeypatch, seed):
         _call(oracle_mod, ctx, pts, w, iters, tol, f"seed {seed}")
     finally:
         ctx.close()
+
+
+def test_new_shapes_after_misses_of_the_midpoint_tree(oracle_mod):
+    """Batches of another shape each call whose roots do not split at the
+    midpoints: after three the tree is passed by for 2, then 4 new shapes; a
+    batch that splits there brings it back."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(14)
+    pieces, tol = 4, 0.25
+    ctx = coupe_amd.DeviceContext(0)
+    try:
+        ctx.set_profiling(True)
+        # (cloud, path, whether the tree was tried and left the call)
+        calls = [("skew", "general", t) for t in (1, 1, 1, 0, 0, 1, 0, 0)]
+        calls += [("even", "general", 0), ("even", "mid", 0), ("skew", "general", 1), ("even", "mid", 0)]
+        for k, (cloud, path, tried) in enumerate(calls):
+            n = 100_000 + k
+            print(f"[gpu] new shapes, call {k}: {cloud}", flush=True)
+            pts = rng.random((n * pieces, 3))
+            if cloud == "skew":
+                pts = pts ** 3
+            w = rng.integers(1, 50, n * pieces).astype(np.float64)
+            out = torch.zeros(n * pieces, dtype=torch.int64, device="cuda")
+            coupe_amd.partition_batch(out, torch.from_numpy(pts).cuda(), torch.from_numpy(w).cuda(),
+                                      [(n, 8, tol)] * pieces, context=ctx)
+            got = out.cpu().numpy().astype(np.uint64)
+            for q in range(pieces):
+                s = slice(q * n, (q + 1) * n)
+                err, exp, _ = oracle_mod.rcb(pts[s], w[s], 8, tol, parallel=True, nthreads=8)
+                assert err == 0 and np.array_equal(got[s], exp), f"call {k} piece {q}"
+            assert path_of(ctx) == path, f"call {k}: {ctx.kernel_times()}"
+            assert ctx.stats()["reruns"] == tried, f"call {k}: {ctx.stats()}"
+    finally:
+        ctx.close()
