@@ -2,7 +2,8 @@
 ids against the oracle, on clouds whose splits lie away from the middle of
 their box, with few and many points per part, duplicates, coordinates over many
 magnitudes (long searches: the rounds queued ahead run out), every weight kind,
-first and later calls of a shape; COUPE_HIP_FRONT=0 takes the general path."""
+first and later calls of a shape; with COUPE_HIP_FRONT=0 the general path takes
+what the midpoint tree, tried first, leaves."""
 import numpy as np
 import pytest
 

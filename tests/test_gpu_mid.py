@@ -2,7 +2,8 @@
 against the oracle, on clouds that leave no node open, a few, most, or the
 root; sizes at the edges of tiles and of the classes of open nodes; every
 weight kind and width; box magnitudes and duplicates that put points on the
-midpoints; first and later calls of a shape."""
+midpoints; first and later calls of a shape.  With COUPE_HIP_MID=0 the
+frontier takes the single problems (test_gpu_paths.py checks which path runs)."""
 import numpy as np
 import pytest
 
@@ -106,7 +107,7 @@ def test_midpoint_tree_in_a_batch(oracle_mod, dim):
 
 def test_grids_and_other_points_of_a_shape(oracle_mod):
     """A shape's calls alternate between points the tree settles, points that
-    leave nodes open and points whose root search goes on (general path)."""
+    leave nodes open and points whose root search goes on (frontier)."""
     torch = pytest.importorskip("torch")
     pts, w = workloads.jgrid(48, 2, True)
     n = len(w)

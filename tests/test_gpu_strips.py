@@ -1,8 +1,9 @@
 """2D grids by strips (COUPE_HIP_GRID_STRIPS=1 sends every 2D call of up to 20
 levels there) against the oracle, id for id: sizes around a band of rows and
-a group of columns (16), a tile (512 columns), the prefix kept in LDS (2048
-cross-sections) and a workgroup's step (4096); subgrids of a few cells and
-empty ones; more subgrids than CUs; weights at one cell, zero, negative."""
+a group of columns (16), their partial scans (64 rows, 512 columns) and the
+workgroup's step along an axis (256 cross-sections); subgrids of a few cells and
+empty ones; more subgrids than CUs; weights at one cell, zero, negative.  Axes
+of more than one step a chunk: test_gpu_strips_long.py."""
 import numpy as np
 import pytest
 
