@@ -1241,8 +1241,8 @@ static MidCounters run_mid(Context &cx, hipStream_t st, const BatchPlan &B, int 
         return std::min(persistent_grid(cx, kernel, items), by_lds);
     };
     {
-        // 16-bit weights share a word with the count (unless a workgroup's share is large)
-        const bool one_word = packable<WL, Acc>() && n / (uint64_t)cx.cu_count < (1ull << 23);
+        // the grid has a workgroup per CU at least, or one per tile
+        const bool one_word = packable<WL, Acc>() && mid_one_word(nt, std::min<uint64_t>(cx.cu_count, nt));
         const uint32_t lds = max_cells * (one_word ? 8u : 12u);
         auto launch = [&](auto kernel, int tpb) {
             const unsigned grid = grid_of(kernel, nt, lds);

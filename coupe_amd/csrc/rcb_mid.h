@@ -123,6 +123,14 @@ __device__ __forceinline__ uint32_t mid_rank(const float4 *rank, int n, float x,
     return __builtin_bit_cast(uint32_t, t.z);
 }
 
+// Whether the shares of a grid stay below 2^24 points, so that the count and
+// the weight of a cell (16-bit weights) fit one word.  The host allots the
+// LDS by it, for the fewest workgroups the launch may have.
+__host__ __device__ constexpr bool mid_one_word(uint64_t tiles, uint64_t grid) {
+    return (tiles + grid - 1) / grid * kTile < (1ull << 24);
+}
+static_assert(mid_one_word(256ull * 8191, 256) && !mid_one_word(256ull * 8191 + 1, 256), "a share of 2^24 points");
+
 // Runs of a wavefront's cells up to which they are added run by run (a random
 // cloud has about 60; 2^27 points in mesh order: 553 us without, 505 with).
 constexpr int kMidRuns = 14;
@@ -143,9 +151,7 @@ k_mid_count(const Tile *__restrict__ tiles, uint32_t n_tiles, const Instance *__
     uint32_t t0, t1;
     tile_range(n_tiles, t0, t1);
     if (t0 >= t1) return;
-    // 16-bit weights: count and weight of a cell in one word (a workgroup's
-    // share stays below 2^24 points)
-    const bool packed = packable<WL, Acc>() && (uint64_t)(t1 - t0) * kTile < (1ull << 24);
+    const bool packed = packable<WL, Acc>() && mid_one_word(n_tiles, gridDim.x);
     Acc *sw = (Acc *)mid_lds;
     uint32_t *sc = nullptr;
     const int tid = threadIdx.x, lane = tid & 63;
