@@ -175,6 +175,7 @@ struct Context {
     int wg_cap = 0;                  // workgroups per CU of the persistent kernels (0: as many as fit)
     // tuned switches per batch class (tune_key), chosen by coupe_hip_autotune
     std::vector<std::pair<uint64_t, coupe_hip_tuning>> tuned;
+    uint64_t level_runs = 0;         // times the general path has run
     bool tuning_now = false;         // the autotuner runs the call: the table is not applied
     bool capturing = false;          // the running call is being captured
     PendingCall pending;             // what the running call queued

@@ -411,6 +411,7 @@ static bool run_levels(Context &cx, hipStream_t st, const BatchPlan &B, int wrap
                        int spec_passes) {
     Counters *ctr = (Counters *)cx.counters.ptr;
     uint32_t *h_search = (uint32_t *)cx.host_scratch;
+    cx.level_runs++;
     Instance *insts = (Instance *)cx.instances.ptr;
     const uint32_t n_inst = (uint32_t)B.inst.size();
     const uint64_t n = B.n;
@@ -2132,7 +2133,11 @@ enum coupe_err autotune(Context &cx, hipStream_t st, uint64_t *d_out, const doub
     };
     coupe_hip_tuning best = current_tuning(cx);
     double best_t = 0.0;
+    const uint64_t runs = cx.level_runs;
     bool ok = measure(best, best_t);
+    // calls that stay off the general path do not read its switches: noise
+    // must not choose them for the calls of the class that end there
+    const bool general = cx.level_runs != runs;
     // one switch at a time from the best so far; a candidate must win by 1%
     auto try_set = [&](auto field, std::initializer_list<uint32_t> values) {
         for (uint32_t v : values) {
@@ -2149,10 +2154,10 @@ enum coupe_err autotune(Context &cx, hipStream_t st, uint64_t *d_out, const doub
         }
     };
     try_set(&coupe_hip_tuning::graphs, {1, 0});
-    try_set(&coupe_hip_tuning::bins, {256, 128, 64, 32});
+    if (general || best.graphs) try_set(&coupe_hip_tuning::bins, {256, 128, 64, 32});
     try_set(&coupe_hip_tuning::workgroups_per_cu, {0, 4, 2, 1});
-    try_set(&coupe_hip_tuning::full_first, {1, 0});
-    try_set(&coupe_hip_tuning::search_chunk, {2, 1, 4});
+    if (general || best.graphs) try_set(&coupe_hip_tuning::full_first, {1, 0});
+    if (general || best.graphs) try_set(&coupe_hip_tuning::search_chunk, {2, 1, 4});
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (!ok) return err != COUPE_ERR_OK ? err : COUPE_ERR_CRASH;

@@ -120,3 +120,30 @@ def test_new_shapes_after_misses_of_the_midpoint_tree(oracle_mod):
             assert ctx.stats()["reruns"] == tried, f"call {k}: {ctx.stats()}"
     finally:
         ctx.close()
+
+
+def test_autotuner_leaves_what_the_call_does_not_read(oracle_mod):
+    """A batch that the midpoint tree and the one-workgroup kernel take whole
+    does not read the general path's bins, first pass and chunks: the tuner
+    keeps them (graphs, which would take that path, must win to be chosen)."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(31)
+    specs = [(n, 3, 6, 0.2) for n in (30_000, 60_000, 5000, 90_000)]
+    total = sum(s[0] for s in specs)
+    pts, w = rng.random(total * 3), rng.integers(1, 50, total).astype(np.float64)
+    out = torch.full((total,), -1, dtype=torch.int64, device="cuda")
+    ctx = coupe_amd.DeviceContext(0)
+    try:
+        print("[gpu] autotune of a batch in place", flush=True)
+        for trial in range(3):
+            chosen = coupe_amd.autotune(out, torch.from_numpy(pts).cuda(), torch.from_numpy(w).cuda(), specs, trials=1,
+                                        context=ctx)
+            if not chosen["graphs"]:
+                assert (chosen["bins"], chosen["full_first"], chosen["search_chunk"]) == (256, 1, 2), chosen
+        got, off = out.cpu().numpy().astype(np.uint64), 0
+        for n, d, iters, tol in specs:
+            err, exp, _ = oracle_mod.rcb(pts[off * 3:(off + n) * 3].reshape(n, 3), w[off:off + n], iters, tol)
+            assert err == 0 and np.array_equal(got[off:off + n], exp)
+            off += n
+    finally:
+        ctx.close()
