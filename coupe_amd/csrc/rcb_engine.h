@@ -98,6 +98,8 @@ struct Hints {
     uint64_t graph_key = 0;             // graph key of its last call (a key is captured when it repeats)
     int mid = -1;                       // the midpoint tree took its last call (-1: not tried, 0: no)
     uint32_t front_rounds = 0;          // rounds the frontier took in its last call
+    bool front_long = false;            // so many that the general path takes the next call
+    uint32_t front_reruns = 0;          // calls of the general path after that which ran again
     uint32_t mid_open = 1;              // open nodes the midpoint tree left (0: none)
     bool no_room = false;               // the paths in place could not have their buffers
     int moves_coherent = -1;            // its moved tiles went to few destinations (-1: not known)

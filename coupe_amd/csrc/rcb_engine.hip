@@ -229,7 +229,10 @@ static bool finish_levels(Context &cx) {
         if (e.mid == 0 || P.mid_skipped) {
             const bool midpoints = P.levels >= 3 && open1[0] == 0 && open1[1] == 0 && open1[2] == 0;
             e.mid = midpoints ? -1 : 0;
-            if (midpoints) cx.mid_misses = cx.mid_wait = 0;
+            if (midpoints) {
+                e.front_long = false;
+                cx.mid_misses = cx.mid_wait = 0;
+            }
         }
     }
     return h->unfinished != 0;
@@ -1115,6 +1118,8 @@ static bool in_place_fits(const Context &cx, const BatchPlan &B, int spec_passes
 }
 // And whether the frontier (rcb_front.h) takes it after that.
 static bool front_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
+    const Hints *seen = cx.hints_for(B.shape);
+    if (seen && seen->front_long && seen->front_reruns < kFrontReruns) return false;
     return cx.front && B.inst.size() == 1 && B.n <= kFrontPoints && in_place_fits(cx, B, spec_passes);
 }
 static bool mid_fits(const Context &cx, const BatchPlan &B, int spec_passes) {
@@ -1532,6 +1537,7 @@ static bool run_typed(Context &cx, hipStream_t st, uint64_t *d_out, const BatchP
                     if (rounds == 0) return kGeneral;
                     Hints &h = cx.remember(B.shape);
                     h.front_rounds = rounds;
+                    h.front_long = B.n > kFrontEven && 2 * rounds > kFrontLong * B.max_levels;
                     // the midpoint tree again when every level took one round
                     if (h.mid == 0 && rounds <= B.max_levels) h.mid = -1;
                     return finish(rounds, kSubMaxNb);
@@ -1891,6 +1897,8 @@ static enum coupe_err rcb_general(Context &cx, hipStream_t st, uint64_t *d_out, 
         if (unfinished) {
             // a split search needed more passes than were queued: again,
             // checking every pass on the host
+            Hints &e = cx.remember(B.shape);
+            if (e.front_long) e.front_reruns++;
             cx.stats = coupe_hip_stats{};
             cx.stats.points = B.n;
             cx.stats.reruns = 1;

@@ -32,6 +32,18 @@ constexpr int kFrontThreads = 1024;
 constexpr uint32_t kFrontCopies = 256;        // workgroups of a round, each with bins of its own
 constexpr int kFrontRounds = 256;             // rounds a call may take
 constexpr uint64_t kFrontPoints = 1ull << 25; // largest call (larger ones: the general path's fewer bytes per level)
+// Calls of more than kFrontEven points whose rounds are more than kFrontLong / 2 a
+// level go to the general path next time (heavy-tailed clouds: a round costs a
+// pass over all points, the general path's later passes only the parts that
+// search; us on the frontier and the general path, 10 levels 3D.  2^23 points:
+// lognormal, 28 rounds, 2170 and 1710; fifth powers of normals, 46, 2460 and
+// 2220; Gaussian mixture, 19, 1180 and 1400.  2^24: 2890 and 2610, 3780 and
+// 3430, 1820 and 2070.  2^21 2D: 24 rounds of 9 levels, 890 and 975), unless
+// its searches outrun what it queues as the points change (Cauchy, 28 rounds,
+// 1840 and 4500): after kFrontReruns such calls the frontier keeps the shape.
+constexpr uint64_t kFrontEven = 1ull << 22;
+constexpr uint32_t kFrontLong = 5;
+constexpr uint32_t kFrontReruns = 2;
 constexpr uint32_t kFrontDecides = 64;        // workgroups of k_front_decide
 constexpr int kDecideThreads = 512;           // (1024 leave too few registers: loads in flight, no spills)
 

@@ -147,3 +147,40 @@ def test_autotuner_leaves_what_the_call_does_not_read(oracle_mod):
             off += n
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("cloud", ["lognormal", "clusters", "changing"])
+def test_long_searches_of_large_calls(oracle_mod, cloud):
+    """More than 2^22 points off the midpoints: a shape whose frontier took many
+    rounds goes to the general path, unless its searches run out there twice;
+    other shapes stay on the frontier."""
+    torch = pytest.importorskip("torch")
+    n, iters, tol = (1 << 22) + 5, 8, 0.01
+    rng = np.random.default_rng(21)
+    w = rng.integers(1, 50, n).astype(np.float64)
+    ctx = coupe_amd.DeviceContext(0)
+    try:
+        ctx.set_profiling(True)
+        paths, reruns = [], []
+        for call in range(3 if cloud != "changing" else 5):
+            if cloud == "clusters":
+                pts = rng.random((8, 3))[rng.integers(0, 8, n)] + 0.05 * rng.normal(0, 1, (n, 3))
+            elif cloud == "lognormal":
+                pts = np.exp(2.0 * np.random.default_rng(5).normal(0, 1, (n, 3)))
+            else:   # windows of other extents each call
+                pts = np.tan(np.pi * (rng.random((n, 3)) - 0.5)) * 10.0 ** (3 * call)
+            label = f"{cloud} call {call}"
+            paths.append(_call(oracle_mod, ctx, pts, w, iters, tol, label))
+            st = ctx.stats()
+            reruns.append(st["reruns"])
+            print(f"[gpu] {label}: {paths[-1]}, {st['passes']} passes, reruns {reruns[-1]}", flush=True)
+        if cloud == "clusters":
+            assert paths == ["front"] * 3
+        elif cloud == "lognormal":
+            assert paths == ["front", "general", "general"]
+        else:
+            assert paths[:2] == ["front", "general"]
+            for k in range(2, len(paths)):
+                assert paths[k] == ("front" if sum(reruns[1:k]) >= 2 else "general"), (paths, reruns)
+    finally:
+        ctx.close()
