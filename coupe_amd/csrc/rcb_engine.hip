@@ -285,7 +285,12 @@ void scan_u64(Context &cx, hipStream_t st, uint64_t *data, const uint32_t *n_dev
 // queue one and two more: a queued pass whose gate stays closed costs about
 // 8 us, the run with host checks that a search outlasting its passes brings
 // costs the call again (5.8e8 points in 4096 instances, three data sets in
-// turn: 39.2 -> 29.6 ms; 2^27-point grids: 6.51 -> 6.62 ms, but no run of 13 ms).
+// turn: 39.2 -> 29.6 ms).  Both sides by size, Gaussian mixtures 3D, 10 levels,
+// three data sets in turn (two at 2^26), mean us without and with the spare
+// passes: 2^18 737 and 758, 2^20 807 and 852, 2^22 1508 and 1092 (4 of 12 calls
+// ran again without), 2^24 2796 and 2081 (4 of 12), 2^25 3526 and 3592, 2^26
+// 6387 and 6358.  They cost 2 to 6% where no call runs again, so smaller calls
+// do without; from 2^26 on they are free.
 constexpr uint64_t kSparePoints = 1ull << 26;
 static int queued_passes(int spec, uint32_t decisions, uint64_t n) {
     const int more = n >= kSparePoints ? 1 : 0;

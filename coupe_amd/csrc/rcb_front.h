@@ -27,20 +27,28 @@
 namespace coupe_hip {
 
 constexpr uint32_t kFrontNodes = 1024;        // parts of a frontier: fewer, each holds more than n / 1024 points
-constexpr uint32_t kFrontBins = 5376;         // bins of a round
+constexpr uint32_t kFrontBins = 5376;         // bins of a round: with the parts what the LDS of a CU holds
 constexpr int kFrontThreads = 1024;
 constexpr uint32_t kFrontCopies = 256;        // workgroups of a round, each with bins of its own
 constexpr int kFrontRounds = 256;             // rounds a call may take
-constexpr uint64_t kFrontPoints = 1ull << 25; // largest call (larger ones: the general path's fewer bytes per level)
-// Calls of more than kFrontEven points whose rounds are more than kFrontLong / 2 a
-// level go to the general path next time (heavy-tailed clouds: a round costs a
-// pass over all points, the general path's later passes only the parts that
-// search; us on the frontier and the general path, 10 levels 3D.  2^23 points:
-// lognormal, 28 rounds, 2170 and 1710; fifth powers of normals, 46, 2460 and
-// 2220; Gaussian mixture, 19, 1180 and 1400.  2^24: 2890 and 2610, 3780 and
-// 3430, 1820 and 2070.  2^21 2D: 24 rounds of 9 levels, 890 and 975), unless
-// its searches outrun what it queues as the points change (Cauchy, 28 rounds,
-// 1840 and 4500): after kFrontReruns such calls the frontier keeps the shape.
+constexpr uint64_t kFrontPoints = 1ull << 25; // largest call: see below
+// kFrontPoints: Gaussian mixtures 3D, 10 levels, points changing, mean us on the
+// frontier and the general path: 2^20 525 and 805, 2^22 905 and 1510, 2^24 1790
+// and 2800, 2^25 3320 and 3530, 2^26 6180 and 6390.  Beyond 2^25 what is left
+// does not pay for the 28 bytes a point the frontier holds besides.
+//
+// Calls of more than kFrontEven points that took more than kFrontLong / 2 rounds
+// a level go to the general path next time: a round costs a pass over all
+// points, the general path's later passes only the parts that still search.  us
+// on the frontier and the general path, 3D, 10 levels.  2^23 points: lognormal,
+// 28 rounds, 2170 and 1710; fifth powers of normals, 46, 2460 and 2220; Gaussian
+// mixture, 19, 1180 and 1400.  2^24: 2890 and 2610, 3780 and 3430, 1820 and 2070.
+// From 1 to 12 levels, tolerances 0.001 and 0.02, 5e6 and 2^24 points alike: up
+// to 2.3 rounds a level the frontier is faster by 0 to 40%, from 2.6 on slower by
+// 0 to 45%.  2^21 points 2D: 24 rounds of 9 levels, 890 and 975, still faster.
+// Where the points change, the general path's searches outrun what it queues
+// (Cauchy points, 28 rounds, 1840 and 4500): after kFrontReruns such calls the
+// frontier keeps the shape.
 constexpr uint64_t kFrontEven = 1ull << 22;
 constexpr uint32_t kFrontLong = 5;
 constexpr uint32_t kFrontReruns = 2;

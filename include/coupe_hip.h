@@ -350,7 +350,7 @@ struct coupe_hip_stats {
 	uint32_t weight_mode;     /* 0 int64 exact sums, 1 f64 sums */
 	uint32_t weight_bytes;    /* bytes per stored weight (2, 4 or 8) */
 	uint32_t bins;            /* histogram bins per part per pass */
-	uint32_t reruns;          /* 1 when the call ran again: a split search outran the queued passes, or the midpoint tree left nodes open where it left none before */
+	uint32_t reruns;          /* 1 when the call ran again: a split search outran the queued passes, the midpoint tree left nodes open where it left none before or left the call to another path, or a path's buffers had no room */
 	uint64_t unit_points;     /* points per work unit */
 	uint64_t device_bytes;    /* device memory held by the context */
 	uint64_t first_read;      /* points read by the children's first passes (two levels per move) */
